@@ -11,7 +11,8 @@
 //              lens[b] rotates k_new (eager RoPE rounding) and writes it and
 //              v_new into the caches (the reference's KVCache.update) instead
 //              of reading that row.
-//  2. merge    one workgroup per (b, hq) rescales and sums the partials.
+//  2. merge    rescales and sums the partials of each (b, hq), by one to 16
+//              wavefronts depending on how many there are (kf_merge.h).
 // With QK-norm weights the per-head RMSNorm of q_new and k_new (the
 // reference's q_norm / k_norm, applied before RoPE) happens where the rows
 // are loaded, instead of in separate launches.
@@ -20,6 +21,7 @@
 // or n_rep > 16) use decode_generic: one wavefront per (b, hq).
 #include "kf_common.h"
 #include "kf_internal.h"
+#include "kf_merge.h"
 #include "kf_mfma.h"
 
 #include <algorithm>
@@ -102,9 +104,11 @@ __global__ __launch_bounds__(256) void append_kernel(const T* __restrict__ k_new
 // Every (sequence b, KV head g) pair p = b * Hkv + g holds nck(b) = ceil((lens[b]
 // + 1) / KC) chunks of KC keys (0 when the length is unusable).  The chunks of
 // all pairs, in (b, g, key) order, form one list of C chunks, and wavefront w
-// of the NW in the grid streams the contiguous range [w C / NW, (w + 1) C / NW):
-// every wavefront reads the same number of bytes (to one chunk), whatever the
-// lengths, and keeps its loads in flight across pair boundaries.  A wavefront
+// of the first NW = min(the grid's, C) streams the contiguous range [w C / NW,
+// (w + 1) C / NW): every wavefront reads the same number of bytes (to one
+// chunk), whatever the lengths, and keeps its loads in flight across pair
+// boundaries; none has an empty range, so every slot the merge visits was
+// written.  A wavefront
 // writes one partial (o, m, l) per pair it touches, in slot w + p: the pairs a
 // wavefront touches are consecutive and the wavefronts touching a pair are
 // consecutive, so (w, p) -> w + p is one-to-one; NW + B * Hkv slots suffice.
@@ -271,10 +275,10 @@ __global__ __launch_bounds__(256, 2) void decode_stream_kernel(
   const int w = wave_id(), lane = threadIdx.x & 63, q4 = lane >> 4, c16 = lane & 15;
   WaveLds& L = lds_all[w];
   const DecodeSched s{lens, B, Hkv, max_len, row_offset, rope_rows};
-  const int NW = gridDim.x * DEC_WAVES, gw = blockIdx.x * DEC_WAVES + w;
-  const int C = total_chunks(s, lane);
+  const int gw = blockIdx.x * DEC_WAVES + w;
+  const int C = total_chunks(s, lane), NW = min((int)gridDim.x * DEC_WAVES, C);
+  if (gw >= NW) return;
   const int c_lo = range_start(gw, C, NW), c_hi = range_start(gw + 1, C, NW);
-  if (c_lo >= c_hi) return;
 
   // the chunk's rows, loaded one step ahead: each set is reloaded for the next
   // chunk as soon as this chunk's products have read it, so one register set
@@ -540,21 +544,17 @@ __global__ __launch_bounds__(256, 2) void decode_stream_kernel(
   }
 }
 
-// One wavefront per (b, hq), four per workgroup: the partials of the
-// wavefronts whose ranges met pair (b, g) are rescaled to a common maximum and
-// summed.  The slot range comes from one pass over lens; the partial outputs
-// of the first MERGE_PRE slots are then loaded together with the (m, l)
-// values, so a merge costs two dependent memory round trips.
-constexpr int MERGE_PRE = 16;
-
-template <typename T, int D>
-__global__ __launch_bounds__(256) void decode_merge_kernel(
+// One row (b, hq) per WPR wavefronts: the partials of the wavefronts whose
+// ranges met pair (b, g), from one pass over lens.  WPR 1: four rows per
+// workgroup; otherwise one.
+template <typename T, int D, int WPR>
+__global__ __launch_bounds__(WPR == 1 ? 256 : 64 * WPR) void decode_merge_kernel(
     const float* __restrict__ opart, const float* __restrict__ mlpart,
-    const int32_t* __restrict__ lens, T* __restrict__ out, int B, int Hq, int Hkv, int NW,
+    const int32_t* __restrict__ lens, T* __restrict__ out, int B, int Hq, int Hkv, int NWmax,
     int max_len, int64_t row_offset, int64_t rope_rows) {
-  constexpr int PER = D / 64;
-  const int lane = threadIdx.x & 63;
-  const int bh = blockIdx.x * 4 + (threadIdx.x >> 6);
+  __shared__ __attribute__((aligned(16))) float sO[WPR > 1 ? WPR * D : 4];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int bh = WPR == 1 ? blockIdx.x * 4 + w : blockIdx.x;
   if (bh >= B * Hq) return;
   const int b = bh / Hq, hq = bh % Hq, n_rep = Hq / Hkv, g = hq / n_rep, h = hq % n_rep;
   const DecodeSched s{lens, B, Hkv, max_len, row_offset, rope_rows};
@@ -567,61 +567,24 @@ __global__ __launch_bounds__(256) void decode_merge_kernel(
     pre += wave_sum_int(b0 + lane < b ? nb : 0);
     if (b >= b0 && b < b0 + 64) n = __shfl(nb, b - b0, 64);
   }
-  const int C = tot * Hkv;
-  T* orow = out + (int64_t)bh * D + lane;
+  const int C = tot * Hkv, NW = min(NWmax, C);
+  const int col = 4 * (lane % (D / 4));
+  T* orow = out + (int64_t)bh * D + col;
+  const bool writer = lane < D / 4 && (WPR == 1 || w == 0);
   if (n == 0) {  // unusable length: NaN output, no cache write happened
 #pragma unroll
-    for (int k = 0; k < PER; ++k) orow[64 * k] = from_f32<T>(NAN);
+    for (int e = 0; e < 4; ++e)
+      if (writer) orow[e] = from_f32<T>(NAN);
     return;
   }
   const int c0 = pre * Hkv + g * n;
   const int w0 = chunk_owner(c0, C, NW), ns = chunk_owner(c0 + n - 1, C, NW) - w0 + 1;
   const int64_t first = ((int64_t)w0 + (int64_t)b * Hkv + g) * n_rep + h;  // slot w0 + p's row
-  const float* ob = opart + first * D + lane;
-  const float* mb = mlpart + first * 2;
-  const int64_t ost = (int64_t)n_rep * D, mst = (int64_t)n_rep * 2;  // per slot
-  // wavefronts with an empty range (C < NW) between w0 and w1 wrote nothing:
-  // their slots hold stale data, get weight 0 and are never added
-  auto live = [&](int j) {
-    return j < ns && range_start(w0 + j, C, NW) != range_start(w0 + j + 1, C, NW);
-  };
-  float po[MERGE_PRE][PER];
+  const f32x4 o = merge_row<D, WPR>(opart + first * D, mlpart + first * 2, (int64_t)n_rep * D,
+                                    (int64_t)n_rep * 2, ns, sO, WPR == 1 ? 0 : w, lane);
 #pragma unroll
-  for (int j = 0; j < MERGE_PRE; ++j)
-#pragma unroll
-    for (int k = 0; k < PER; ++k) po[j][k] = j < ns ? ob[j * ost + 64 * k] : 0.f;
-  const bool live0 = live(lane);
-  float2 ml0 = make_float2(-INFINITY, 0.f);
-  if (live0) ml0 = *(const float2*)(mb + lane * mst);
-  float M = ml0.x;
-  for (int j = 64 + lane; j < ns; j += 64)
-    if (live(j)) M = fmaxf(M, mb[j * mst]);
-  M = wave_max(M);
-  const float wgt0 = live0 ? fast_exp2(ml0.x - M) : 0.f;
-  float lt = live0 ? ml0.y * wgt0 : 0.f;
-  for (int j = 64 + lane; j < ns; j += 64)
-    if (live(j)) lt += mb[j * mst + 1] * fast_exp2(mb[j * mst] - M);
-  lt = wave_sum(lt);
-  float o[PER];
-#pragma unroll
-  for (int k = 0; k < PER; ++k) o[k] = 0.f;
-#pragma unroll
-  for (int j = 0; j < MERGE_PRE; ++j) {
-    const float wj = __shfl(wgt0, j, 64);
-    if (wj != 0.f)
-#pragma unroll
-      for (int k = 0; k < PER; ++k) o[k] += po[j][k] * wj;
-  }
-  for (int j = MERGE_PRE; j < ns; ++j) {
-    const float wj = j < 64 ? __shfl(wgt0, j, 64)
-                            : (live(j) ? fast_exp2(mb[j * mst] - M) : 0.f);
-    if (wj != 0.f)
-#pragma unroll
-      for (int k = 0; k < PER; ++k) o[k] += ob[j * ost + 64 * k] * wj;
-  }
-  const float inv = 1.f / lt;
-#pragma unroll
-  for (int k = 0; k < PER; ++k) orow[64 * k] = from_f32<T>(o[k] * inv);
+  for (int e = 0; e < 4; ++e)
+    if (writer) orow[e] = from_f32<T>(o[e]);
 }
 
 // One wavefront per (b, hq); keys 0..lens[b] read from the (already appended)
@@ -708,8 +671,12 @@ int launch_append(const T* k_new, const T* v_new, const float* cos, const float*
   return KF_OK;
 }
 
-// Grid of the stream kernel: two workgroups per CU, at most DEC_GRID_MAX.
-int decode_grid() { return std::max(1, std::min(DEC_GRID_MAX, 2 * device_cu_count())); }
+// Grid of the stream kernel: two workgroups per CU, at most DEC_GRID_MAX and
+// no more than the longest sequences could give a chunk per wavefront.
+int decode_grid(int64_t max_chunks) {
+  const int64_t cap = std::max(1, std::min(DEC_GRID_MAX, 2 * device_cu_count()));
+  return (int)std::min(cap, (max_chunks + DEC_WAVES - 1) / DEC_WAVES);
+}
 
 template <typename T, int D>
 int launch_stream(const DecodeArgs& a, float* opart, float* mlpart, int grid) {
@@ -721,6 +688,20 @@ int launch_stream(const DecodeArgs& a, float* opart, float* mlpart, int grid) {
             a.rope_rows, a.max_len, (T*)a.k_cache, (T*)a.v_cache, a.lens, opart, mlpart,
             a.B, a.Hq, a.Hkv, a.Smax, a.Hq / a.Hkv, a.scale * kLog2e, a.q_norm_w, a.k_norm_w,
             a.norm_eps);
+  KF_CHECK_LAUNCH();
+  return KF_OK;
+}
+
+template <typename T, int D>
+int launch_merge(const DecodeArgs& a, const float* opart, const float* mlpart, int nw, int wpr) {
+  const int rows = a.B * a.Hq;
+  KF_LAUNCH("decode_merge",
+            (wpr == 1   ? decode_merge_kernel<T, D, 1>
+             : wpr == 4 ? decode_merge_kernel<T, D, 4>
+                        : decode_merge_kernel<T, D, 16>),
+            dim3(wpr == 1 ? (rows + 3) / 4 : rows), dim3(wpr == 1 ? 256 : 64 * wpr), 0, a.stream,
+            opart, mlpart, a.lens, (T*)a.out, a.B, a.Hq, a.Hkv, nw, a.max_len, a.rope_row_offset,
+            a.rope_rows);
   KF_CHECK_LAUNCH();
   return KF_OK;
 }
@@ -742,18 +723,17 @@ int decode_typed(const DecodeArgs& a, void* workspace) {
     const size_t slots = decode_slots(a.B, a.Hkv);
     float* opart = (float*)workspace;
     float* mlpart = opart + slots * n_rep * a.D;
-    const int grid = decode_grid();
+    const int64_t pairs = (int64_t)a.B * a.Hkv, nck = (a.max_len + KC - 1) / KC;
+    const int grid = decode_grid(pairs * nck);
+    // partials per row: the wavefronts' shares that meet one pair
+    const int wpr = merge_waves((int)std::min(nck, grid * DEC_WAVES / pairs + 1));
     if constexpr (__is_same(T, bf16) || __is_same(T, f16)) {
       rc = a.D == 128 ? launch_stream<T, 128>(a, opart, mlpart, grid)
                       : launch_stream<T, 64>(a, opart, mlpart, grid);
       if (rc) return rc;
-      KF_LAUNCH("decode_merge",
-                (a.D == 128 ? decode_merge_kernel<T, 128> : decode_merge_kernel<T, 64>),
-                dim3((a.B * a.Hq + 3) / 4), dim3(256), 0, a.stream, opart, mlpart, a.lens,
-                (T*)a.out, a.B, a.Hq, a.Hkv, grid * DEC_WAVES, a.max_len, a.rope_row_offset,
-                a.rope_rows);
-      KF_CHECK_LAUNCH();
-      return KF_OK;
+      rc = a.D == 128 ? launch_merge<T, 128>(a, opart, mlpart, grid * DEC_WAVES, wpr)
+                      : launch_merge<T, 64>(a, opart, mlpart, grid * DEC_WAVES, wpr);
+      return rc;
     }
   }
   rc = launch_append<T>((const T*)a.k_new, (const T*)a.v_new, a.cos, a.sin, (T*)a.k_cache,

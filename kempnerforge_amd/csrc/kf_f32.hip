@@ -30,7 +30,10 @@
 // into the other of two buffers, one barrier per tile; the tiles that need
 // RoPE (K, and Q in dK/dV) come from a prepass that writes the rotated rows.
 #include "kf_internal.h"
+#include "kf_merge.h"
 #include "kf_mfma.h"
+
+#include <algorithm>
 
 namespace kf {
 
@@ -1010,6 +1013,12 @@ __device__ __forceinline__ float rms_scale_f32(float x, float ss, int D, float e
 // decode_merge_f32 combines an item's splits.
 constexpr int DEC_KEYS = 64;  // keys per step (4 wavefronts x 16)
 
+// Keys per split of a sequence of L keys: whole steps, at most nsplit splits.
+__device__ __forceinline__ int split_keys(int L, int nsplit) {
+  const int per = (L + nsplit - 1) / nsplit;
+  return (per + DEC_KEYS - 1) / DEC_KEYS * DEC_KEYS;
+}
+
 template <int D, bool QKN>
 __global__ __launch_bounds__(256, 2) void decode_f32_kernel(
     const float* __restrict__ q_new, const float* __restrict__ cos, const float* __restrict__ sin,
@@ -1028,18 +1037,11 @@ __global__ __launch_bounds__(256, 2) void decode_f32_kernel(
   const int64_t trow = (int64_t)len - row_offset;
   const bool ok = len >= 0 && len < max_len && trow >= 0 && trow < rope_rows;
   const int L = ok ? len + 1 : 0;
-  const int per = (L + nsplit - 1) / nsplit;
-  const int chunk = (per + DEC_KEYS - 1) / DEC_KEYS * DEC_KEYS;
+  const int chunk = split_keys(L, nsplit);
   const int lo = split * chunk, hi = min(L, lo + chunk);
   float* op = opart + (int64_t)item * n_rep * D;
   float* mp = mlpart + (int64_t)item * n_rep * 2;
-  if (lo >= hi) {  // nothing in this split: an empty partial
-    if (threadIdx.x < n_rep) {
-      mp[2 * threadIdx.x] = -INFINITY;
-      mp[2 * threadIdx.x + 1] = 0.f;
-    }
-    return;
-  }
+  if (lo >= hi) return;  // nothing in this split: the merge does not visit it
   const int nsteps = (hi - lo + DEC_KEYS - 1) / DEC_KEYS;
   const float* kb = kc + ((int64_t)b * Hkv + hk) * Smax * D;
   const float* vb = vc + ((int64_t)b * Hkv + hk) * Smax * D;
@@ -1176,38 +1178,44 @@ __global__ __launch_bounds__(256, 2) void decode_f32_kernel(
 }
 
 // out[b, hq] = the splits' partials combined (max and sums in log2 units);
-// NaN for a sequence whose length fails the checks.  One wavefront per row.
-template <int D>
-__global__ __launch_bounds__(256) void decode_merge_f32_kernel(
+// NaN for a sequence whose length fails the checks.  Rows per wavefronts as in
+// the 16-bit merge.
+template <int D, int WPR>
+__global__ __launch_bounds__(WPR == 1 ? 256 : 64 * WPR) void decode_merge_f32_kernel(
     const float* __restrict__ opart, const float* __restrict__ mlpart,
     const int32_t* __restrict__ lens, float* __restrict__ out, int B, int Hq, int Hkv,
     int nsplit, int max_len, int64_t row_offset, int64_t rope_rows) {
-  const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  __shared__ __attribute__((aligned(16))) float sO[WPR > 1 ? WPR * D : 4];
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int row = WPR == 1 ? blockIdx.x * 4 + w : blockIdx.x;
   if (row >= B * Hq) return;
   const int b = row / Hq, hq = row % Hq, n_rep = Hq / Hkv, hk = hq / n_rep, h = hq % n_rep;
   const int len = lens[b];
   const int64_t trow = (int64_t)len - row_offset;
-  float* orow = out + (int64_t)row * D;
+  float* orow = out + (int64_t)row * D + 4 * (lane % (D / 4));
+  const bool writer = lane < D / 4 && (WPR == 1 || w == 0);
   if (!(len >= 0 && len < max_len && trow >= 0 && trow < rope_rows)) {
-    for (int d = lane; d < D; d += 64) orow[d] = NAN;
+    if (writer) *(f32x4*)orow = f32x4{NAN, NAN, NAN, NAN};
     return;
   }
-  const int64_t item0 = ((int64_t)b * Hkv + hk) * nsplit;
-  float mx = -INFINITY;
-  for (int s = 0; s < nsplit; ++s) mx = fmaxf(mx, mlpart[((item0 + s) * n_rep + h) * 2]);
-  float acc[D / 64] = {}, lt = 0.f;
-  for (int s = 0; s < nsplit; ++s) {
-    const float* ml = mlpart + ((item0 + s) * n_rep + h) * 2;
-    if (ml[1] == 0.f) continue;
-    const float wgt = fast_exp2(ml[0] - mx);
-    lt += wgt * ml[1];
-    const float* o = opart + ((item0 + s) * n_rep + h) * D;
-#pragma unroll
-    for (int k = 0; k < D / 64; ++k) acc[k] += wgt * o[64 * k + lane];
-  }
-  const float inv = 1.f / lt;
-#pragma unroll
-  for (int k = 0; k < D / 64; ++k) orow[64 * k + lane] = acc[k] * inv;
+  // the splits that hold keys (decode_f32_kernel's rule)
+  const int chunk = split_keys(len + 1, nsplit), ns = (len + chunk) / chunk;
+  const int64_t first = (((int64_t)b * Hkv + hk) * nsplit) * n_rep + h;
+  const f32x4 o = merge_row<D, WPR>(opart + first * D, mlpart + first * 2, (int64_t)n_rep * D,
+                                    (int64_t)n_rep * 2, ns, sO, WPR == 1 ? 0 : w, lane);
+  if (writer) *(f32x4*)orow = o;
+}
+
+template <int D>
+void launch_merge_f32(const DecodeArgs& a, const float* opart, const float* mlpart, int nsplit) {
+  const int rows = a.B * a.Hq, wpr = merge_waves(nsplit);
+  KF_LAUNCH("decode_merge_f32",
+            (wpr == 1   ? decode_merge_f32_kernel<D, 1>
+             : wpr == 4 ? decode_merge_f32_kernel<D, 4>
+                        : decode_merge_f32_kernel<D, 16>),
+            dim3(wpr == 1 ? (rows + 3) / 4 : rows), dim3(wpr == 1 ? 256 : 64 * wpr), 0, a.stream,
+            opart, mlpart, a.lens, (float*)a.out, a.B, a.Hq, a.Hkv, nsplit, a.max_len,
+            a.rope_row_offset, a.rope_rows);
 }
 
 template <int D>
@@ -1497,7 +1505,9 @@ bool decode_f32_supported(const DecodeArgs& a) {
 int decode_f32(const DecodeArgs& a, void* workspace, size_t slots) {
   const int n_rep = a.Hq / a.Hkv;
   const int64_t pairs = (int64_t)a.B * a.Hkv;
-  const int nsplit = (int)(1 + (int64_t)(slots - pairs) / pairs);  // items fit the slots
+  // items fit the slots, and no sequence has more splits than steps
+  const int nsplit = (int)std::min<int64_t>(1 + (int64_t)(slots - pairs) / pairs,
+                                            (a.max_len + DEC_KEYS - 1) / DEC_KEYS);
   const int64_t items = pairs * nsplit;
   KF_CHECK_ARG(items < (1LL << 31) && (size_t)items <= slots, "decode grid too large");
   float* opart = (float*)workspace;
@@ -1517,10 +1527,8 @@ int decode_f32(const DecodeArgs& a, void* workspace, size_t slots) {
     else KF_DEC_F32(64, false);
   }
 #undef KF_DEC_F32
-  KF_LAUNCH("decode_merge_f32",
-            (a.D == 128 ? decode_merge_f32_kernel<128> : decode_merge_f32_kernel<64>),
-            dim3((a.B * a.Hq + 3) / 4), dim3(256), 0, a.stream, opart, mlpart, a.lens,
-            (float*)a.out, a.B, a.Hq, a.Hkv, nsplit, a.max_len, a.rope_row_offset, a.rope_rows);
+  if (a.D == 128) launch_merge_f32<128>(a, opart, mlpart, nsplit);
+  else launch_merge_f32<64>(a, opart, mlpart, nsplit);
   KF_CHECK_LAUNCH();
   return KF_OK;
 }
