@@ -73,12 +73,27 @@ static int check_masks(const int32_t* doc, const int32_t* kvalid, int causal, in
 static size_t fwd_ws(const FwdArgs& a) {
   if (fwd_mfma_supported(a)) return fwd_mfma_workspace(a.B, a.Sk, a.Hkv, a.D);
   if (fwd_f32_supported(a)) return a.k_rotated ? 0 : fwd_f32_workspace(a.B, a.Sk, a.Hkv, a.D);
+  if (fwd_wide_supported(a)) return fwd_wide_workspace(a);
   return 0;
+}
+
+// Head sizes 64 and 128 need the workspace their size call asks for.  At the
+// others the generic kernels, which need none (or less), serve a call whose
+// workspace is too small for the matrix-core kernels.
+static bool own_dim(int D) { return D == 64 || D == 128; }
+static bool takes_f32(const FwdArgs& a, const void* workspace, size_t bytes) {
+  if (!fwd_f32_supported(a)) return false;
+  const size_t need = fwd_ws(a);
+  return own_dim(a.D) || need == 0 || (workspace && bytes >= need);
+}
+static bool takes_wide(const FwdArgs& a, const void* workspace, size_t bytes) {
+  return fwd_wide_supported(a) && workspace && bytes >= fwd_wide_workspace(a);
 }
 
 static size_t bwd_ws(const BwdArgs& a) {
   if (bwd_mfma_supported(a)) return bwd_mfma_workspace(a.B, a.S, a.Hq, a.Hkv, a.D);
   if (bwd_f32_supported(a)) return bwd_f32_workspace(a.B, a.S, a.Hq, a.Hkv, a.D);
+  if (bwd_wide_supported(a)) return bwd_wide_workspace(a, false);
   return bwd_generic_workspace(a.B, a.S, a.Hq);
 }
 
@@ -129,7 +144,7 @@ int kf_attn_fwd(const void* q, const void* k, const void* v, const float* rope_c
     }
     return fwd_mfma(a, workspace);
   }
-  if (fwd_f32_supported(a)) {
+  if (takes_f32(a, workspace, workspace_bytes)) {
     const size_t need = fwd_ws(a);
     if (workspace_bytes < need || (need && !workspace)) {
       set_error("workspace too small: need %zu bytes, got %zu", need, workspace_bytes);
@@ -137,6 +152,7 @@ int kf_attn_fwd(const void* q, const void* k, const void* v, const float* rope_c
     }
     return fwd_f32(a, workspace);
   }
+  if (takes_wide(a, workspace, workspace_bytes)) return fwd_wide(a, workspace);
   return fwd_generic(a);
 }
 
@@ -173,7 +189,8 @@ int kf_attn_bwd_workspace_size_ds(int B, int S, int Hq, int Hkv, int D, int dtyp
   const BwdArgs a = sizing_args(B, S, Hq, Hkv, D, dtype, causal);
   *bytes = bwd_mfma_supported(a)  ? bwd_mfma_workspace_ds(a)
            : bwd_f32_supported(a) ? bwd_f32_workspace_ds(B, S, Hq, Hkv, D, causal)
-                                  : bwd_ws(a);
+           : bwd_wide_supported(a) ? bwd_wide_workspace(a, true)
+                                   : bwd_ws(a);
   return KF_OK;
 }
 
@@ -204,13 +221,17 @@ int kf_attn_bwd(const void* q, const void* k, const void* v, const float* rope_c
     }
     return bwd_mfma(a, workspace, workspace_bytes);
   }
-  const size_t need = bwd_ws(a);
+  if (bwd_wide_supported(a) && workspace && workspace_bytes >= bwd_wide_workspace(a, false))
+    return bwd_wide(a, workspace, workspace_bytes);
+  const bool f32 =
+      bwd_f32_supported(a) &&
+      (own_dim(D) || (workspace && workspace_bytes >= bwd_f32_workspace(B, S, Hq, Hkv, D)));
+  const size_t need = f32 ? bwd_f32_workspace(B, S, Hq, Hkv, D) : bwd_generic_workspace(B, S, Hq);
   if (workspace_bytes < need || !workspace) {
     set_error("workspace too small: need %zu bytes, got %zu", need, workspace_bytes);
     return KF_ERR_WORKSPACE;
   }
-  if (bwd_f32_supported(a)) return bwd_f32(a, workspace, workspace_bytes);
-  return bwd_generic(a, workspace);
+  return f32 ? bwd_f32(a, workspace, workspace_bytes) : bwd_generic(a, workspace);
 }
 
 // Whether the rotated-operand pair (kf_attn_fwd_rot / kf_attn_bwd_rot) takes
@@ -445,7 +466,7 @@ int kf_attn_capture(const void* q, const void* k, const void* v, const float* ro
     }
     return capture_probs_mfma(a, probs, workspace);
   }
-  if (fwd_f32_supported(a)) {
+  if (takes_f32(a, workspace, workspace_bytes)) {
     const size_t need = fwd_ws(a);
     if (workspace_bytes < need || (need && !workspace)) {
       set_error("workspace too small: need %zu bytes, got %zu", need, workspace_bytes);
@@ -453,6 +474,7 @@ int kf_attn_capture(const void* q, const void* k, const void* v, const float* ro
     }
     return capture_f32(a, probs, workspace);
   }
+  if (takes_wide(a, workspace, workspace_bytes)) return capture_wide(a, probs, workspace);
   rc = fwd_generic(a);
   if (rc) return rc;
   return capture_probs_generic(a, lse, probs);

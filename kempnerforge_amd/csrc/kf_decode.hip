@@ -568,8 +568,7 @@ __global__ __launch_bounds__(WPR == 1 ? 256 : 64 * WPR) void decode_merge_kernel
     if (b >= b0 && b < b0 + 64) n = __shfl(nb, b - b0, 64);
   }
   const int C = tot * Hkv, NW = min(NWmax, C);
-  const int col = 4 * (lane % (D / 4));
-  T* orow = out + (int64_t)bh * D + col;
+  T* orow = out + (int64_t)bh * D + 4 * lane;
   const bool writer = lane < D / 4 && (WPR == 1 || w == 0);
   if (n == 0) {  // unusable length: NaN output, no cache write happened
 #pragma unroll

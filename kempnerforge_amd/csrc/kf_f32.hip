@@ -24,9 +24,12 @@
 // second half (chunk_of), so the rows a lane loads itself rotate in registers.
 //
 // LDS tiles are [32 rows][D] floats with 16-byte chunk c of row r at position
-// c ^ (r % 16): the chunk reads (16 consecutive rows, one chunk per pass) and
-// the element reads (rows 4 apart, 16 consecutive floats each) both meet 64
-// distinct banks.  Tiles reach LDS by direct global->LDS loads one tile ahead,
+// c ^ (r % 16) (D 64, 128): the chunk reads (16 consecutive rows, one chunk per
+// pass) and the element reads (rows 4 apart, 16 consecutive floats each) both
+// meet 64 distinct banks.  D 32 and 96 have 8 and 24 chunks per row, which
+// only a 3-bit swizzle permutes: c ^ (r / 2 % 8), with the 32-bank step of odd
+// rows, keeps the chunk reads conflict-free; the element reads meet each bank
+// twice (8 cycles of MFMA per 4-byte read leave room for it).  Tiles reach LDS by direct global->LDS loads one tile ahead,
 // into the other of two buffers, one barrier per tile; the tiles that need
 // RoPE (K, and Q in dK/dV) come from a prepass that writes the rotated rows.
 #include "kf_internal.h"
@@ -34,6 +37,7 @@
 #include "kf_mfma.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace kf {
 
@@ -58,10 +62,15 @@ __device__ __forceinline__ int chunk_of(int j, int g) {
   constexpr int H = D / 32;
   return j < H ? H * g + j : D / 8 + H * g + (j - H);
 }
+// chunk swizzle of row r of an LDS tile: chunk c sits at position c ^ fsw(r)
+template <int D>
+__device__ __forceinline__ int fsw(int r) {
+  return D % 64 == 0 ? r & 15 : (r >> 1) & 7;
+}
 // float index of chunk c of row r of an LDS tile
 template <int D>
 __device__ __forceinline__ int tix(int r, int c) {
-  return (r * (D / 4) + (c ^ (r & 15))) * 4;
+  return (r * (D / 4) + (c ^ fsw<D>(r))) * 4;
 }
 // element (r, d) of an LDS tile
 template <int D>
@@ -115,7 +124,7 @@ __device__ __forceinline__ void tile_dma(const float* g, uint32_t ld, float* lds
   for (int j = 0; j < PER; ++j) {
     const int L = (w * PER + j) * 64 + lane, row = L / R, pc = L % R;
     const uint32_t off =
-        ((uint32_t)min(row, rows_valid - 1) * ld + (uint32_t)(pc ^ (row & 15)) * 4u) * 4u;
+        ((uint32_t)min(row, rows_valid - 1) * ld + (uint32_t)(pc ^ fsw<D>(row)) * 4u) * 4u;
     mfma::dma16(mfma::lds_addr(lds + (w * PER + j) * 256), off, g);
   }
 }
@@ -243,13 +252,15 @@ __global__ __launch_bounds__(256) void rows_f32_kernel(const float* __restrict__
 
 // Per query row (b, h, i), i < Sp: -lse log2(e) and Delta = sum_d dO O, in
 // 64-float groups per 32 positions ([B Hq][Sp/32][nl x 32, Delta x 32]);
-// rows past S get -inf and 0 (probability zero).  16 lanes per row.
-template <int D>
-__global__ __launch_bounds__(256) void stats_f32_kernel(const float* __restrict__ o,
-                                                        const float* __restrict__ dout,
+// rows past S get -inf and 0 (probability zero).  o and dout are [B, S, Hq, D]
+// of their own type, D a multiple of 4.  16 lanes per row.
+template <typename T>
+__global__ __launch_bounds__(256) void stats_f32_kernel(const T* __restrict__ o,
+                                                        const T* __restrict__ dout,
                                                         const float* __restrict__ lse,
                                                         float* __restrict__ stats, int S, int Sp,
-                                                        int Hq, int64_t rows) {
+                                                        int Hq, int D, int64_t rows) {
+  typedef T t4 __attribute__((ext_vector_type(4)));
   const int64_t row = (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4);  // (b Hq + h) Sp + i
   const int l = threadIdx.x & 15;
   const int i = (int)(row % Sp);
@@ -258,11 +269,11 @@ __global__ __launch_bounds__(256) void stats_f32_kernel(const float* __restrict_
   float s = 0.f;
   if (valid) {
     const int64_t off = ((bh / Hq * S + i) * Hq + bh % Hq) * D;
-#pragma unroll
     for (int c = l; c < D / 4; c += 16) {
-      const f32x4 a = *(const f32x4*)(o + off + 4 * c);
-      const f32x4 b = *(const f32x4*)(dout + off + 4 * c);
-      s += a[0] * b[0] + a[1] * b[1] + a[2] * b[2] + a[3] * b[3];
+      const t4 a = *(const t4*)(o + off + 4 * c);
+      const t4 b = *(const t4*)(dout + off + 4 * c);
+      s += to_f32(a[0]) * to_f32(b[0]) + to_f32(a[1]) * to_f32(b[1]) +
+           to_f32(a[2]) * to_f32(b[2]) + to_f32(a[3]) * to_f32(b[3]);
     }
   }
 #pragma unroll
@@ -410,7 +421,7 @@ __device__ __forceinline__ bool row_sees(const KeyWalk<MODE>& k, int k0, int j, 
 // rows of all its query heads share each K/V tile); S^T = K·Q^T per 32-key
 // tile, online softmax in the lane, O^T += V^T·P^T.  K comes rotated: element
 // (b, g, key, d) at kt + b kb_b + g kb_h + key kld + d (the prepass's rows or
-// a rotated cache).
+// a rotated cache); q_rot: q comes rotated too.
 template <int D, int MODE>
 __global__ __launch_bounds__(256, 2) void fwd_f32_kernel(
     const float* __restrict__ q, const float* __restrict__ cos, const float* __restrict__ sin,
@@ -418,7 +429,7 @@ __global__ __launch_bounds__(256, 2) void fwd_f32_kernel(
     int64_t vsh, int vss, float* __restrict__ out, float* __restrict__ lse, int Sq, int Sk,
     int Hq, int Hkv, int n_rep, int bm_pos, int nqb, int causal, float scale_log2,
     const int32_t* __restrict__ mask, const int2* __restrict__ ranges,
-    const int* __restrict__ first_valid, int nt32) {
+    const int* __restrict__ first_valid, int nt32, int q_rot) {
   constexpr int NJ = D / 16, NB = D / 16;
   __shared__ __attribute__((aligned(16))) float sK[2][F_BN * D];
   __shared__ __attribute__((aligned(16))) float sV[2][F_BN * D];
@@ -445,7 +456,7 @@ __global__ __launch_bounds__(256, 2) void fwd_f32_kernel(
 
   f32x4 qr[NJ];
   load_row_share<D>(q + (((int64_t)ri.b * Sq + ri.pos) * Hq + ri.hq) * D, cos, sin, ri.pos, g,
-                    ri.q_valid, true, qr);
+                    ri.q_valid, !q_rot, qr);
 
   float m = -INFINITY, l = 0.f;
   f32x4 o[NB];
@@ -527,7 +538,7 @@ __global__ __launch_bounds__(256, 2) void capture_f32_kernel(
     const float* kt, int64_t kb_b, int64_t kb_h, int kld, const float* __restrict__ lse,
     float* __restrict__ probs, int Sq, int Sk, int Hq, int Hkv, int n_rep, int bm_pos, int nqb,
     int causal, float scale_log2, const int32_t* __restrict__ mask,
-    const int2* __restrict__ ranges, const int* __restrict__ first_valid, int nt32) {
+    const int2* __restrict__ ranges, const int* __restrict__ first_valid, int nt32, int q_rot) {
   constexpr int NJ = D / 16;
   __shared__ __attribute__((aligned(16))) float sK[2][F_BN * D];
   __shared__ uint16_t sList[MODE == MASK_DOC ? F_MAX_TILES : 1];
@@ -551,7 +562,7 @@ __global__ __launch_bounds__(256, 2) void capture_f32_kernel(
 
   f32x4 qr[NJ];
   load_row_share<D>(q + (((int64_t)ri.b * Sq + ri.pos) * Hq + ri.hq) * D, cos, sin, ri.pos, g,
-                    ri.q_valid, true, qr);
+                    ri.q_valid, !q_rot, qr);
   const float nl = ri.q_valid ? -lse[((int64_t)ri.b * Hq + ri.hq) * Sq + ri.pos] * kLog2e : 0.f;
   float* prow = probs + (((int64_t)ri.b * Hq + ri.hq) * Sq + ri.pos) * Sk;
   const bool vec = (Sk & 3) == 0 && ((uintptr_t)probs & 15) == 0;  // rows 16-byte aligned
@@ -1192,7 +1203,7 @@ __global__ __launch_bounds__(WPR == 1 ? 256 : 64 * WPR) void decode_merge_f32_ke
   const int b = row / Hq, hq = row % Hq, n_rep = Hq / Hkv, hk = hq / n_rep, h = hq % n_rep;
   const int len = lens[b];
   const int64_t trow = (int64_t)len - row_offset;
-  float* orow = out + (int64_t)row * D + 4 * (lane % (D / 4));
+  float* orow = out + (int64_t)row * D + 4 * lane;
   const bool writer = lane < D / 4 && (WPR == 1 || w == 0);
   if (!(len >= 0 && len < max_len && trow >= 0 && trow < rope_rows)) {
     if (writer) *(f32x4*)orow = f32x4{NAN, NAN, NAN, NAN};
@@ -1271,7 +1282,7 @@ void launch_fwd_f32(const FwdArgs& a, const float* kt, int64_t kb_b, int64_t kb_
             (const float*)a.q, a.cos, a.sin, kt, kb_b, kb_h, kld, (const float*)a.v, a.vsb, a.vsh,
             (int)a.vss, (float*)a.out, a.lse, a.Sq, a.Sk, a.Hq, a.Hkv, n_rep, bm_pos, nqb,
             a.causal, a.scale * kLog2e, a.doc ? a.doc : a.kvalid, mr.ranges, mr.first_valid,
-            mr.nt32);
+            mr.nt32, a.q_rotated);
 }
 
 template <int D>
@@ -1296,7 +1307,7 @@ int fwd_f32_t(const FwdArgs& a, void* workspace) {
   const int mode = mask_mode_of(a.doc, a.kvalid);
   MaskRec mr{nullptr, nullptr, 0};
   if (mode != MASK_NONE) {
-    mr = mask_rec(workspace, fwd_krot_bytes(a.B, a.Sk, a.Hkv, D), a.B, a.Sk);
+    mr = mask_rec(workspace, a.k_rotated ? 0 : fwd_krot_bytes(a.B, a.Sk, a.Hkv, D), a.B, a.Sk);
     const int rc = launch_mask_prep(a.doc ? a.doc : a.kvalid, mode, a.B, a.Sk, mr, a.stream);
     if (rc) return rc;
   }
@@ -1358,56 +1369,60 @@ size_t rec_bytes(int B, int S, int Hq, int causal) {
 }
 
 template <int D>
-int bwd_f32_t(const BwdArgs& a, void* workspace, float* rec) {
+int bwd_f32_t(const BwdArgs& a, const F32BwdWs& w, float* rec) {
   const int n_rep = a.Hq / a.Hkv, bm_pos = F_ROWS / n_rep;
   const int nqb = (a.S + bm_pos - 1) / bm_pos;
-  const int Sp = (a.S + F_BK - 1) / F_BK * F_BK;
   const int64_t nqblk = (int64_t)nqb * a.B * a.Hkv;
-  const int64_t nkblk = (int64_t)(Sp / F_BK) * a.B * a.Hkv;
+  const int64_t nkblk = (int64_t)(w.Sp / F_BK) * a.B * a.Hkv;
   KF_CHECK_ARG(nqblk < (1LL << 31) && nkblk < (1LL << 31), "grid too large");
-  size_t sum_off = 0;
-  const size_t base = bwd_base_bytes(a.B, a.S, a.Hq, a.Hkv, D, &sum_off);
-  float* qrot = (float*)workspace;
-  float* krot = qrot + (size_t)a.B * a.Hq * Sp * D;
-  float* stats = krot + (size_t)a.B * a.Hkv * Sp * D;
-  double* sum64 = (double*)((char*)workspace + sum_off);
-  const int64_t qss = (int64_t)a.Hq * D, kss = (int64_t)a.Hkv * D;
-  int rc = launch_rows<D>((const float*)a.q, a.S * qss, qss, D, a.cos, a.sin, qrot, a.B, a.S, Sp,
-                          a.Hq, 1, a.stream);
-  if (rc) return rc;
-  rc = launch_rows<D>((const float*)a.k, a.S * kss, kss, D, a.cos, a.sin, krot, a.B, a.S, Sp,
-                      a.Hkv, 1, a.stream);
-  if (rc) return rc;
-  const int64_t rows = (int64_t)a.B * a.Hq * Sp;
-  KF_LAUNCH("stats_f32", (stats_f32_kernel<D>), dim3((unsigned)((rows + 15) / 16)), dim3(256), 0,
-            a.stream, (const float*)a.out, (const float*)a.dout, a.lse, stats, a.S, Sp, a.Hq,
-            rows);
   const int mode = mask_mode_of(a.doc, a.kvalid);
   MaskRec mr{nullptr, nullptr, 0};
   if (mode != MASK_NONE) {
-    mr = mask_rec(workspace, base, a.B, a.S);
-    rc = launch_mask_prep(a.doc ? a.doc : a.kvalid, mode, a.B, a.S, mr, a.stream);
+    mr = mask_rec(w.masks, 0, a.B, a.S);
+    const int rc = launch_mask_prep(a.doc ? a.doc : a.kvalid, mode, a.B, a.S, mr, a.stream);
     if (rc) return rc;
   }
   if (mode == MASK_DOC)
-    launch_bwd_kernels<D, MASK_DOC>(a, qrot, krot, stats, sum64, Sp, n_rep, bm_pos, nqb,
+    launch_bwd_kernels<D, MASK_DOC>(a, w.qrot, w.krot, w.stats, w.sum64, w.Sp, n_rep, bm_pos, nqb,
                                     (unsigned)nqblk, (unsigned)nkblk, mr, rec);
   else if (mode == MASK_KPM)
-    launch_bwd_kernels<D, MASK_KPM>(a, qrot, krot, stats, sum64, Sp, n_rep, bm_pos, nqb,
+    launch_bwd_kernels<D, MASK_KPM>(a, w.qrot, w.krot, w.stats, w.sum64, w.Sp, n_rep, bm_pos, nqb,
                                     (unsigned)nqblk, (unsigned)nkblk, mr, rec);
   else
-    launch_bwd_kernels<D, MASK_NONE>(a, qrot, krot, stats, sum64, Sp, n_rep, bm_pos, nqb,
-                                     (unsigned)nqblk, (unsigned)nkblk, mr, rec);
+    launch_bwd_kernels<D, MASK_NONE>(a, w.qrot, w.krot, w.stats, w.sum64, w.Sp, n_rep, bm_pos,
+                                     nqb, (unsigned)nqblk, (unsigned)nkblk, mr, rec);
   KF_CHECK_LAUNCH();
   return KF_OK;
 }
 
+template <int D>
+int bwd_rows_t(const BwdArgs& a, const F32BwdWs& w) {
+  const int64_t qss = (int64_t)a.Hq * D, kss = (int64_t)a.Hkv * D;
+  const int rc = launch_rows<D>((const float*)a.q, a.S * qss, qss, D, a.cos, a.sin, w.qrot, a.B,
+                                a.S, w.Sp, a.Hq, 1, a.stream);
+  if (rc) return rc;
+  return launch_rows<D>((const float*)a.k, a.S * kss, kss, D, a.cos, a.sin, w.krot, a.B, a.S,
+                        w.Sp, a.Hkv, 1, a.stream);
+}
+
 bool al16(const void* p) { return ((uintptr_t)p & 15) == 0; }
+
+// f(integral_constant<D>) for the head sizes the kernels are built for
+bool f32_dim(int D) { return D == 32 || D == 64 || D == 96 || D == 128; }
+template <typename F>
+int by_dim(int D, F f) {
+  switch (D) {
+    case 32: return f(std::integral_constant<int, 32>{});
+    case 64: return f(std::integral_constant<int, 64>{});
+    case 96: return f(std::integral_constant<int, 96>{});
+    default: return f(std::integral_constant<int, 128>{});
+  }
+}
 
 }  // namespace
 
 bool fwd_f32_supported(const FwdArgs& a) {
-  if (a.dtype != F32 || (a.D != 64 && a.D != 128)) return false;
+  if (a.dtype != F32 || !f32_dim(a.D)) return false;
   if (a.rot || (a.doc && a.kvalid)) return false;
   if (a.Sq < 1 || a.Sk < 1 || a.Hkv < 1 || a.Hq % a.Hkv) return false;
   if (a.Hq / a.Hkv > F_ROWS) return false;
@@ -1428,7 +1443,7 @@ size_t fwd_f32_workspace(int B, int Sk, int Hkv, int D) {
 }
 
 int fwd_f32(const FwdArgs& a, void* workspace) {
-  return a.D == 128 ? fwd_f32_t<128>(a, workspace) : fwd_f32_t<64>(a, workspace);
+  return by_dim(a.D, [&](auto d) { return fwd_f32_t<decltype(d)::value>(a, workspace); });
 }
 
 int capture_f32(const FwdArgs& a, float* probs, void* workspace) {
@@ -1448,25 +1463,25 @@ int capture_f32(const FwdArgs& a, float* probs, void* workspace) {
   }
   const int mode = mask_mode_of(a.doc, a.kvalid);
   MaskRec mr{nullptr, nullptr, 0};
-  if (mode != MASK_NONE) mr = mask_rec(workspace, fwd_krot_bytes(a.B, a.Sk, a.Hkv, a.D), a.B, a.Sk);
+  if (mode != MASK_NONE)
+    mr = mask_rec(workspace, a.k_rotated ? 0 : fwd_krot_bytes(a.B, a.Sk, a.Hkv, a.D), a.B, a.Sk);
   const int32_t* mask = a.doc ? a.doc : a.kvalid;
-#define KF_CAP_F32(DD, M)                                                                        KF_LAUNCH("capture_f32", (capture_f32_kernel<DD, M>), dim3(nblk), dim3(256), 0, a.stream,                (const float*)a.q, a.cos, a.sin, kt, kb_b, kb_h, (int)kld, a.lse, probs, a.Sq,                  a.Sk, a.Hq, a.Hkv, n_rep, bm_pos, nqb, a.causal, a.scale * kLog2e, mask,                       mr.ranges, mr.first_valid, mr.nt32)
-  if (a.D == 128) {
-    if (mode == MASK_DOC) KF_CAP_F32(128, MASK_DOC);
-    else if (mode == MASK_KPM) KF_CAP_F32(128, MASK_KPM);
-    else KF_CAP_F32(128, MASK_NONE);
-  } else {
-    if (mode == MASK_DOC) KF_CAP_F32(64, MASK_DOC);
-    else if (mode == MASK_KPM) KF_CAP_F32(64, MASK_KPM);
-    else KF_CAP_F32(64, MASK_NONE);
-  }
-#undef KF_CAP_F32
-  KF_CHECK_LAUNCH();
-  return KF_OK;
+  return by_dim(a.D, [&](auto d) {
+    constexpr int DD = decltype(d)::value;
+    KF_LAUNCH("capture_f32",
+              (mode == MASK_DOC   ? capture_f32_kernel<DD, MASK_DOC>
+               : mode == MASK_KPM ? capture_f32_kernel<DD, MASK_KPM>
+                                  : capture_f32_kernel<DD, MASK_NONE>),
+              dim3(nblk), dim3(256), 0, a.stream, (const float*)a.q, a.cos, a.sin, kt, kb_b, kb_h,
+              (int)kld, a.lse, probs, a.Sq, a.Sk, a.Hq, a.Hkv, n_rep, bm_pos, nqb, a.causal,
+              a.scale * kLog2e, mask, mr.ranges, mr.first_valid, mr.nt32, a.q_rotated);
+    KF_CHECK_LAUNCH();
+    return KF_OK;
+  });
 }
 
 bool bwd_f32_supported(const BwdArgs& a) {
-  if (a.dtype != F32 || (a.D != 64 && a.D != 128)) return false;
+  if (a.dtype != F32 || !f32_dim(a.D)) return false;
   if (a.rot || (a.doc && a.kvalid)) return false;
   if (a.S < 1 || a.Hkv < 1 || a.Hq % a.Hkv) return false;
   if (a.Hq / a.Hkv > F_ROWS || (int64_t)a.Hq * a.D > (1 << 24)) return false;
@@ -1485,18 +1500,54 @@ size_t bwd_f32_workspace_ds(int B, int S, int Hq, int Hkv, int D, int causal) {
   return rb ? al256(bwd_f32_workspace(B, S, Hq, Hkv, D)) + rb : bwd_f32_workspace(B, S, Hq, Hkv, D);
 }
 
-int bwd_f32(const BwdArgs& a, void* workspace, size_t workspace_bytes) {
+F32BwdWs bwd_f32_carve(int B, int S, int Hq, int Hkv, int D, void* workspace) {
+  F32BwdWs w;
+  w.Sp = (S + F_BK - 1) / F_BK * F_BK;
+  size_t sum_off = 0;
+  const size_t base = bwd_base_bytes(B, S, Hq, Hkv, D, &sum_off);
+  w.qrot = (float*)workspace;
+  w.krot = w.qrot + (size_t)B * Hq * w.Sp * D;
+  w.stats = w.krot + (size_t)B * Hkv * w.Sp * D;
+  w.sum64 = (double*)((char*)workspace + sum_off);
+  w.masks = (char*)workspace + al256(base);
+  return w;
+}
+
+int bwd_f32_stats(const void* out, const void* dout, const float* lse, int dtype, int B, int S,
+                  int Hq, int D, const F32BwdWs& w, hipStream_t stream) {
+  const int64_t rows = (int64_t)B * Hq * w.Sp;
+  auto launch = [&](auto t) {
+    using T = decltype(t);
+    KF_LAUNCH("stats_f32", (stats_f32_kernel<T>), dim3((unsigned)((rows + 15) / 16)), dim3(256),
+              0, stream, (const T*)out, (const T*)dout, lse, w.stats, S, w.Sp, Hq, D, rows);
+  };
+  if (dtype == BF16) launch(bf16{});
+  else if (dtype == F16) launch(f16{});
+  else launch(float{});
+  KF_CHECK_LAUNCH();
+  return KF_OK;
+}
+
+int bwd_f32_kernels(const BwdArgs& a, const F32BwdWs& w, void* workspace, size_t workspace_bytes) {
   // the dS records when there is no explicit mask and the workspace holds them
   float* rec = nullptr;
   if (!a.doc && !a.kvalid && rec_bytes(a.B, a.S, a.Hq, a.causal) != 0 &&
       workspace_bytes >= bwd_f32_workspace_ds(a.B, a.S, a.Hq, a.Hkv, a.D, a.causal))
     rec = (float*)((char*)workspace + al256(bwd_f32_workspace(a.B, a.S, a.Hq, a.Hkv, a.D)));
-  return a.D == 128 ? bwd_f32_t<128>(a, workspace, rec) : bwd_f32_t<64>(a, workspace, rec);
+  return by_dim(a.D, [&](auto d) { return bwd_f32_t<decltype(d)::value>(a, w, rec); });
 }
 
+int bwd_f32(const BwdArgs& a, void* workspace, size_t workspace_bytes) {
+  const F32BwdWs w = bwd_f32_carve(a.B, a.S, a.Hq, a.Hkv, a.D, workspace);
+  int rc = by_dim(a.D, [&](auto d) { return bwd_rows_t<decltype(d)::value>(a, w); });
+  if (rc) return rc;
+  rc = bwd_f32_stats(a.out, a.dout, a.lse, F32, a.B, a.S, a.Hq, a.D, w, a.stream);
+  if (rc) return rc;
+  return bwd_f32_kernels(a, w, workspace, workspace_bytes);
+}
 
 bool decode_f32_supported(const DecodeArgs& a) {
-  if (a.dtype != F32 || (a.D != 64 && a.D != 128) || a.Hkv < 1 || a.Hq % a.Hkv) return false;
+  if (a.dtype != F32 || !f32_dim(a.D) || a.Hkv < 1 || a.Hq % a.Hkv) return false;
   if (a.Hq / a.Hkv > 16) return false;
   return al16(a.q_new) && al16(a.k_cache) && al16(a.v_cache) && al16(a.cos) && al16(a.sin) &&
          al16(a.out);
@@ -1514,23 +1565,17 @@ int decode_f32(const DecodeArgs& a, void* workspace, size_t slots) {
   float* mlpart = opart + slots * n_rep * a.D;
   const bool qkn = a.q_norm_w != nullptr;
   const float sl = a.scale * kLog2e;
-#define KF_DEC_F32(DD, Q)                                                                      \
-  KF_LAUNCH("decode_f32", (decode_f32_kernel<DD, Q>), dim3((unsigned)items), dim3(256), 0,    \
-            a.stream, (const float*)a.q_new, a.cos, a.sin, a.rope_row_offset, a.rope_rows,     \
-            a.max_len, (const float*)a.k_cache, (const float*)a.v_cache, a.lens, opart, mlpart, \
-            a.Hq, a.Hkv, a.Smax, n_rep, nsplit, sl, a.q_norm_w, a.norm_eps)
-  if (a.D == 128) {
-    if (qkn) KF_DEC_F32(128, true);
-    else KF_DEC_F32(128, false);
-  } else {
-    if (qkn) KF_DEC_F32(64, true);
-    else KF_DEC_F32(64, false);
-  }
-#undef KF_DEC_F32
-  if (a.D == 128) launch_merge_f32<128>(a, opart, mlpart, nsplit);
-  else launch_merge_f32<64>(a, opart, mlpart, nsplit);
-  KF_CHECK_LAUNCH();
-  return KF_OK;
+  return by_dim(a.D, [&](auto d) {
+    constexpr int DD = decltype(d)::value;
+    KF_LAUNCH("decode_f32", (qkn ? decode_f32_kernel<DD, true> : decode_f32_kernel<DD, false>),
+              dim3((unsigned)items), dim3(256), 0, a.stream, (const float*)a.q_new, a.cos, a.sin,
+              a.rope_row_offset, a.rope_rows, a.max_len, (const float*)a.k_cache,
+              (const float*)a.v_cache, a.lens, opart, mlpart, a.Hq, a.Hkv, a.Smax, n_rep, nsplit,
+              sl, a.q_norm_w, a.norm_eps);
+    launch_merge_f32<DD>(a, opart, mlpart, nsplit);
+    KF_CHECK_LAUNCH();
+    return KF_OK;
+  });
 }
 
 }  // namespace kf

@@ -21,6 +21,7 @@ struct FwdArgs {
   int B, Sq, Sk, Hq, Hkv, D;
   int64_t ksb, kss, ksh, vsb, vss, vsh;
   int k_rotated;      // 1: k already holds post-RoPE keys (KV-cache contents)
+  int q_rotated = 0;  // 1: q already holds post-RoPE rows (float32 kernels only)
   int causal;         // 1: top-left causal mask (query i sees keys j <= i)
   const int32_t* doc; // [B, S] document id per position (packed sequences) or null;
                       // query i then also needs doc[i] == doc[j] (requires Sq == Sk)
@@ -58,9 +59,10 @@ size_t bwd_generic_workspace(int B, int S, int Hq);
 int bwd_generic(const BwdArgs& a, void* workspace);
 int capture_probs_generic(const FwdArgs& a, const float* lse, float* probs);
 
-// float32 MFMA kernels (kf_f32.hip): no explicit masks, head_dim 64 or 128.
-// Workspaces: the forward's rotated K (unused when a.k_rotated); the
-// backward's rotated Q and K and per-row softmax statistics.
+// float32 MFMA kernels (kf_f32.hip): one explicit mask kind at most, head_dim
+// 32, 64, 96 or 128.  Workspaces: the forward's rotated K (none when
+// a.k_rotated) and tile records; the backward's rotated Q and K, per-row softmax
+// statistics, group sums and tile records.
 bool fwd_f32_supported(const FwdArgs& a);
 size_t fwd_f32_workspace(int B, int Sk, int Hkv, int D);
 int fwd_f32(const FwdArgs& a, void* workspace);
@@ -73,6 +75,30 @@ size_t bwd_f32_workspace(int B, int S, int Hq, int Hkv, int D);
 // reaches it: dQ then multiplies them by K instead of recomputing S and dP)
 size_t bwd_f32_workspace_ds(int B, int S, int Hq, int Hkv, int D, int causal);
 int bwd_f32(const BwdArgs& a, void* workspace, size_t workspace_bytes);
+// bwd_f32 in parts, for operands prepared elsewhere: the carved workspace, the
+// row statistics of out and dout ([B, S, Hq, D] of `dtype`), and the kernels
+// (which read w.qrot, w.krot, w.stats, and a.v, a.dout, a.cos, a.sin in float32)
+struct F32BwdWs {
+  float *qrot, *krot;  // [B*Hq][Sp][D], [B*Hkv][Sp][D] after RoPE, rows past S zero
+  float* stats;
+  double* sum64;
+  void* masks;
+  int Sp;              // S rounded up to 64
+};
+F32BwdWs bwd_f32_carve(int B, int S, int Hq, int Hkv, int D, void* workspace);
+int bwd_f32_stats(const void* out, const void* dout, const float* lse, int dtype, int B, int S,
+                  int Hq, int D, const F32BwdWs& w, hipStream_t stream);
+int bwd_f32_kernels(const BwdArgs& a, const F32BwdWs& w, void* workspace, size_t workspace_bytes);
+
+// Head sizes without kernels of their own (kf_wide.hip): multiples of 16 up to
+// 128, run by the float32 kernels on float32 copies padded to a multiple of 32.
+bool fwd_wide_supported(const FwdArgs& a);
+size_t fwd_wide_workspace(const FwdArgs& a);
+int fwd_wide(const FwdArgs& a, void* workspace);
+int capture_wide(const FwdArgs& a, float* probs, void* workspace);
+bool bwd_wide_supported(const BwdArgs& a);
+size_t bwd_wide_workspace(const BwdArgs& a, bool with_ds);
+int bwd_wide(const BwdArgs& a, void* workspace, size_t workspace_bytes);
 
 // bf16 MFMA kernels (kf_fwd.hip, kf_bwd.hip, kf_capture.hip)
 bool fwd_mfma_supported(const FwdArgs& a);

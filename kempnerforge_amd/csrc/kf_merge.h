@@ -32,8 +32,10 @@ template <int D, int WPR>
 __device__ __forceinline__ f32x4 merge_row(const float* __restrict__ ob,
                                            const float* __restrict__ mb, int64_t ost,
                                            int64_t mst, int ns, float* sO, int wv, int lane) {
-  constexpr int LPS = D / 4, SPI = 64 / LPS;  // lanes per partial, partials per instruction
-  const int sub = lane / LPS, col = 4 * (lane % LPS);
+  // lanes per partial (a power of two; D 96 leaves 8 of 32 idle), partials per
+  // instruction
+  constexpr int LPS = D == 96 ? 32 : D / 4, SPI = 64 / LPS;
+  const int sub = lane / LPS, col = min(4 * (lane % LPS), D - 4);
   f32x4 po[MU];
   float pm[MU];
   auto slot = [&](int i) { return (i * WPR + wv) * SPI + sub; };
