@@ -584,7 +584,7 @@ def _short(name: str) -> str:
                   r"mask_prep_f32|capture_f32|decode_merge_f32|decode_f32|"
                   r"kv_prep|fwd_mfma|fwd32|q_prep_bwd|bwd_dkdv|bwd_dq_ds2|bwd_dq_ds|bwd_dq|decode_stream|"
                   r"decode_merge|capture_probs_mfma|kv_append|append|doc_block_tiles|"
-                  r"order_by_count|kpm_row_flags|dkdv_reduce|widen|narrow)_kernel", name)
+                  r"order_by_count|kpm_row_keys|dkdv_reduce|widen|narrow)_kernel", name)
     if m:
         # fwd32_kernel is the unmasked forward's kernel, launched as fwd_mfma;
         # bwd_dq_ds2_kernel (two query tiles per workgroup) as bwd_dq_ds

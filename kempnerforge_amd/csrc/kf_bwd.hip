@@ -167,7 +167,7 @@ struct DkdvStage {
 // MASK_KPM: qlist as above, drow the key-validity row, fv the first valid
 // key's position: query rows before it (guarded) see every key, other rows
 // need the key valid and not after them.
-template <typename T, int D, bool DSROLE, int MODE, bool STORE, bool PART>
+template <typename T, int D, bool DSROLE, int MODE, bool STORE, bool LIM, bool PART>
 __device__ __forceinline__ void dkdv_role(
     DkdvStage<T, D>* st, u32x4* sP, const T* __restrict__ krot, const T* __restrict__ v,
     const T* __restrict__ qrot, const T* __restrict__ dout,
@@ -176,7 +176,7 @@ __device__ __forceinline__ void dkdv_role(
     T* __restrict__ dv, int S, int P, int Hq, int Hkv, int n_rep, int b, int g, int bh, int k0,
     int w, int lane, float scale_log2, float scale, int causal, const int32_t* __restrict__ drow,
     const uint16_t* qlist, int nlist, int32_t (*sQD)[BQ], int fv, u32x4* __restrict__ dsb,
-    int nqtp, bool live, int part, int nsplit, float* __restrict__ pout) {
+    int nqtp, int nkeys, int part, int nsplit, float* __restrict__ pout) {
   constexpr bool DOC = MODE == MASK_DOC, KPM = MODE == MASK_KPM, LIST = DOC || KPM;
   // key padding keeps records only for a batch row whose first key is valid:
   // it has no guarded rows, so every dS tile lies in the causal record layout
@@ -196,12 +196,13 @@ __device__ __forceinline__ void dkdv_role(
   const int nqt = (S + BQ - 1) / BQ;
   const int qt0 = causal ? k0 / BQ : 0;
   const int per_head = LIST ? nlist : nqt - qt0;
-  // (live false: no query tile, dK / dV stored as zeros; a later launch
-  // writes this item's results)
+  // LIM: only the batch row's first nkeys keys are attended.  A block past
+  // them walks no query tile and stores zeros (with nkeys 0, a row of the KPM
+  // launch, that launch then writes the row's results)
   // PART: part `part` of `nsplit` takes the group's query heads
   // [h_base, h_base + n_rep / nsplit); otherwise all n_rep
   const int nh = PART ? n_rep / nsplit : n_rep, h_base = PART ? part * nh : 0;
-  const int total = per_head > 0 && live ? per_head * nh : 0;
+  const int total = per_head > 0 && (!LIM || k0 < nkeys) ? per_head * nh : 0;
   // iteration -> query tile entry (tile | DOC_MASK_FLAG when listed), head-major
   auto entry = [&](int it) -> int {
     return LIST ? __builtin_amdgcn_readfirstlane((int)qlist[it % per_head]) : qt0 + it % per_head;
@@ -223,10 +224,10 @@ __device__ __forceinline__ void dkdv_role(
     // +inf, so they contribute nothing)
     tile_to_lds<BQ, KR, 8, LIST>(dout + (((int64_t)b * S + q0) * Hq + hq) * D, Hq * D, S_.o, w,
                                  lane, S - q0);
-    if (LIST || PART) {
+    if (LIST || PART || LIM) {
       // the row statistics' LDS addresses from the stage array's base plus
-      // constant offsets: with the pointer into the stage member, the masked
-      // and split kernels fail to compile ("Operand has incorrect register
+      // constant offsets: with the pointer into the stage member, the masked,
+      // split and key-limited kernels fail to compile ("Operand has incorrect register
       // class": a constant generic-to-LDS address cast lowered with an
       // illegal null test)
       using Stage = DkdvStage<T, D>;
@@ -249,12 +250,12 @@ __device__ __forceinline__ void dkdv_role(
   // for P waves, V (read in place, [B, S, Hkv, D]; zero past S) for dS waves
   bf16x8 bf[KS];
   {
-    // (masked modes: key and half laundered, so that the 64-bit row address
+    // (masked and key-limited modes: key and half laundered, so that the 64-bit row address
     // is formed here per item rather than hoisted out of the persistent loop
     // and kept in scratch)
     const int key_l = key;
     int hh_l = hh;
-    if (LIST) asm volatile("" : "+v"(hh_l));
+    if (LIST || LIM) asm volatile("" : "+v"(hh_l));
     const bool ok = !DSROLE || key_l < S;
     const T* src = DSROLE ? v + (((int64_t)b * S + (ok ? key_l : 0)) * Hkv + g) * D + 8 * hh_l
                              : krot + ((int64_t)bh * P + key_l) * D + 8 * hh_l;
@@ -295,8 +296,9 @@ __device__ __forceinline__ void dkdv_role(
     const DkdvStage<T, D>& S_ = st[buf];
     const int e = entry(it);
     const int q0 = tile_of(e) * BQ;
-    const int rel = key - q0;  // rows r of this tile see the key when r >= rel
-    const bool diag = causal && q0 < k0 + BKV;
+    // rows r of this tile see the key when r >= rel (LIM: none a key past nkeys)
+    const int rel = LIM && key >= nkeys ? INT_MAX : key - q0;
+    const bool diag = (causal && q0 < k0 + BKV) || (LIM && k0 + BKV > nkeys);
     const bool dmask = LIST && (e & DOC_MASK_FLAG);
 
     // this lane's 32 rows' -lse / scale (P waves) or -Delta (dS waves), the
@@ -468,7 +470,7 @@ __device__ __forceinline__ void dkdv_role(
   }
   const int key_e = key;
   int hoff = 4 * hh;
-  if (LIST) asm volatile("" : "+v"(hoff));
+  if (LIST || LIM) asm volatile("" : "+v"(hoff));
   if (DSROLE) {
     T* dkr = dk + (((int64_t)b * S + key_e) * Hkv + g) * D + hoff;
     const float* cr = cos + (int64_t)key_e * HALF + hoff;
@@ -517,12 +519,12 @@ __device__ __forceinline__ void dkdv_stage_first(
   if (w == 2) dma4(lds_addr(sqd), (uint32_t)min(q0 + lane, S - 1) * 4u, drow);
 }
 
-// kpm_flags (causal key padding; per batch row, 1 = every key valid): rows
-// without padding run the unmasked kernel (SPLIT), the others the KPM one,
-// which runs after it and skips the rows without padding; the unmasked launch
-// walks no query tile for the padded rows' items (their dK / dV are written
-// as zeros, then overwritten by the KPM launch).
-template <typename T, int D, int MODE, bool STORE, bool SPLIT = false, bool PART = false>
+// kpm_keys (causal key padding; kpm_row_keys_kernel): the batch rows whose valid
+// keys are the first kpm_keys[b] run the unmasked kernel (LIM), the others
+// (kpm_keys 0) the KPM one, which runs after it and skips the former; the
+// unmasked launch walks no query tile for the latter's items (their dK / dV
+// are written as zeros, then overwritten by the KPM launch).
+template <typename T, int D, int MODE, bool STORE, bool LIM = false, bool PART = false>
 __global__ __launch_bounds__(512, 1) void bwd_dkdv_kernel(
     const T* __restrict__ krot, const T* __restrict__ v, const T* __restrict__ qrot,
     const T* __restrict__ dout, const float* __restrict__ lse2, const float* __restrict__ delta,
@@ -530,7 +532,7 @@ __global__ __launch_bounds__(512, 1) void bwd_dkdv_kernel(
     T* __restrict__ dv, int S, int P, int Hq, int Hkv, int n_rep, int nkb, int nitems,
     float scale_log2,
     float scale, int causal, const int32_t* __restrict__ aux, const int2* __restrict__ ranges,
-    u32x4* __restrict__ dsb, const int* __restrict__ order, const int* __restrict__ kpm_flags,
+    u32x4* __restrict__ dsb, const int* __restrict__ order, const int* __restrict__ kpm_keys,
     int nsplit, float* __restrict__ dkp, float* __restrict__ dvp, int64_t part_stride) {
   constexpr bool DOC = MODE == MASK_DOC, KPM = MODE == MASK_KPM;
   __shared__ __attribute__((aligned(16))) DkdvStage<T, D> st[2];
@@ -565,14 +567,15 @@ __global__ __launch_bounds__(512, 1) void bwd_dkdv_kernel(
       const int bk = order[rank / Hkv];
       logical = ((bk / nkb) * Hkv + rank % Hkv) * nkb + bk % nkb;
     }
-    const int bh = logical / nkb;
+    int bh = logical / nkb;
     const int kb = logical % nkb;  // ascending: the longest causal key tiles first
+    if (LIM || KPM) bh = kpm_head(bh, nitems / (nkb * nsplit) / Hkv, Hkv);
     const int b = bh / Hkv, g = bh % Hkv;
     const int k0 = kb * BKV;
     const int32_t* drow = DOC || KPM ? aux + (int64_t)b * S : nullptr;
     const int2* rec = ranges + (int64_t)b * (P / BN);
-    if (KPM && kpm_flags != nullptr && kpm_flags[b] != 0) continue;
-    const bool live = !SPLIT || kpm_flags[b] != 0;
+    if (KPM && kpm_keys != nullptr && kpm_keys[b] != 0) continue;
+    const int nkeys = LIM ? kpm_keys[b] : S;
     int nlist = 0, fv = 0;
     if constexpr (KPM) {
       if (w == 0) {
@@ -611,16 +614,16 @@ __global__ __launch_bounds__(512, 1) void bwd_dkdv_kernel(
       nlist = __builtin_amdgcn_readfirstlane(sCount);
     }
     if (w >= 4)
-      dkdv_role<T, D, true, MODE, STORE, PART>(st, sP, krot, v, qrot, dout, lse2, delta, cos, sin, dk,
+      dkdv_role<T, D, true, MODE, STORE, LIM, PART>(st, sP, krot, v, qrot, dout, lse2, delta, cos, sin, dk,
                                       dv, S, P, Hq, Hkv, n_rep, b, g, bh, k0, w, lane,
                                       scale_log2, scale, causal, drow, sList, nlist, sQD, fv,
-                                      dsb, P / DSQ, live, part, nsplit,
+                                      dsb, P / DSQ, nkeys, part, nsplit,
                                       PART ? dkp + part * part_stride : nullptr);
     else
-      dkdv_role<T, D, false, MODE, STORE, PART>(st, sP, krot, v, qrot, dout, lse2, delta, cos, sin, dk,
+      dkdv_role<T, D, false, MODE, STORE, LIM, PART>(st, sP, krot, v, qrot, dout, lse2, delta, cos, sin, dk,
                                        dv, S, P, Hq, Hkv, n_rep, b, g, bh, k0, w, lane,
                                        scale_log2, scale, causal, drow, sList, nlist, sQD, fv,
-                                       dsb, P / DSQ, live, part, nsplit,
+                                       dsb, P / DSQ, nkeys, part, nsplit,
                                        PART ? dvp + part * part_stride : nullptr);
     __syncthreads();  // LDS of this item is free for the next
   }
@@ -697,8 +700,9 @@ __global__ __launch_bounds__(512, 1) void bwd_dq_kernel(
   // persistent: one block of rows per round
   const XcdItems xi = xcd_items(nitems);
   for (int rnd = 0;; ++rnd) {
-    const int logical = xcd_item(xi, rnd);
+    int logical = xcd_item(xi, rnd);
     if (logical < 0) break;
+    if (KPM) logical = kpm_head(logical / nqb, nitems / nqb / Hkv, Hkv) * nqb + logical % nqb;
     // kpm_skip_clean: the batch rows whose key 0 is valid have their dQ from
     // the dS records (bwd_dq_ds); this launch serves the others
     if (KPM && kpm_skip_clean &&
@@ -955,7 +959,8 @@ __global__ __launch_bounds__(64 * HB) void bwd_dq_ds_kernel(
   const int ngrp = n_rep / HB;
   const int logical = xcd_logical_id(blockIdx.x, gridDim.x, nqt);
   const int qt = nqt - 1 - logical % nqt;
-  const int hg = (logical / nqt) % ngrp, bh = logical / nqt / ngrp;
+  const int hg = (logical / nqt) % ngrp, hidx = logical / nqt / ngrp;
+  const int bh = KPM ? kpm_head(hidx, gridDim.x / (nqt * ngrp) / Hkv, Hkv) : hidx;
   const int b = bh / Hkv, g = bh % Hkv;
   const int nqtp = P / DSQ;
   int nk = causal ? min(2 * qt + 2, (S + DSK - 1) / DSK) : (S + DSK - 1) / DSK;
@@ -1506,13 +1511,13 @@ int launch_bwd(const BwdArgs& a, void* workspace, bool keep_ds) {
   const int grid_cap = a.doc || a.kvalid ? INT_MAX : device_cu_count() / 8 * 8;
   const int mode = a.doc ? MASK_DOC : a.kvalid ? MASK_KPM : MASK_NONE;
   const int32_t* aux = a.doc ? a.doc : a.kvalid;
-  // causal key padding: the batch rows whose keys are all valid go to the
-  // unmasked (persistent) kernel first, the rest to the KPM one
-  const int* kpm_flags = mode == MASK_KPM && a.causal ? w.counts : nullptr;
+  // causal key padding: the batch rows padded on the right only (or not at
+  // all) go to the unmasked (persistent) kernel first, the rest to the KPM one
+  const int* kpm_keys = mode == MASK_KPM && a.causal ? w.counts : nullptr;
   // Small grids (dkdv_small_grid) take the unmasked kernel's PART variant,
-  // whose float32 parts dkdv_reduce adds; key padding's rows without padding
-  // take the same variant as an unmasked launch, so an all-True mask gives the
-  // unmasked result bit for bit
+  // whose float32 parts dkdv_reduce adds; key padding's rows of the unmasked
+  // kernel take the same variant as an unmasked launch, so an all-True mask
+  // gives the unmasked result bit for bit
   const int64_t part_stride = (int64_t)a.B * a.Hkv * a.S * D;
   const bool small = dkdv_small_grid(a.B, a.S, a.Hq, a.Hkv);
   auto reduce_parts = [&](int nsplit, float* dkp, float* dvp) {
@@ -1523,8 +1528,8 @@ int launch_bwd(const BwdArgs& a, void* workspace, bool keep_ds) {
               nsplit, part_stride, a.cos, a.sin, (T*)a.dk, (T*)a.dv, a.S, a.Hkv, a.scale,
               (int)nrows);
   };
-  if (kpm_flags) {
-    const int rc = launch_kpm_row_flags(w.ranges, P / BN, a.S, a.B, w.counts, a.stream);
+  if (kpm_keys) {
+    const int rc = launch_kpm_row_keys(a.kvalid, a.S, a.B, w.counts, a.stream);
     if (rc) return rc;
     const int ns = dkdv_splits(a.B, a.S, a.Hq, a.Hkv);
     float* dkp = small ? w.dkvp : nullptr;
@@ -1538,7 +1543,7 @@ int launch_bwd(const BwdArgs& a, void* workspace, bool keep_ds) {
               dim3(std::min(ni, device_cu_count() / 8 * 8)), dim3(512), 0, a.stream,
               (const T*)w.krot, (const T*)a.v, (const T*)w.qrot, (const T*)a.dout, w.lse2, w.delta,
               a.cos, a.sin, (T*)a.dk, (T*)a.dv, a.S, P, a.Hq, a.Hkv, n_rep, nkb, ni, scale_log2,
-              a.scale, a.causal, nullptr, w.ranges, w.dsb, nullptr, kpm_flags, ns, dkp, dvp,
+              a.scale, a.causal, nullptr, w.ranges, w.dsb, nullptr, kpm_keys, ns, dkp, dvp,
               part_stride);
     if (small) reduce_parts(ns, dkp, dvp);
   }
@@ -1559,7 +1564,7 @@ int launch_bwd(const BwdArgs& a, void* workspace, bool keep_ds) {
             dim3(std::min(nitems, grid_cap)), dim3(512), 0, a.stream, (const T*)w.krot,
             (const T*)a.v, (const T*)w.qrot, (const T*)a.dout, w.lse2, w.delta, a.cos, a.sin,
             (T*)a.dk, (T*)a.dv, a.S, P, a.Hq, a.Hkv, n_rep, nkb, nitems, scale_log2, a.scale,
-            a.causal, aux, w.ranges, w.dsb, order, kpm_flags, nsplit, dkp, dvp, part_stride);
+            a.causal, aux, w.ranges, w.dsb, order, kpm_keys, nsplit, dkp, dvp, part_stride);
   if (part) reduce_parts(nsplit, dkp, dvp);
   KF_CHECK_LAUNCH();
   if (keep_ds) {

@@ -214,7 +214,7 @@ __global__ __launch_bounds__(256, 2) void fwd_mfma_kernel(
     float* __restrict__ lse, int Sq, int Sk, int Skp, int krows, int Hq, int Hkv, int n_rep,
     int bm_pos, int nqb, float scale_log2, int causal, const int32_t* __restrict__ aux,
     const int2* __restrict__ ranges, T* __restrict__ qrot, const int* __restrict__ order,
-    const int* __restrict__ kpm_flags) {
+    const int* __restrict__ kpm_keys) {
   constexpr bool DOC = MODE == MASK_DOC, KPM = MODE == MASK_KPM, LIST = DOC || KPM;
   constexpr int KS = D / 16, DT = D / 32;
   constexpr int KR = D / 8;  // 16-byte chunks per K / V row
@@ -233,6 +233,8 @@ __global__ __launch_bounds__(256, 2) void fwd_mfma_kernel(
     const int bq = order[blockIdx.x / Hkv];
     logical = ((bq / nqb) * Hkv + (int)blockIdx.x % Hkv) * nqb + (nqb - 1 - bq % nqb);
   }
+  if (KPM)
+    logical = kpm_head(logical / nqb, gridDim.x / nqb / Hkv, Hkv) * nqb + logical % nqb;
   const RowInfo ri = row_info(logical, nqb, Hkv, n_rep, bm_pos, Sq, w * 32 + c32);
   const int bh = ri.b * Hkv + ri.g;
 
@@ -240,8 +242,8 @@ __global__ __launch_bounds__(256, 2) void fwd_mfma_kernel(
   int ntiles = (kend + BN - 1) / BN;
   const int32_t* arow = LIST ? aux + (int64_t)ri.b * Sk : nullptr;
   const int2* rec = ranges + (int64_t)ri.b * (Skp / BN);
-  // kpm_flags (per batch row, 1 = every key valid): those rows are fwd32_kernel's
-  if (KPM && kpm_flags != nullptr && kpm_flags[ri.b] != 0) return;
+  // the rows whose valid keys are a prefix are fwd32_kernel's (kpm_row_keys_kernel)
+  if (KPM && kpm_keys != nullptr && kpm_keys[ri.b] != 0) return;
   const T* kbase = krot + (int64_t)bh * krows * D;
   const T* vbase = vn + (int64_t)bh * D * Skp;  // V^T, keys in fragment order
   auto stage = [&](int t, int buf) {
@@ -488,18 +490,24 @@ __global__ __launch_bounds__(256, 3) void fwd32_kernel(
     const T* __restrict__ krot, const T* __restrict__ vn, T* __restrict__ out,
     float* __restrict__ lse, int Sq, int Sk, int Skp, int krows, int Hq, int Hkv, int n_rep,
     int bm_pos, int nqb, float scale_log2, int causal, T* __restrict__ qrot,
-    const int* __restrict__ kpm_flags) {
+    const int* __restrict__ kpm_keys) {
   constexpr int KS = D / 16, DT = D / 32;
   constexpr int KR = D / 8;  // 16-byte chunks per K row
   __shared__ __attribute__((aligned(16))) T sK[2][FBN * D];
   __shared__ __attribute__((aligned(16))) T sV[2][D * FBN];
 
   const int tid = threadIdx.x, w = wave_id(), lane = tid & 63, hh = lane >> 5, c32 = lane & 31;
-  const int logical = xcd_logical_id(blockIdx.x, gridDim.x, nqb);
+  int logical = xcd_logical_id(blockIdx.x, gridDim.x, nqb);
+  if (kpm_keys != nullptr)
+    logical = kpm_head(logical / nqb, gridDim.x / nqb / Hkv, Hkv) * nqb + logical % nqb;
   const RowInfo ri = row_info(logical, nqb, Hkv, n_rep, bm_pos, Sq, w * 32 + c32);
-  // key padding (kpm_flags per batch row, 1 = every key valid): only the rows
-  // without padding (plain causal attention); fwd_mfma_kernel takes the others
-  if (kpm_flags != nullptr && kpm_flags[ri.b] == 0) return;
+  // key padding: the batch rows whose valid keys are the first kpm_keys[b]
+  // (0: none such; fwd_mfma_kernel takes the row), which is causal attention
+  // over that many keys
+  if (kpm_keys != nullptr) {
+    Sk = kpm_keys[ri.b];
+    if (Sk == 0) return;
+  }
   const int bh = ri.b * Hkv + ri.g;
   const int kend = causal ? min(Sk, min(ri.p0 + bm_pos, Sq)) : Sk;
   const int ntiles = (kend + FBN - 1) / FBN;
@@ -1048,20 +1056,39 @@ int launch_kv_prep(const FwdArgs& a, void* krot, int krows, void* vn, int Skp, i
 }
 
 namespace {
-// flags[b] = 1 when every key of batch row b is valid (from its tile records),
-// else 0: one wavefront per batch row
-__global__ __launch_bounds__(64) void kpm_row_flags_kernel(const int2* __restrict__ ranges,
-                                                           int rstride, int S,
-                                                           int* __restrict__ flags) {
-  const bool all = kpm_all_valid(ranges + (int64_t)blockIdx.x * rstride, S, threadIdx.x);
-  if (threadIdx.x == 0) flags[blockIdx.x] = all ? 1 : 0;
+// keys[b] = n when the valid keys of batch row b are exactly the first n > 0
+// (right padding, or none), else 0.  One workgroup per batch row: a prefix has
+// its last valid key at position count - 1.
+__global__ __launch_bounds__(256) void kpm_row_keys_kernel(const int32_t* __restrict__ kvalid,
+                                                           int S, int* __restrict__ keys) {
+  __shared__ int sN[4], sLast[4];
+  const int32_t* row = kvalid + (int64_t)blockIdx.x * S;
+  int n = 0, last = -1;
+#pragma unroll 4
+  for (int j = threadIdx.x; j < S; j += 256)
+    if (row[j] != 0) {
+      ++n;
+      last = j;
+    }
+  last = wave_max_i(last);
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) n += __shfl_xor(n, o, 64);
+  const int w = threadIdx.x >> 6;
+  if ((threadIdx.x & 63) == 0) {
+    sN[w] = n;
+    sLast[w] = last;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    n = sN[0] + sN[1] + sN[2] + sN[3];
+    last = max(max(sLast[0], sLast[1]), max(sLast[2], sLast[3]));
+    keys[blockIdx.x] = last + 1 == n ? n : 0;
+  }
 }
 }  // namespace
 
-int launch_kpm_row_flags(const int2* ranges, int rstride, int S, int B, int* flags,
-                         hipStream_t stream) {
-  KF_LAUNCH("kpm_row_flags", kpm_row_flags_kernel, dim3(B), dim3(64), 0, stream, ranges, rstride,
-            S, flags);
+int launch_kpm_row_keys(const int32_t* kvalid, int S, int B, int* keys, hipStream_t stream) {
+  KF_LAUNCH("kpm_row_keys", kpm_row_keys_kernel, dim3(B), dim3(256), 0, stream, kvalid, S, keys);
   KF_CHECK_LAUNCH();
   return KF_OK;
 }
@@ -1105,20 +1132,20 @@ int mask_mode(const FwdArgs& a) { return a.doc ? MASK_DOC : a.kvalid ? MASK_KPM 
 
 template <typename T, int D, int MODE>
 void launch_fwd_kernel(const FwdArgs& a, const FwdWs& w, int Skp, int n_rep, int bm_pos, int nqb,
-                       unsigned nblk, const int* order, const int* kpm_flags = nullptr) {
+                       unsigned nblk, const int* order, const int* kpm_keys = nullptr) {
   KF_LAUNCH("fwd_mfma", (fwd_mfma_kernel<T, D, MODE>), dim3(nblk), dim3(256), 0, a.stream,
             (const T*)a.q, a.cos, a.sin, (const T*)w.krot, (const T*)w.vn, (T*)a.out, a.lse, a.Sq,
             a.Sk, Skp, w.krows, a.Hq, a.Hkv, n_rep, bm_pos, nqb, a.scale * kLog2e, a.causal,
-            a.doc ? a.doc : a.kvalid, w.ranges, (T*)w.qrot, order, kpm_flags);
+            a.doc ? a.doc : a.kvalid, w.ranges, (T*)w.qrot, order, kpm_keys);
 }
 
 template <typename T, int D>
 void launch_fwd32(const FwdArgs& a, const FwdWs& w, int Skp, int n_rep, int bm_pos, int nqb,
-                  unsigned nblk, const int* kpm_flags) {
+                  unsigned nblk, const int* kpm_keys) {
   KF_LAUNCH("fwd_mfma", (fwd32_kernel<T, D>), dim3(nblk), dim3(256), 0, a.stream, (const T*)a.q,
             a.cos, a.sin, (const T*)w.krot, (const T*)w.vn, (T*)a.out, a.lse, a.Sq, a.Sk, Skp,
             w.krows, a.Hq, a.Hkv, n_rep, bm_pos, nqb, a.scale * kLog2e, a.causal, (T*)w.qrot,
-            kpm_flags);
+            kpm_keys);
 }
 
 template <typename T, int D>
@@ -1129,13 +1156,13 @@ void launch_fwd_mode(const FwdArgs& a, const FwdWs& w, int Skp, int n_rep, int b
       launch_fwd_kernel<T, D, MASK_DOC>(a, w, Skp, n_rep, bm_pos, nqb, nblk, w.order);
       break;
     case MASK_KPM:
-      // causal self-attention: batch rows without padding run the unmasked
-      // kernel, the others the masked one (each launch skips the other's rows)
+      // batch rows padded on the right only (or not at all) run the unmasked
+      // kernel with that many keys, the others the masked one (each launch
+      // skips the other's rows); w.counts holds the rows' key counts
     {
-      // (w.counts holds the per-row flags: launch_kpm_row_flags in fwd_mfma)
-      const int* flags = a.causal && a.Sq == a.Sk ? w.counts : nullptr;
-      if (flags) launch_fwd32<T, D>(a, w, Skp, n_rep, bm_pos, nqb, nblk, flags);
-      launch_fwd_kernel<T, D, MASK_KPM>(a, w, Skp, n_rep, bm_pos, nqb, nblk, nullptr, flags);
+      const int* keys = a.causal && a.Sq == a.Sk ? w.counts : nullptr;
+      if (keys) launch_fwd32<T, D>(a, w, Skp, n_rep, bm_pos, nqb, nblk, keys);
+      launch_fwd_kernel<T, D, MASK_KPM>(a, w, Skp, n_rep, bm_pos, nqb, nblk, nullptr, keys);
       break;
     }
     default: launch_fwd32<T, D>(a, w, Skp, n_rep, bm_pos, nqb, nblk, nullptr);
@@ -1184,7 +1211,7 @@ int fwd_mfma(const FwdArgs& a, void* workspace) {
     if (rc) return rc;
   }
   if (a.kvalid && a.causal && a.Sq == a.Sk) {
-    rc = launch_kpm_row_flags(w.ranges, Skp / BN, a.Sk, a.B, w.counts, a.stream);
+    rc = launch_kpm_row_keys(a.kvalid, a.Sk, a.B, w.counts, a.stream);
     if (rc) return rc;
   }
   const bool h = a.dtype == F16;

@@ -390,18 +390,13 @@ __device__ __forceinline__ int kpm_first_valid(const int2* __restrict__ rec, int
   return INT_MAX;
 }
 
-// True when every key of the batch row is valid (tile t holds min(64, S - 64 t)
-// valid keys), from the row's tile records; wavefront-uniform.  Such a row is
-// plain causal attention: the launches with key padding hand its rows to the
-// unmasked kernels.
-__device__ __forceinline__ bool kpm_all_valid(const int2* __restrict__ rec, int S, int lane) {
-  const int ntiles = (S + BN - 1) / BN;
-  bool short_tile = false;
-  for (int base = 0; base < ntiles; base += 64) {
-    const int t = base + lane;
-    if (t < ntiles) short_tile |= rec[t].x != min(BN, S - BN * t);
-  }
-  return __builtin_amdgcn_ballot_w64(short_tile) == 0;
+// Launches with key padding number their (batch row, KV head) groups with the
+// batch rows fastest: group idx of B * Hkv.  An XCD takes a contiguous range of
+// groups, and with a batch row's heads adjacent the XCDs of short (or skipped)
+// rows ran dry: six rows of 1531 positions, each XCD holding the heads of one or
+// two rows, took 1.29 ms forward and backward.
+__device__ __forceinline__ int kpm_head(int idx, int B, int Hkv) {
+  return (idx % B) * Hkv + idx / B;
 }
 
 // Lists, in ascending order, tiles t in [t0, t1) for which pick(t, rec[t])
