@@ -167,7 +167,7 @@ struct DkdvStage {
 // MASK_KPM: qlist as above, drow the key-validity row, fv the first valid
 // key's position: query rows before it (guarded) see every key, other rows
 // need the key valid and not after them.
-template <typename T, int D, bool DSROLE, int MODE, bool STORE, bool LIM, bool PART>
+template <typename T, int D, bool DSROLE, int MODE, bool STORE, bool LIM, bool PART, bool DEAL>
 __device__ __forceinline__ void dkdv_role(
     DkdvStage<T, D>* st, u32x4* sP, const T* __restrict__ krot, const T* __restrict__ v,
     const T* __restrict__ qrot, const T* __restrict__ dout,
@@ -224,10 +224,10 @@ __device__ __forceinline__ void dkdv_role(
     // +inf, so they contribute nothing)
     tile_to_lds<BQ, KR, 8, LIST>(dout + (((int64_t)b * S + q0) * Hq + hq) * D, Hq * D, S_.o, w,
                                  lane, S - q0);
-    if (LIST || PART || LIM) {
+    if (LIST || PART || DEAL) {
       // the row statistics' LDS addresses from the stage array's base plus
       // constant offsets: with the pointer into the stage member, the masked,
-      // split and key-limited kernels fail to compile ("Operand has incorrect register
+      // split and dealt kernels fail to compile ("Operand has incorrect register
       // class": a constant generic-to-LDS address cast lowered with an
       // illegal null test)
       using Stage = DkdvStage<T, D>;
@@ -250,12 +250,12 @@ __device__ __forceinline__ void dkdv_role(
   // for P waves, V (read in place, [B, S, Hkv, D]; zero past S) for dS waves
   bf16x8 bf[KS];
   {
-    // (masked and key-limited modes: key and half laundered, so that the 64-bit row address
+    // (masked and dealt kernels: key and half laundered, so that the 64-bit row address
     // is formed here per item rather than hoisted out of the persistent loop
     // and kept in scratch)
     const int key_l = key;
     int hh_l = hh;
-    if (LIST || LIM) asm volatile("" : "+v"(hh_l));
+    if (LIST || DEAL) asm volatile("" : "+v"(hh_l));
     const bool ok = !DSROLE || key_l < S;
     const T* src = DSROLE ? v + (((int64_t)b * S + (ok ? key_l : 0)) * Hkv + g) * D + 8 * hh_l
                              : krot + ((int64_t)bh * P + key_l) * D + 8 * hh_l;
@@ -470,7 +470,7 @@ __device__ __forceinline__ void dkdv_role(
   }
   const int key_e = key;
   int hoff = 4 * hh;
-  if (LIST || LIM) asm volatile("" : "+v"(hoff));
+  if (LIST || DEAL) asm volatile("" : "+v"(hoff));
   if (DSROLE) {
     T* dkr = dk + (((int64_t)b * S + key_e) * Hkv + g) * D + hoff;
     const float* cr = cos + (int64_t)key_e * HALF + hoff;
@@ -524,7 +524,10 @@ __device__ __forceinline__ void dkdv_stage_first(
 // (kpm_keys 0) the KPM one, which runs after it and skips the former; the
 // unmasked launch walks no query tile for the latter's items (their dK / dV
 // are written as zeros, then overwritten by the KPM launch).
-template <typename T, int D, int MODE, bool STORE, bool LIM = false, bool PART = false>
+// DEAL: the items dealt longest first over all groups (dealt_order) instead of
+// group by group; dkdv_deal says when.
+template <typename T, int D, int MODE, bool STORE, bool LIM = false, bool PART = false,
+          bool DEAL = LIM>
 __global__ __launch_bounds__(512, 1) void bwd_dkdv_kernel(
     const T* __restrict__ krot, const T* __restrict__ v, const T* __restrict__ qrot,
     const T* __restrict__ dout, const float* __restrict__ lse2, const float* __restrict__ delta,
@@ -546,11 +549,11 @@ __global__ __launch_bounds__(512, 1) void bwd_dkdv_kernel(
   // query heads (unmasked kernels only)
   const XcdItems xi = xcd_items(nitems);
   for (int rnd = 0;; ++rnd) {
-    // PART (the small-grid variant): the shares dealt longest first over all
-    // (KV head, part) groups of nkb key blocks
+    // DEAL, PART (the small-grid variant): the shares dealt longest first over
+    // all KV heads' (PART: parts') groups of nkb key blocks
     int logical = xcd_item(xi, rnd);
     if (logical < 0) break;
-    if (PART) logical = dealt_order(logical, nitems, nkb);
+    if (PART || DEAL) logical = dealt_order(logical, nitems, nkb);
     // PART items are numbered (KV head, part, key block), key blocks fastest,
     // so an XCD's contiguous share holds whole longest-first sweeps of key
     // blocks (wavefront-uniform; readfirstlane keeps the staging bases scalar)
@@ -614,13 +617,13 @@ __global__ __launch_bounds__(512, 1) void bwd_dkdv_kernel(
       nlist = __builtin_amdgcn_readfirstlane(sCount);
     }
     if (w >= 4)
-      dkdv_role<T, D, true, MODE, STORE, LIM, PART>(st, sP, krot, v, qrot, dout, lse2, delta, cos, sin, dk,
+      dkdv_role<T, D, true, MODE, STORE, LIM, PART, DEAL>(st, sP, krot, v, qrot, dout, lse2, delta, cos, sin, dk,
                                       dv, S, P, Hq, Hkv, n_rep, b, g, bh, k0, w, lane,
                                       scale_log2, scale, causal, drow, sList, nlist, sQD, fv,
                                       dsb, P / DSQ, nkeys, part, nsplit,
                                       PART ? dkp + part * part_stride : nullptr);
     else
-      dkdv_role<T, D, false, MODE, STORE, LIM, PART>(st, sP, krot, v, qrot, dout, lse2, delta, cos, sin, dk,
+      dkdv_role<T, D, false, MODE, STORE, LIM, PART, DEAL>(st, sP, krot, v, qrot, dout, lse2, delta, cos, sin, dk,
                                        dv, S, P, Hq, Hkv, n_rep, b, g, bh, k0, w, lane,
                                        scale_log2, scale, causal, drow, sList, nlist, sQD, fv,
                                        dsb, P / DSQ, nkeys, part, nsplit,
@@ -1380,6 +1383,19 @@ int dkdv_splits(int B, int S, int Hq, int Hkv) {
   return n;
 }
 
+// Whether an unmasked, unsplit dK/dV launch deals its items longest first over
+// all KV heads.  Group by group (fewer heads' query tiles in flight on an XCD)
+// the zigzag rounds of G workgroups pair long items with short ones only when
+// a round holds whole sweeps of key blocks or a sweep whole rounds.  Measured
+// (32 query heads of 128, dK/dV alone, group by group / dealt): S = 1531, B = 6
+// 430 / 293 us, S = 3000, B = 4 820 / 663, S = 5000, B = 2 (64 heads) 2159 /
+// 1816; balanced either way, S = 4096, B = 4 1160 / 1170 and S = 16384 (64 heads)
+// 9219 / 9330.
+bool dkdv_deal(int nkb) {
+  const int G = device_cu_count() / 8;
+  return G % nkb != 0 && nkb % G != 0;
+}
+
 size_t align256(size_t n) { return (n + 255) / 256 * 256; }
 
 // Whether the unmasked dK/dV launch takes the small-grid variant (PART):
@@ -1559,6 +1575,8 @@ int launch_bwd(const BwdArgs& a, void* workspace, bool keep_ds) {
                                            : bwd_dkdv_kernel<T, D, MASK_KPM, false>)
              : part             ? (keep_ds ? bwd_dkdv_kernel<T, D, MASK_NONE, true, false, true>
                                            : bwd_dkdv_kernel<T, D, MASK_NONE, false, false, true>)
+             : dkdv_deal(nkb)   ? (keep_ds ? bwd_dkdv_kernel<T, D, MASK_NONE, true, false, false, true>
+                                           : bwd_dkdv_kernel<T, D, MASK_NONE, false, false, false, true>)
              : keep_ds          ? bwd_dkdv_kernel<T, D, MASK_NONE, true>
                                 : bwd_dkdv_kernel<T, D, MASK_NONE, false>),
             dim3(std::min(nitems, grid_cap)), dim3(512), 0, a.stream, (const T*)w.krot,
