@@ -667,6 +667,9 @@ __global__ __launch_bounds__(256, 3) void fwd32_kernel(
     lse[((int64_t)rl.b * Hq + rl.hq) * Sq + rl.pos] = (m + log2f(ltot)) * kLn2;
 }
 
+// four floats at a 4-byte aligned address (global vector accesses need no more)
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+
 // Capture: LSE, the probabilities P = exp(s - lse) as float32 [B, Hq, Sq, Sk]
 // and out = P·V in one launch; a workgroup takes the query blocks r and
 // nqb-1-r of one KV head, one after the other.  The workgroup walks a block's
@@ -808,7 +811,11 @@ __global__ __launch_bounds__(256, 2) void capture_probs_mfma_kernel(
     // in 2*ntiles pieces, one at the start of each tile iteration of the two
     // walks (ahead of that iteration's tile loads), so the zeros stream out
     // while the block computes instead of after it.
-    const bool vec4 = (Sk & 3) == 0;  // 16-byte aligned rows
+    // Rows that start off 64-byte blocks leave by write-back stores, which L2
+    // joins into whole lines: a non-temporal store of part of a block is a
+    // partial write to memory (S = 3000: 433 against 530 us; on whole blocks
+    // non-temporal is ahead, 270 against 361 at S = 2000, 64 heads).
+    const bool nt = (Sk & 15) == 0;
     const int zstart = ntiles * BN;
     const int zper = causal && zstart < Sk ? (nrows + 2 * ntiles - 1) / (2 * ntiles) : 0;
     auto zero_rows = [&](int z) {
@@ -819,10 +826,12 @@ __global__ __launch_bounds__(256, 2) void capture_probs_mfma_kernel(
         float* zrow =
             probs + (((int64_t)ri.b * Hq + (int64_t)ri.g * n_rep + r / bm_pos) * Sq + pos) * Sk;
         for (int key = zstart + tid * 4; key < Sk; key += 256 * 4) {
-          if (vec4) {
+          if (nt) {
             __builtin_nontemporal_store(f32x4{0.f, 0.f, 0.f, 0.f}, (f32x4*)(zrow + key));
+          } else if (key + 3 < Sk) {
+            *(f32x4u*)(zrow + key) = f32x4u{0.f, 0.f, 0.f, 0.f};
           } else {
-            for (int e = key; e < min(key + 4, Sk); ++e) zrow[e] = 0.f;
+            for (int e = key; e < Sk; ++e) zrow[e] = 0.f;
           }
         }
       }
@@ -907,7 +916,7 @@ __global__ __launch_bounds__(256, 2) void capture_probs_mfma_kernel(
     f32x16 held[2];  // P of the previous tile, stored by the next
     // true when every lane of store_p(t)'s 8 store instructions is active, so
     // that exactly 8 vector-memory instructions issue
-    auto full_p = [&](int t) { return pvalid == 15 && vec4 && (t + 1) * BN <= Sk; };
+    auto full_p = [&](int t) { return pvalid == 15 && (t + 1) * BN <= Sk; };
     auto store_p = [&](int t) {
 #pragma unroll
       for (int mt = 0; mt < 2; ++mt) {
@@ -922,11 +931,13 @@ __global__ __launch_bounds__(256, 2) void capture_probs_mfma_kernel(
           const f32x4 v4 = *(const f32x4*)&stg[rr * 32 + ((cl ^ (rr & 7)) * 4)];
           const int key = t * BN + 32 * mt + 4 * cl;
           if (!((pvalid >> j) & 1)) continue;
-          if (vec4) {
+          if (nt) {
             if (key < Sk) __builtin_nontemporal_store(v4, (f32x4*)(prs[j] + key));
+          } else if (key + 3 < Sk) {
+            *(f32x4u*)(prs[j] + key) = v4;
           } else {
 #pragma unroll
-            for (int e = 0; e < 4; ++e)
+            for (int e = 0; e < 3; ++e)
               if (key + e < Sk) prs[j][key + e] = v4[e];
           }
         }
@@ -999,6 +1010,115 @@ __global__ __launch_bounds__(256, 2) void capture_probs_mfma_kernel(
         }
     }
   }
+}
+
+// Probabilities of a small capture after the forward (out and lse): P =
+// exp(s - lse) recomputed tile by tile, a workgroup taking CAP_TILES 64-key
+// tiles of one query block (zeros right of the causal frontier).  The fused
+// kernel above has one workgroup per pair of query blocks, each walking its
+// key tiles twice, and at a few hundred positions that leaves most CUs idle and
+// the rest in a serial chain; here the work is as many independent workgroups
+// as there are pieces of P, at the price of the forward's P·V rows computed in
+// a launch of their own.  Store layout as in the fused kernel.
+constexpr int CAP_TILES = 4;
+template <typename T, int D>
+__global__ __launch_bounds__(256, 3) void capture_tiles_kernel(
+    const T* __restrict__ q, const float* __restrict__ cos, const float* __restrict__ sin,
+    const T* __restrict__ krot, const float* __restrict__ lse, float* __restrict__ probs, int Sq,
+    int Sk, int Skp, int Hq, int Hkv, int n_rep, int bm_pos, int nqb, int nch, float scale_log2,
+    int causal) {
+  constexpr int KS = D / 16, KR = D / 8;
+  __shared__ __attribute__((aligned(16))) T sK[2][BN * D];
+  __shared__ __attribute__((aligned(16))) float sP[4][32 * 32];  // per wave: 32 rows x 32 keys
+
+  const int w = wave_id(), lane = threadIdx.x & 63, hh = lane >> 5, c32 = lane & 31;
+  const int logical = xcd_logical_id(blockIdx.x, gridDim.x, nqb * nch);
+  const RowInfo ri = row_info(logical / nch, nqb, Hkv, n_rep, bm_pos, Sq, w * 32 + c32);
+  const int bh = ri.b * Hkv + ri.g;
+  const int ntiles = (Sk + BN - 1) / BN;
+  const int t0 = (logical % nch) * CAP_TILES, t1 = min(t0 + CAP_TILES, ntiles);
+  // tiles from tv on lie right of the block's last row
+  const int qmax = min(ri.p0 + bm_pos, Sq) - 1;
+  const int tv = causal ? min(t1, max(t0, qmax / BN + 1)) : t1;
+  const T* kbase = krot + (int64_t)bh * Skp * D;
+  auto stage = [&](int t, int buf) {
+    tile_to_lds<BN, KR>(kbase + (int64_t)t * BN * D, D, sK[buf], w, lane);
+  };
+  if (t0 < tv) stage(t0, 0);
+
+  // lane l stores rows 8 j + l / 8 (j = 0..3) of the wavefront, keys 4 (l % 8) .. + 3
+  const bool nt = (Sk & 15) == 0;  // as in the fused kernel
+  const int cl = lane & 7;
+  float* prs[4];
+  int pvalid = 0;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const RowInfo rj =
+        row_info(logical / nch, nqb, Hkv, n_rep, bm_pos, Sq, w * 32 + 8 * j + (lane >> 3));
+    pvalid |= (int)rj.q_valid << j;
+    prs[j] = probs + (((int64_t)rj.b * Hq + rj.hq) * Sq + (rj.q_valid ? rj.pos : 0)) * Sk + 4 * cl;
+  }
+  auto put4 = [&](int j, int k, const f32x4& x) {  // keys k + 4 cl .. + 3 of row j
+    if (!((pvalid >> j) & 1)) return;
+    const int key = k + 4 * cl;
+    if (nt) {
+      if (key < Sk) __builtin_nontemporal_store(x, (f32x4*)(prs[j] + k));
+    } else if (key + 3 < Sk) {
+      *(f32x4u*)(prs[j] + k) = x;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 3; ++e)
+        if (key + e < Sk) prs[j][k + e] = x[e];
+    }
+  };
+
+  if (t0 < tv) {
+    bf16x8 qf[KS];
+    load_q_frag<T, D>(q, cos, sin, ri, Sq, Hq, hh, qf);
+    const float L =
+        ri.q_valid ? lse[((int64_t)ri.b * Hq + ri.hq) * Sq + ri.pos] * kLog2e : 0.f;
+    float* stg = sP[w];
+    lds_copy_wait();
+    __syncthreads();
+    for (int t = t0; t < tv; ++t) {
+      const int buf = (t - t0) & 1, k0 = t * BN;
+      if (t + 1 < tv) stage(t + 1, buf ^ 1);
+      const int lim = (causal ? min(ri.pos, Sk - 1) : Sk - 1) - k0;  // last visible key
+      f32x16 s[2];
+#pragma unroll
+      for (int mt = 0; mt < 2; ++mt) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s[mt][i] = 0.f;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks)
+          s[mt] = mfma32<T>(lds_frag<KR>(sK[buf], 32 * mt + c32, 2 * ks + hh), qf[ks], s[mt]);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const float p = fast_exp2(__builtin_fmaf(s[mt][i], scale_log2, -L));
+          s[mt][i] = 32 * mt + 8 * (i >> 2) + 4 * hh + (i & 3) > lim ? 0.f : p;
+        }
+      }
+      // the wait before the stores: they count in vmcnt, and issued first they
+      // would hold the tile loads' wait until they are written
+      lds_copy_wait();
+#pragma unroll
+      for (int mt = 0; mt < 2; ++mt) {
+#pragma unroll
+        for (int g4 = 0; g4 < 4; ++g4)
+          *(f32x4*)&stg[c32 * 32 + (((2 * g4 + hh) ^ (c32 & 7)) * 4)] =
+              f32x4{s[mt][4 * g4], s[mt][4 * g4 + 1], s[mt][4 * g4 + 2], s[mt][4 * g4 + 3]};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int rr = 8 * j + (lane >> 3);
+          put4(j, k0 + 32 * mt, *(const f32x4*)&stg[rr * 32 + ((cl ^ (rr & 7)) * 4)]);
+        }
+      }
+      __syncthreads();
+    }
+  }
+  for (int k = tv * BN; k < t1 * BN; k += 32)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) put4(j, k, f32x4{0.f, 0.f, 0.f, 0.f});
 }
 
 int pick_bm_pos(int n_rep) { return n_rep <= ROWS ? ROWS / n_rep : 0; }
@@ -1226,9 +1346,48 @@ int fwd_mfma(const FwdArgs& a, void* workspace) {
   return KF_OK;
 }
 
+namespace {
+template <typename T, int D>
+void launch_capture_tiles(const FwdArgs& a, const FwdWs& w, float* probs, int Skp) {
+  const int n_rep = a.Hq / a.Hkv, bm_pos = pick_bm_pos(n_rep);
+  const int nqb = (a.Sq + bm_pos - 1) / bm_pos;
+  const int nch = (Skp / BN + CAP_TILES - 1) / CAP_TILES;
+  KF_LAUNCH("capture_probs_mfma", (capture_tiles_kernel<T, D>),
+            dim3((unsigned)(nqb * nch * a.B * a.Hkv)), dim3(256), 0, a.stream, (const T*)a.q,
+            a.cos, a.sin, (const T*)w.krot, a.lse, probs, a.Sq, a.Sk, Skp, a.Hq, a.Hkv, n_rep,
+            bm_pos, nqb, nch, a.scale * kLog2e, a.causal);
+}
+}  // namespace
+
+// Whether the probabilities are formed after the forward (capture_tiles_kernel)
+// instead of in the fused kernel: when the latter would have less than one
+// workgroup per CU.  Whole capture, fused / after the forward (D 128, one
+// sequence): 8 workgroups (S = 128, 32/8 heads) 53 / 26 us, 104 (S = 777) 145 /
+// 58, 128 (S = 1024) 119 / 76, 192 (S = 1536) 147 / 121, 256 (S = 2000) 168 /
+// 199, 512 (S = 2048, 64/8 heads) 257 / 335.  Explicit masks stay fused.
+bool capture_after_fwd(const FwdArgs& a) {
+  if (a.doc || a.kvalid) return false;
+  const int bm_pos = pick_bm_pos(a.Hq / a.Hkv), nqb = (a.Sq + bm_pos - 1) / bm_pos;
+  return (int64_t)((nqb + 1) / 2) * a.B * a.Hkv < device_cu_count();
+}
+
 int capture_probs_mfma(const FwdArgs& a, float* probs, void* workspace) {
   const int Skp = (a.Sk + BN - 1) / BN * BN;
   const FwdWs w = carve_fwd(a, workspace, Skp);
+  if (capture_after_fwd(a)) {
+    const int rc = fwd_mfma(a, workspace);
+    if (rc) return rc;
+    const bool h = a.dtype == F16;
+    if (a.D == 128) {
+      if (h) launch_capture_tiles<f16, 128>(a, w, probs, Skp);
+      else launch_capture_tiles<bf16, 128>(a, w, probs, Skp);
+    } else {
+      if (h) launch_capture_tiles<f16, 64>(a, w, probs, Skp);
+      else launch_capture_tiles<bf16, 64>(a, w, probs, Skp);
+    }
+    KF_CHECK_LAUNCH();
+    return KF_OK;
+  }
   int rc = launch_kv_prep(a, w.krot, Skp, w.vn, Skp, w.ranges, KV_V_TRANSPOSED);
   if (rc) return rc;
   const int n_rep = a.Hq / a.Hkv;

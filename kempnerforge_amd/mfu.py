@@ -163,7 +163,7 @@ def attention_kernel_flops(pairs: int, head_dim: int, backward: bool = True) -> 
 
 # ---------------------------------------------------------------- profiler
 _ATTN_KEYS = ("fwd_mfma", "bwd_dkdv", "bwd_dq", "q_prep_bwd", "kv_prep", "decode_stream",
-              "decode_merge", "decode_generic", "capture_probs", "fwd_generic",
+              "decode_merge", "decode_generic", "capture_probs", "capture_tiles", "fwd_generic",
               "bwd_dq_generic", "bwd_dkdv_generic", "cache_append", "append_kernel",
               "doc_block_tiles", "order_by_count", "widen_kernel", "narrow_kernel", "_f32_kernel",
               "kf::attn", "flash", "fmha", "attention")
