@@ -15,10 +15,12 @@ only accept GPU tensors: there is no CPU path.
 from __future__ import annotations
 
 import ctypes
+import functools
 import weakref
 from typing import Optional
 
 import torch
+from torch.autograd.function import once_differentiable
 
 from kempnerforge_amd import _lib
 
@@ -35,19 +37,29 @@ def _dtype_code(t: torch.Tensor) -> int:
 
 def _require_gpu(*ts: torch.Tensor) -> None:
     for t in ts:
-        if t.device.type != "cuda":
+        if not t.is_cuda:
             raise RuntimeError(
                 "kempnerforge_amd attention runs only on a ROCm GPU (gfx950); got a tensor on "
                 f"{t.device}. There is no CPU fallback."
             )
 
 
-def _stream(t: torch.Tensor) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+# (ctypes takes plain ints where the signatures say void pointer)
+def _stream(t: torch.Tensor) -> int:
+    return torch._C._cuda_getCurrentRawStream(t.device.index)
 
 
-def _ptr(t: torch.Tensor | None) -> ctypes.c_void_p:
-    return ctypes.c_void_p(0 if t is None else t.data_ptr())
+def _ptr(t: torch.Tensor | None) -> int:
+    return 0 if t is None else t.data_ptr()
+
+
+@functools.lru_cache(maxsize=4096)
+def _size(entry: str, device: int, *sizes: int) -> int:
+    """Bytes from a ``*_workspace_size`` entry point, asked once per sizes
+    (``device``: the library sizes some workspaces by its compute units)."""
+    n = _lib.size_out()
+    _lib.check(getattr(_lib.load(), entry)(*sizes, ctypes.byref(n)), entry)
+    return n.value
 
 
 def _aligned(t: torch.Tensor) -> torch.Tensor:
@@ -127,10 +139,8 @@ def fwd_raw(q, k, v, cos, sin, *, causal: bool, k_rotated: bool, k_layout: str =
     dt = _dtype_code(q)
     out = torch.empty_like(q)
     lse = torch.empty(B, Hq, Sq, dtype=torch.float32, device=q.device)
-    nbytes = _lib.size_out()
-    _lib.check(lib.kf_attn_fwd_workspace_size(B, Sq, Sk, Hq, Hkv, D, dt, ctypes.byref(nbytes)),
-               "kf_attn_fwd_workspace_size")
-    ws = _workspace(nbytes.value, q.device)
+    ws = _workspace(_size("kf_attn_fwd_workspace_size", q.device.index, B, Sq, Sk, Hq, Hkv, D, dt),
+                    q.device)
     _lib.check(lib.kf_attn_fwd(_ptr(q), _ptr(k), _ptr(v), _ptr(cos), _ptr(sin), _ptr(out),
                                _ptr(lse), _ptr(ws), ws.numel(), B, Sq, Sk, Hq, Hkv, D, *kstr,
                                *vstr, int(k_rotated), int(causal), _ptr(doc), _ptr(kv), dt,
@@ -239,22 +249,18 @@ def bwd_raw(q, k, v, cos, sin, out, lse, dout, *, causal: bool, doc_ids=None,
     kv = _key_valid(key_padding_mask, B, S, q.device)
     dt = _dtype_code(q)
     dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
-    nbytes = _lib.size_out()
-    _lib.check(lib.kf_attn_bwd_workspace_size(B, S, Hq, Hkv, D, dt, ctypes.byref(nbytes)),
-               "kf_attn_bwd_workspace_size")
+    nbytes = _size("kf_attn_bwd_workspace_size", q.device.index, B, S, Hq, Hkv, D, dt)
     low_memory = _BWD_LOW_MEMORY if low_memory is None else low_memory
     # key padding keeps dS only causally, and only for the batch rows whose key
     # 0 is valid (decided on the device; the others recompute)
     if not low_memory and (kv is None or causal):
-        with_ds = _lib.size_out()
-        _lib.check(lib.kf_attn_bwd_workspace_size_ds(B, S, Hq, Hkv, D, dt, int(causal),
-                                                     ctypes.byref(with_ds)),
-                   "kf_attn_bwd_workspace_size_ds")
+        with_ds = _size("kf_attn_bwd_workspace_size_ds", q.device.index, B, S, Hq, Hkv, D, dt,
+                        int(causal))
         key = ("bwd", q.device, B, S, Hq, Hkv, D, q.dtype, bool(causal), doc is not None,
                kv is not None)
-        if _keep_ds_for(key, with_ds.value - nbytes.value, q.device):
+        if _keep_ds_for(key, with_ds - nbytes, q.device):
             nbytes = with_ds
-    ws = _workspace(nbytes.value, q.device)
+    ws = _workspace(nbytes, q.device)
     _lib.check(lib.kf_attn_bwd(_ptr(q), _ptr(k), _ptr(v), _ptr(cos), _ptr(sin), _ptr(out),
                                _ptr(lse), _ptr(dout), _ptr(dq), _ptr(dk), _ptr(dv), _ptr(ws),
                                ws.numel(), B, S, Hq, Hkv, D, int(causal), _ptr(doc), _ptr(kv),
@@ -266,6 +272,7 @@ def bwd_raw(q, k, v, cos, sin, out, lse, dout, *, causal: bool, doc_ids=None,
 _KF_ERR_UNSUPPORTED = 2
 
 
+@functools.lru_cache(maxsize=4096)
 def rot_size(B: int, S: int, Hq: int, Hkv: int, D: int, dtype: torch.dtype, has_doc: bool,
              has_key_padding: bool) -> int:
     """Bytes of the rotated-operand buffer of :func:`fwd_rot_raw`, or 0 when that
@@ -318,10 +325,8 @@ def fwd_rot_raw(q, k, v, cos, sin, *, causal: bool, doc_ids=None, key_padding_ma
     out = torch.empty_like(q)
     lse = torch.empty(B, Hq, S, dtype=torch.float32, device=q.device)
     rot = torch.empty(nrot // q.element_size(), dtype=q.dtype, device=q.device)
-    nbytes = _lib.size_out()
-    _lib.check(lib.kf_attn_fwd_workspace_size(B, S, S, Hq, Hkv, D, dt, ctypes.byref(nbytes)),
-               "kf_attn_fwd_workspace_size")
-    ws = _workspace(nbytes.value, q.device)
+    ws = _workspace(_size("kf_attn_fwd_workspace_size", q.device.index, B, S, S, Hq, Hkv, D, dt),
+                    q.device)
     rc = lib.kf_attn_fwd_rot(_ptr(q), _ptr(k), _ptr(v), _ptr(cos), _ptr(sin), _ptr(out),
                              _ptr(lse), _ptr(rot), _ptr(ws), ws.numel(), B, S, Hq, Hkv, D,
                              int(causal), _ptr(doc), _ptr(kv), dt, _stream(q))
@@ -357,21 +362,17 @@ def bwd_rot_raw(rot, v, cos, sin, out, lse, dout, *, causal: bool, doc_ids=None,
             f"{rot.numel() * rot.element_size()} bytes of {rot.dtype} on {rot.device}")
     dt = _dtype_code(out)
     dq, dk, dv = torch.empty_like(out), torch.empty_like(v), torch.empty_like(v)
-    nbytes = _lib.size_out()
-    _lib.check(lib.kf_attn_bwd_rot_workspace_size(B, S, Hq, Hkv, D, dt, int(causal), 0,
-                                                  ctypes.byref(nbytes)),
-               "kf_attn_bwd_rot_workspace_size")
+    sizes = ("kf_attn_bwd_rot_workspace_size", out.device.index, B, S, Hq, Hkv, D, dt,
+             int(causal))
+    nbytes = _size(*sizes, 0)
     low_memory = _BWD_LOW_MEMORY if low_memory is None else low_memory
     if not low_memory and (kv is None or causal):  # as in bwd_raw
-        with_ds = _lib.size_out()
-        _lib.check(lib.kf_attn_bwd_rot_workspace_size(B, S, Hq, Hkv, D, dt, int(causal), 1,
-                                                      ctypes.byref(with_ds)),
-                   "kf_attn_bwd_rot_workspace_size")
+        with_ds = _size(*sizes, 1)
         key = ("bwd_rot", out.device, B, S, Hq, Hkv, D, out.dtype, bool(causal), doc is not None,
                kv is not None)
-        if _keep_ds_for(key, with_ds.value - nbytes.value, out.device):
+        if _keep_ds_for(key, with_ds - nbytes, out.device):
             nbytes = with_ds
-    ws = _workspace(nbytes.value, out.device)
+    ws = _workspace(nbytes, out.device)
     _lib.check(lib.kf_attn_bwd_rot(_ptr(rot), _ptr(v), _ptr(cos), _ptr(sin), _ptr(out),
                                    _ptr(lse), _ptr(dout), _ptr(dq), _ptr(dk), _ptr(dv),
                                    _ptr(ws), ws.numel(), B, S, Hq, Hkv, D, int(causal),
@@ -404,6 +405,7 @@ def decode_raw(q_new, k_new, v_new, k_cache, v_cache, lens, cos, sin, *, rope_ro
         qnw, knw = (_norm_weight(w, D, q_new.device) for w in (q_norm_weight, k_norm_weight))
     dt = _dtype_code(q_new)
     out = torch.empty_like(q_new)
+    # (max_len grows every step: asked per step, not kept)
     nbytes = _lib.size_out()
     _lib.check(lib.kf_attn_decode_workspace_size(B, Hq, Hkv, D, max_len, dt, ctypes.byref(nbytes)),
                "kf_attn_decode_workspace_size")
@@ -483,10 +485,8 @@ def capture_raw(q, k, v, cos, sin, *, causal: bool, k_rotated: bool, k_layout: s
     out = torch.empty_like(q)
     lse = torch.empty(B, Hq, Sq, dtype=torch.float32, device=q.device)
     probs = torch.empty(B, Hq, Sq, Sk, dtype=torch.float32, device=q.device)
-    nbytes = _lib.size_out()
-    _lib.check(lib.kf_attn_capture_workspace_size(B, Sq, Sk, Hq, Hkv, D, dt, ctypes.byref(nbytes)),
-               "kf_attn_capture_workspace_size")
-    ws = _workspace(nbytes.value, q.device)
+    ws = _workspace(_size("kf_attn_capture_workspace_size", q.device.index, B, Sq, Sk, Hq, Hkv, D,
+                          dt), q.device)
     _lib.check(lib.kf_attn_capture(_ptr(q), _ptr(k), _ptr(v), _ptr(cos), _ptr(sin), _ptr(probs),
                                    _ptr(out), _ptr(lse), _ptr(ws), ws.numel(), B, Sq, Sk, Hq, Hkv,
                                    D, *kstr, *vstr, int(k_rotated), int(causal), _ptr(doc),
@@ -586,6 +586,61 @@ def _backward(ctx, dout, dlse, drot):
 attn_fwd.register_autograd(_backward, setup_context=_setup_context)
 
 
+class _Attention(torch.autograd.Function):
+    """The autograd formula of ``kf::attn_fwd`` without the dispatcher: what
+    :func:`attention` applies in plain eager calls.  Registering the op costs a
+    Python call per dispatch key and direction (about 100 us of host time per
+    training pass), which is most of a small layer's step."""
+
+    @staticmethod
+    def forward(ctx, q, k, v, cos, sin, causal, doc_ids, key_padding_mask):
+        res = fwd_rot_raw(q, k, v, cos, sin, causal=causal, doc_ids=doc_ids,
+                          key_padding_mask=key_padding_mask)
+        ctx.set_materialize_grads(False)
+        ctx.causal = causal
+        ctx.use_rot = res is not None
+        if res is not None:
+            out, lse, rot = res
+            ctx.save_for_backward(rot, v, cos, sin, out, lse, doc_ids, key_padding_mask)
+        else:
+            out, lse = fwd_raw(q, k, v, cos, sin, causal=causal, k_rotated=False,
+                               doc_ids=doc_ids, key_padding_mask=key_padding_mask)
+            ctx.save_for_backward(q, k, v, cos, sin, out, lse, doc_ids, key_padding_mask)
+        return out
+
+    @staticmethod
+    @once_differentiable
+    def backward(ctx, dout):
+        if dout is None:
+            return (None,) * 8
+        if ctx.use_rot:
+            rot, v, cos, sin, out, lse, doc_ids, key_padding_mask = ctx.saved_tensors
+            grads = bwd_rot_raw(rot, v, cos, sin, out, lse, dout, causal=ctx.causal,
+                                doc_ids=doc_ids, key_padding_mask=key_padding_mask)
+        else:
+            q, k, v, cos, sin, out, lse, doc_ids, key_padding_mask = ctx.saved_tensors
+            grads = bwd_raw(q, k, v, cos, sin, out, lse, dout, causal=ctx.causal,
+                            doc_ids=doc_ids, key_padding_mask=key_padding_mask)
+        return grads + (None,) * 5
+
+
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
+
+
+def _plain_eager(*ts) -> bool:
+    """Whether nothing but autograd looks at this call: plain GPU tensors, and
+    no tracer, function transform, forward-mode level or dispatch / function
+    mode (compile, export, fake tensors, selective checkpointing, vmap, jvp ...)
+    that has to see the registered operator."""
+    if (torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() > 0
+            or torch._C._len_torch_function_stack() > 0
+            or torch._C._get_tracing_state() is not None
+            or torch._C._functorch.peek_interpreter_stack() is not None
+            or torch.autograd.forward_ad._current_level >= 0):
+        return False
+    return all(t is None or (type(t) in _PLAIN and t.is_cuda) for t in ts)
+
+
 def attention(q, k, v, rope_cos, rope_sin, *, causal: bool = True, doc_ids=None,
               key_padding_mask=None) -> torch.Tensor:
     """Differentiable RoPE + GQA + (causal) attention on BSHD tensors.
@@ -603,6 +658,12 @@ def attention(q, k, v, rope_cos, rope_sin, *, causal: bool = True, doc_ids=None,
     # written (q and k rotated, (B*Hkv + B*Hq)*S*D elements) and never read
     keep_rot = torch.is_grad_enabled() and (q.requires_grad or k.requires_grad
                                             or v.requires_grad)
+    if _plain_eager(q, k, v, rope_cos, rope_sin, doc_ids, key_padding_mask):
+        if keep_rot:
+            return _Attention.apply(q, k, v, rope_cos, rope_sin, causal, doc_ids,
+                                    key_padding_mask)
+        return fwd_raw(q, k, v, rope_cos, rope_sin, causal=causal, k_rotated=False,
+                       doc_ids=doc_ids, key_padding_mask=key_padding_mask)[0]
     out, _, _ = attn_fwd(q, k, v, rope_cos, rope_sin, causal, doc_ids, key_padding_mask,
                          keep_rot)
     return out
