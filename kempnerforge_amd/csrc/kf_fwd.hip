@@ -483,24 +483,34 @@ __global__ __launch_bounds__(256, 2) void fwd_mfma_kernel(
 // 64-key tiles).  Same rows per workgroup and the same per-key arithmetic as
 // fwd_mfma_kernel; the running max is taken per 32-key tile, so the points
 // where the output is rescaled (and with them the last bits) can differ.
-constexpr int FBN = 32;  // keys per tile of fwd32_kernel
-template <typename T, int D>
-__global__ __launch_bounds__(256, 3) void fwd32_kernel(
+//
+// KSL = 2, for grids that leave the chip idle: a workgroup takes half the rows
+// (64) and its wavefronts split the keys, wavefront w the rows 32 (w / 2) ..
+// + 31 over the 32-key half w % 2 of each 64-key tile.  A small causal grid
+// runs as long as its longest row block's chain of tiles, whatever the total
+// work; this halves the chain and doubles the blocks.  Both halves' (max, sum,
+// O) meet in LDS after the loop, in float32.  fwd_slices says when.
+constexpr int FBN = 32;  // keys per wavefront and tile of fwd32_kernel
+template <typename T, int D, int KSL>
+__global__ __launch_bounds__(256, KSL == 1 ? 3 : 2) void fwd32_kernel(
     const T* __restrict__ q, const float* __restrict__ cos, const float* __restrict__ sin,
     const T* __restrict__ krot, const T* __restrict__ vn, T* __restrict__ out,
     float* __restrict__ lse, int Sq, int Sk, int Skp, int krows, int Hq, int Hkv, int n_rep,
     int bm_pos, int nqb, float scale_log2, int causal, T* __restrict__ qrot,
     const int* __restrict__ kpm_keys) {
   constexpr int KS = D / 16, DT = D / 32;
-  constexpr int KR = D / 8;  // 16-byte chunks per K row
-  __shared__ __attribute__((aligned(16))) T sK[2][FBN * D];
-  __shared__ __attribute__((aligned(16))) T sV[2][D * FBN];
+  constexpr int KR = D / 8;       // 16-byte chunks per K row
+  constexpr int TK = FBN * KSL;   // keys per staged tile
+  __shared__ __attribute__((aligned(16))) T sK[2][TK * D];
+  __shared__ __attribute__((aligned(16))) T sV[2][D * TK];
+  __shared__ float sML[KSL == 1 ? 1 : 2][2][64];  // per row group: (max, sum) of the second half
 
   const int tid = threadIdx.x, w = wave_id(), lane = tid & 63, hh = lane >> 5, c32 = lane & 31;
+  const int rg = w / KSL, sl = w % KSL;  // row group, key half
   int logical = xcd_logical_id(blockIdx.x, gridDim.x, nqb);
   if (kpm_keys != nullptr)
     logical = kpm_head(logical / nqb, gridDim.x / nqb / Hkv, Hkv) * nqb + logical % nqb;
-  const RowInfo ri = row_info(logical, nqb, Hkv, n_rep, bm_pos, Sq, w * 32 + c32);
+  const RowInfo ri = row_info(logical, nqb, Hkv, n_rep, bm_pos, Sq, rg * 32 + c32);
   // key padding: the batch rows whose valid keys are the first kpm_keys[b]
   // (0: none such; fwd_mfma_kernel takes the row), which is causal attention
   // over that many keys
@@ -510,12 +520,12 @@ __global__ __launch_bounds__(256, 3) void fwd32_kernel(
   }
   const int bh = ri.b * Hkv + ri.g;
   const int kend = causal ? min(Sk, min(ri.p0 + bm_pos, Sq)) : Sk;
-  const int ntiles = (kend + FBN - 1) / FBN;
+  const int ntiles = (kend + TK - 1) / TK;
   const T* kbase = krot + (int64_t)bh * krows * D;
   const T* vbase = vn + (int64_t)bh * D * Skp;  // V^T, keys in fragment order
   auto stage = [&](int t, int buf) {
-    tile_to_lds<FBN, KR>(kbase + (int64_t)t * FBN * D, D, sK[buf], w, lane);
-    tile_to_lds<D, FBN / 8>(vbase + (int64_t)t * FBN, Skp, sV[buf], w, lane);
+    tile_to_lds<TK, KR>(kbase + (int64_t)t * TK * D, D, sK[buf], w, lane);
+    tile_to_lds<D, TK / 8>(vbase + (int64_t)t * TK, Skp, sV[buf], w, lane);
   };
   if (ntiles > 0) stage(0, 0);
 
@@ -523,6 +533,11 @@ __global__ __launch_bounds__(256, 3) void fwd32_kernel(
   load_q_frag<T, D>(q, cos, sin, ri, Sq, Hq, hh, qf);
 
   float m = -INFINITY, lsum = 0.f;
+  // KSL 2: a half may hold no visible key for a while, or at all, its max still
+  // -inf: no inf - inf then (a factor of 1, an exponent base of 0)
+  auto factor = [](float from, float to) {
+    return KSL == 2 && from == to ? 1.f : fast_exp2(from - to);
+  };
   f32x16 acc[DT];
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt)
@@ -537,12 +552,12 @@ __global__ __launch_bounds__(256, 3) void fwd32_kernel(
     const T* tK = sK[buf];
     const T* tV = sV[buf];
 
-    // S^T of the tile's 32 keys x this wavefront's 32 rows
+    // S^T of the half tile's 32 keys x this wavefront's 32 rows
     f32x16 s;
 #pragma unroll
     for (int i = 0; i < 16; ++i) s[i] = 0.f;
     {
-      auto kfrag = [&](int j) { return lds_frag<KR>(tK, c32, 2 * j + hh); };
+      auto kfrag = [&](int j) { return lds_frag<KR>(tK, FBN * sl + c32, 2 * j + hh); };
       bf16x8 fa[KS];
 #pragma unroll
       for (int j = 0; j < FWD_PF; ++j) fa[j] = kfrag(j);
@@ -555,7 +570,7 @@ __global__ __launch_bounds__(256, 3) void fwd32_kernel(
       __builtin_amdgcn_sched_barrier(0);
     }
 
-    const int k0 = it * FBN;
+    const int k0 = it * TK + FBN * sl;
     if ((causal && k0 + FBN - 1 > ri.p0) || (k0 + FBN > Sk)) {
       // last visible key of this lane's row, relative to k0 (branch-free select)
       const int lim = (causal ? min(ri.pos, Sk - 1) : Sk - 1) - k0;
@@ -571,7 +586,7 @@ __global__ __launch_bounds__(256, 3) void fwd32_kernel(
     tmax = pair_max32(tmax) * scale_log2;
     if (__builtin_amdgcn_ballot_w64(tmax > m + RESCALE_SLACK) != 0) {
       const float mnew = fmaxf(m, tmax);
-      const float alpha = fast_exp2(m - mnew);
+      const float alpha = factor(m, mnew);
       lsum *= alpha;
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt)
@@ -579,12 +594,13 @@ __global__ __launch_bounds__(256, 3) void fwd32_kernel(
         for (int i = 0; i < 16; ++i) acc[dt][i] *= alpha;
       m = mnew;
     }
+    const float base = KSL == 2 && m == -INFINITY ? 0.f : m;
     float psum = 0.f;
     u32x4 pk[2];
 #pragma unroll
     for (int i = 0; i < 16; i += 2) {
-      const float p0 = fast_exp2(__builtin_fmaf(s[i], scale_log2, -m));
-      const float p1 = fast_exp2(__builtin_fmaf(s[i + 1], scale_log2, -m));
+      const float p0 = fast_exp2(__builtin_fmaf(s[i], scale_log2, -base));
+      const float p1 = fast_exp2(__builtin_fmaf(s[i + 1], scale_log2, -base));
       psum += p0 + p1;
       pk[i >> 3][(i & 7) >> 1] = pack2<T>(p0, p1);
     }
@@ -592,7 +608,7 @@ __global__ __launch_bounds__(256, 3) void fwd32_kernel(
     {
       constexpr int NV = 2 * DT;
       auto vfrag = [&](int j) {
-        return lds_frag<FBN / 8>(tV, 32 * (j % DT) + c32, 2 * (j / DT) + hh);
+        return lds_frag<TK / 8>(tV, 32 * (j % DT) + c32, FBN / 8 * sl + 2 * (j / DT) + hh);
       };
       bf16x8 fb[NV];
 #pragma unroll
@@ -613,46 +629,85 @@ __global__ __launch_bounds__(256, 3) void fwd32_kernel(
     if (it + 1 < ntiles) tile_body(it + 1, std::integral_constant<int, 1>{});
   }
 
+  if constexpr (KSL == 2) {
+    // the second half's sums to the first half's wavefront (the tile buffers
+    // are free after the loop's last barrier)
+    f32x4* slab = (f32x4*)(rg == 0 ? sK[0] : sV[0]);  // 64 lanes x DT x 16 floats = TK * D * 2 B
+    if (sl == 1) {
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int gi = 0; gi < 4; ++gi)
+          slab[(4 * dt + gi) * 64 + lane] = f32x4{acc[dt][4 * gi], acc[dt][4 * gi + 1],
+                                                  acc[dt][4 * gi + 2], acc[dt][4 * gi + 3]};
+      sML[rg][0][lane] = m;
+      sML[rg][1][lane] = lsum;
+    }
+    __syncthreads();
+    if (sl == 0) {
+      const float m1 = sML[rg][0][lane], mnew = fmaxf(m, m1);
+      const float a0 = factor(m, mnew), a1 = factor(m1, mnew);
+      m = mnew;
+      lsum = lsum * a0 + sML[rg][1][lane] * a1;
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int gi = 0; gi < 4; ++gi) {
+          const f32x4 o = slab[(4 * dt + gi) * 64 + lane];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[dt][4 * gi + e] = acc[dt][4 * gi + e] * a0 + o[e] * a1;
+        }
+    }
+    __syncthreads();
+  }
   const float ltot = pair_sum32(lsum);
   const float inv = 1.f / ltot;
   // The output leaves through LDS (the tile buffers are free after the loop's
   // last barrier): each wavefront writes its 32 rows into its own 32 x D slice,
   // 16-byte chunks XOR-swizzled by row, then stores whole 16-byte chunks, each
   // row by KR consecutive lanes, so a store instruction covers 64 / KR whole
-  // rows instead of 16 bytes of each of 32 rows.
-  T* slice = w < 2 ? sK[w] : sV[w - 2];  // FBN x D elements = 32 rows x D
+  // rows instead of 16 bytes of each of 32 rows.  (KSL 2: one slice per row
+  // group, written by its first wavefront and stored by both, half the rows each.)
+  T* slice = KSL == 1 ? (w < 2 ? sK[w] : sV[w - 2]) : sK[rg];  // 32 rows x D
+  constexpr int NST = 32 * KR / 64 / KSL;  // store instructions per wavefront
+  if (KSL == 1 || sl == 0) {
 #pragma unroll
-  for (int dt = 0; dt < DT; ++dt)
+    for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-    for (int gi = 0; gi < 4; ++gi) {
-      const int ch = 4 * dt + gi;  // 16-byte chunk of columns 32 dt + 8 gi ..
-      u32x2 pk2;
-      pk2[0] = pack2<T>(acc[dt][4 * gi] * inv, acc[dt][4 * gi + 1] * inv);
-      pk2[1] = pack2<T>(acc[dt][4 * gi + 2] * inv, acc[dt][4 * gi + 3] * inv);
-      *(u32x2*)(slice + (c32 * KR + (ch ^ (c32 & (KR - 1)))) * 8 + 4 * hh) = pk2;
-    }
+      for (int gi = 0; gi < 4; ++gi) {
+        const int ch = 4 * dt + gi;  // 16-byte chunk of columns 32 dt + 8 gi ..
+        u32x2 pk2;
+        pk2[0] = pack2<T>(acc[dt][4 * gi] * inv, acc[dt][4 * gi + 1] * inv);
+        pk2[1] = pack2<T>(acc[dt][4 * gi + 2] * inv, acc[dt][4 * gi + 3] * inv);
+        *(u32x2*)(slice + (c32 * KR + (ch ^ (c32 & (KR - 1)))) * 8 + 4 * hh) = pk2;
+      }
+  }
   __syncthreads();
 #pragma unroll
-  for (int i2 = 0; i2 < 32 * KR / 64; ++i2) {
-    const int L = 64 * i2 + lane, row = L / KR, ch = L % KR;
+  for (int i2 = 0; i2 < NST; ++i2) {
+    const int L = 64 * (NST * sl + i2) + lane, row = L / KR, ch = L % KR;
     const u32x4 v = *(const u32x4*)(slice + (row * KR + (ch ^ (row & (KR - 1)))) * 8);
-    const RowInfo rj = row_info(logical, nqb, Hkv, n_rep, bm_pos, Sq, w * 32 + row);
+    const RowInfo rj = row_info(logical, nqb, Hkv, n_rep, bm_pos, Sq, rg * 32 + row);
     if (rj.q_valid) *(u32x4*)(out + (((int64_t)rj.b * Sq + rj.pos) * Hq + rj.hq) * D + 8 * ch) = v;
   }
   if (qrot != nullptr) {
     // the rotated q rows for the backward, the same way (read there long after:
     // streaming stores); fragment ks holds the row's 16-byte chunk c below
+    if (KSL == 2) __syncthreads();  // the slice's other wavefront has read it
+    if (KSL == 1 || sl == 0) {
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      const int c = ks < KS / 2 ? 2 * ks + hh : KR / 2 + 2 * (ks - KS / 2) + hh;
-      *(u32x4*)(slice + (c32 * KR + (c ^ (c32 & (KR - 1)))) * 8) = __builtin_bit_cast(u32x4, qf[ks]);
+      for (int ks = 0; ks < KS; ++ks) {
+        const int c = ks < KS / 2 ? 2 * ks + hh : KR / 2 + 2 * (ks - KS / 2) + hh;
+        *(u32x4*)(slice + (c32 * KR + (c ^ (c32 & (KR - 1)))) * 8) =
+            __builtin_bit_cast(u32x4, qf[ks]);
+      }
     }
     __syncthreads();
 #pragma unroll
-    for (int i2 = 0; i2 < 32 * KR / 64; ++i2) {
-      const int L = 64 * i2 + lane, row = L / KR, ch = L % KR;
+    for (int i2 = 0; i2 < NST; ++i2) {
+      const int L = 64 * (NST * sl + i2) + lane, row = L / KR, ch = L % KR;
       const u32x4 v = *(const u32x4*)(slice + (row * KR + (ch ^ (row & (KR - 1)))) * 8);
-      const RowInfo rj = row_info(logical, nqb, Hkv, n_rep, bm_pos, Sq, w * 32 + row);
+      const RowInfo rj = row_info(logical, nqb, Hkv, n_rep, bm_pos, Sq, rg * 32 + row);
       if (rj.q_valid)
         __builtin_nontemporal_store(
             v, (u32x4*)(qrot + (((int64_t)rj.b * Hq + rj.hq) * krows + rj.pos) * D + 8 * ch));
@@ -660,10 +715,10 @@ __global__ __launch_bounds__(256, 3) void fwd32_kernel(
   }
   // this row's LSE: its index recomputed here from a laundered row number, so
   // the prologue's 64-bit value is not kept live (in scratch) across the loop
-  int r_l = w * 32 + c32;
+  int r_l = rg * 32 + c32;
   asm volatile("" : "+v"(r_l));
   const RowInfo rl = row_info(logical, nqb, Hkv, n_rep, bm_pos, Sq, r_l);
-  if (rl.q_valid && lse != nullptr && hh == 0)
+  if (rl.q_valid && lse != nullptr && hh == 0 && (KSL == 1 || sl == 0))
     lse[((int64_t)rl.b * Hq + rl.hq) * Sq + rl.pos] = (m + log2f(ltot)) * kLn2;
 }
 
@@ -1259,13 +1314,31 @@ void launch_fwd_kernel(const FwdArgs& a, const FwdWs& w, int Skp, int n_rep, int
             a.doc ? a.doc : a.kvalid, w.ranges, (T*)w.qrot, order, kpm_keys);
 }
 
+// Key slices per workgroup of an unmasked forward of nblk 128-row blocks: two
+// up to one block per CU (D 64, whose two slices still leave four workgroups
+// per CU: three).  A wavefront's chain of tiles is then what the launch lasts
+// (0.8 us per tile, whatever the ring depth: three or four staged tiles gained
+// nothing).  One / two slices, forward kernel alone: D 128, 32/8 heads S = 256
+// 14.9 / 13.0 us, 512 19.2 / 16.7, 1000 (256 blocks) 28.9 / 26.1, 1999 (504) 54.9
+// / 56.7, 3000 (752) 91 / 105; D 64, 12 heads S = 2048 37 / 27, B = 2 S = 1024 22.7
+// / 18.1, B = 4 S = 2048 (768) 62 / 51.
+int fwd_slices(int64_t nblk, int n_rep, int D) {
+  return n_rep <= ROWS / 2 && nblk <= (D == 64 ? 3 : 1) * (int64_t)device_cu_count() ? 2 : 1;
+}
+
 template <typename T, int D>
 void launch_fwd32(const FwdArgs& a, const FwdWs& w, int Skp, int n_rep, int bm_pos, int nqb,
                   unsigned nblk, const int* kpm_keys) {
-  KF_LAUNCH("fwd_mfma", (fwd32_kernel<T, D>), dim3(nblk), dim3(256), 0, a.stream, (const T*)a.q,
-            a.cos, a.sin, (const T*)w.krot, (const T*)w.vn, (T*)a.out, a.lse, a.Sq, a.Sk, Skp,
-            w.krows, a.Hq, a.Hkv, n_rep, bm_pos, nqb, a.scale * kLog2e, a.causal, (T*)w.qrot,
-            kpm_keys);
+  const int ksl = fwd_slices(nblk, n_rep, D);
+  if (ksl == 2) {
+    bm_pos = ROWS / 2 / n_rep;
+    nqb = (a.Sq + bm_pos - 1) / bm_pos;
+    nblk = (unsigned)nqb * a.B * a.Hkv;
+  }
+  KF_LAUNCH("fwd_mfma", (ksl == 2 ? fwd32_kernel<T, D, 2> : fwd32_kernel<T, D, 1>), dim3(nblk),
+            dim3(256), 0, a.stream, (const T*)a.q, a.cos, a.sin, (const T*)w.krot, (const T*)w.vn,
+            (T*)a.out, a.lse, a.Sq, a.Sk, Skp, w.krows, a.Hq, a.Hkv, n_rep, bm_pos, nqb,
+            a.scale * kLog2e, a.causal, (T*)w.qrot, kpm_keys);
 }
 
 template <typename T, int D>

@@ -1,0 +1,62 @@
+"""The forward's two-slice workgroups (small grids): row blocks and key halves
+at their edges, halves without a visible key, and the last grid that takes them."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from gpu_util import DEV, TOL, announce, check_out, seeded
+from kempnerforge_amd import ops
+from oracle import attention_ref as ref
+
+pytestmark = pytest.mark.gpu
+
+BF16, F16 = torch.bfloat16, torch.float16
+
+
+@pytest.mark.parametrize("cfg", [
+    # dtype, B, S, Hq, Hkv, D, causal
+    (BF16, 1, 1, 4, 2, 128, True),       # second half empty
+    (BF16, 1, 32, 2, 2, 128, True),
+    (BF16, 2, 33, 2, 1, 64, False),      # one key in the second half
+    (F16, 1, 65, 6, 2, 128, True),       # n_rep 3: 63 of 64 rows; a third half tile
+    (BF16, 1, 200, 64, 1, 128, True),    # n_rep 64: one position per block
+    (BF16, 1, 200, 80, 1, 64, True),     # n_rep 80: one slice
+    (F16, 2, 500, 10, 2, 64, False),
+    (BF16, 1, 1024, 32, 8, 128, True),   # 256 blocks (CUs of the chip): two slices
+    (BF16, 1, 1028, 32, 8, 128, True),   # one more: one slice
+], ids=lambda c: "-".join(map(str, (str(c[0])[6:],) + c[1:])))
+def test_shapes(cfg):
+    dtype, B, S, Hq, Hkv, D, causal = cfg
+    announce(f"fwd slices {cfg}")
+    q, k, v = (seeded((B, S, h, D), i, dtype) for i, h in enumerate((Hq, Hkv, Hkv)))
+    cos, sin = ref.rope_tables(D, S, 5e5)
+    args = [t.to(DEV) for t in (q, k, v, cos, sin)]
+    out, lse = ops.fwd_raw(*args, causal=causal, k_rotated=False)
+    o_ref, l_ref = ref.attention_fwd(q, k, v, cos, sin, causal=causal)
+    check_out(out, o_ref, TOL[dtype], "out")
+    check_out(lse, l_ref, 1e-3, "lse")
+    res = ops.fwd_rot_raw(*args, causal=causal)  # the rotated q rows, stored by both slices
+    P = (S + 127) // 128 * 128
+    rot_q = res[2][B * Hkv * P * D:].view(B, Hq, P, D)
+    assert torch.equal(rot_q[:, :, :S].cpu(), ref.apply_rope(q.transpose(1, 2), cos, sin))
+    assert (rot_q[:, :, S:] == 0).all() and torch.equal(res[0], out)
+
+
+def test_infinite_keys_in_one_half():
+    """Scores of -inf over a whole half tile: probability zero there, not NaN,
+    whichever half holds them."""
+    announce("fwd slices -inf scores")
+    B, S, H, D = 1, 64, 1, 64
+    cos, sin = torch.ones(S, D // 2), torch.zeros(S, D // 2)  # no rotation
+    q = torch.zeros(B, S, H, D, dtype=BF16)
+    q[..., 0] = 1.0
+    v = seeded((B, S, H, D), 2, BF16)
+    for half in (0, 1):
+        k = torch.zeros(B, S, H, D, dtype=BF16)
+        k[:, 32 * half:32 * half + 32, :, 0] = -float("inf")
+        out, _ = ops.fwd_raw(*(t.to(DEV) for t in (q, k, v, cos, sin)), causal=False,
+                             k_rotated=True)
+        keep = v[:, 32:] if half == 0 else v[:, :32]
+        check_out(out, keep.float().mean(1, keepdim=True).expand(B, S, H, D), TOL[BF16], "out")
