@@ -46,7 +46,6 @@ namespace {
 using mfma::row_info;
 using mfma::RowInfo;
 using mfma::wave_id;
-using mfma::xcd_logical_id;
 
 constexpr int F_ROWS = 64;  // query rows per workgroup (forward, dQ): 4 wavefronts x 16
 constexpr int F_BN = 32;    // keys per tile (forward, dQ), query positions per tile (dK/dV)
@@ -219,35 +218,43 @@ __device__ __forceinline__ void accum_t2(const float* ta, const f32x4& pa0, cons
 }
 
 // ------------------------------------------------------------------ prepass
-// dst[(b H + h) Sp + s][D] = src[b, s, h, :] after RoPE at table row s (rot)
-// or as is; rows s in [S, Sp) zero.  One thread per chunk pair.
+// dst[(b H + h) Sp + s][D] = src[b, s, h, :] after RoPE at table row s; rows s
+// in [S, Sp) zero.  One thread per chunk pair; blockIdx.y picks the operand
+// (the backward rotates q and k in one launch).
+struct RowsJob {
+  const float* src;
+  int64_t sb, ss, sh;
+  float* dst;
+  int H;
+  int64_t pairs;  // threads
+};
+struct RowsJobs {
+  RowsJob j[2];
+};
 template <int D>
-__global__ __launch_bounds__(256) void rows_f32_kernel(const float* __restrict__ src, int64_t sb,
-                                                       int64_t ss, int64_t sh,
+__global__ __launch_bounds__(256) void rows_f32_kernel(RowsJobs jobs,
                                                        const float* __restrict__ cos,
-                                                       const float* __restrict__ sin,
-                                                       float* __restrict__ dst, int S, int Sp,
-                                                       int H, int rot, int64_t pairs) {
+                                                       const float* __restrict__ sin, int S,
+                                                       int Sp) {
+  const RowsJob& a = jobs.j[blockIdx.y];
   const int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (p >= pairs) return;
+  if (p >= a.pairs) return;
   const int c = (int)(p % (D / 8));
   const int64_t rowi = p / (D / 8);
   const int s = (int)(rowi % Sp);
   const int64_t bh = rowi / Sp;
-  const int h = (int)(bh % H);
-  const int64_t b = bh / H;
+  const int h = (int)(bh % a.H);
+  const int64_t b = bh / a.H;
   f32x4 x1 = zero4(), x2 = zero4();
   if (s < S) {
-    const float* row = src + b * sb + (int64_t)s * ss + (int64_t)h * sh;
+    const float* row = a.src + b * a.sb + (int64_t)s * a.ss + (int64_t)h * a.sh;
     x1 = *(const f32x4*)(row + 4 * c);
     x2 = *(const f32x4*)(row + D / 2 + 4 * c);
-    if (rot) {
-      const int64_t o = (int64_t)s * (D / 2) + 4 * c;
-      rope4(x1, x2, *(const f32x4*)(cos + o), *(const f32x4*)(sin + o));
-    }
+    const int64_t o = (int64_t)s * (D / 2) + 4 * c;
+    rope4(x1, x2, *(const f32x4*)(cos + o), *(const f32x4*)(sin + o));
   }
-  *(f32x4*)(dst + rowi * D + 4 * c) = x1;
-  *(f32x4*)(dst + rowi * D + D / 2 + 4 * c) = x2;
+  *(f32x4*)(a.dst + rowi * D + 4 * c) = x1;
+  *(f32x4*)(a.dst + rowi * D + D / 2 + 4 * c) = x2;
 }
 
 // Per query row (b, h, i), i < Sp: -lse log2(e) and Delta = sum_d dO O, in
@@ -437,7 +444,7 @@ __global__ __launch_bounds__(256, 2) void fwd_f32_kernel(
   __shared__ int sCount;
 
   const int lane = threadIdx.x & 63, g = lane >> 4, c16 = lane & 15, w = wave_id();
-  const int logical = xcd_logical_id(blockIdx.x, gridDim.x, nqb);
+  const int logical = mfma::paired_id(blockIdx.x, gridDim.x, nqb);
   const RowInfo ri = row_info(logical, nqb, Hkv, n_rep, bm_pos, Sq, w * 16 + c16);
   const KeyWalk<MODE> kw =
       key_walk<MODE>(ri, causal ? min(Sk, min(ri.p0 + bm_pos, Sq)) : Sk, Sk, bm_pos, mask,
@@ -545,7 +552,7 @@ __global__ __launch_bounds__(256, 2) void capture_f32_kernel(
   __shared__ int sCount;
 
   const int lane = threadIdx.x & 63, g = lane >> 4, c16 = lane & 15, w = wave_id();
-  const int logical = xcd_logical_id(blockIdx.x, gridDim.x, nqb);
+  const int logical = mfma::paired_id(blockIdx.x, gridDim.x, nqb);
   const RowInfo ri = row_info(logical, nqb, Hkv, n_rep, bm_pos, Sq, w * 16 + c16);
   const KeyWalk<MODE> kw =
       key_walk<MODE>(ri, causal ? min(Sk, min(ri.p0 + bm_pos, Sq)) : Sk, Sk, bm_pos, mask,
@@ -685,7 +692,7 @@ __global__ __launch_bounds__(256, 2) void bwd_dq_f32_kernel(
   __shared__ int sCount;
 
   const int lane = threadIdx.x & 63, g = lane >> 4, c16 = lane & 15, w = wave_id();
-  const int logical = xcd_logical_id(blockIdx.x, gridDim.x, nqb);
+  const int logical = mfma::paired_id(blockIdx.x, gridDim.x, nqb);
   const RowInfo ri = row_info(logical, nqb, Hkv, n_rep, bm_pos, S, w * 16 + c16);
   const KeyWalk<MODE> kw = key_walk<MODE>(ri, causal ? min(S, ri.p0 + bm_pos) : S, S, bm_pos,
                                           mask, ranges, first_valid, nt32, sList, &sCount, w,
@@ -764,7 +771,7 @@ __global__ __launch_bounds__(256, 2) void bwd_dq_rec_f32_kernel(
   __shared__ __attribute__((aligned(16))) float sK[2][F_BN * D];
 
   const int lane = threadIdx.x & 63, g = lane >> 4, c16 = lane & 15, w = wave_id();
-  const int logical = xcd_logical_id(blockIdx.x, gridDim.x, nqb);
+  const int logical = mfma::paired_id(blockIdx.x, gridDim.x, nqb);
   const RowInfo ri = row_info(logical, nqb, Hkv, n_rep, bm_pos, S, w * 16 + c16);
   const int kend = causal ? min(S, ri.p0 + bm_pos) : S;
   const int ntiles = (kend + F_BN - 1) / F_BN;
@@ -808,14 +815,19 @@ __global__ __launch_bounds__(256, 2) void bwd_dq_rec_f32_kernel(
 // (under MASK_DOC only the listed ones; under MASK_KPM also the guarded rows'
 // tiles below it): S = Q·K^T and dP = dO·V^T per 32-position tile, then
 // dV^T += dO^T·P and dK^T += Q^T·dS.  Key blocks are numbered longest first.
-template <int D, int MODE, bool REC = false>
+// PART, for grids that leave the chip idle (dkdv_parts): an item is one query
+// head of the group and one of nseg equal runs of its query tiles; its float32
+// sums go to part[] ([head, run][B Hkv][S][dK D, dV D]), which
+// dkdv_parts_f32_kernel adds in float64.
+template <int D, int MODE, bool REC = false, bool PART = false>
 __global__ __launch_bounds__(256, 2) void bwd_dkdv_f32_kernel(
     const float* qr_rows, const float* __restrict__ kr_rows, const float* __restrict__ v,
     const float* __restrict__ cos, const float* __restrict__ sin, const float* dout,
     const float* stats, double* __restrict__ sum64, float* __restrict__ dk,
     float* __restrict__ dv, int S, int Sp, int Hq, int Hkv, int n_rep, int causal, float scale,
     float scale_log2, const int32_t* __restrict__ mask, const int2* __restrict__ ranges,
-    const int* __restrict__ first_valid, int nt32, float* __restrict__ rec, int64_t rec_nt) {
+    const int* __restrict__ first_valid, int nt32, float* __restrict__ rec, int64_t rec_nt,
+    int nseg, float* __restrict__ part) {
   constexpr int NJ = D / 16, NB = D / 16;
   __shared__ __attribute__((aligned(16))) float sQ[2][F_BN * D];
   __shared__ __attribute__((aligned(16))) float sO[2][F_BN * D];
@@ -825,8 +837,16 @@ __global__ __launch_bounds__(256, 2) void bwd_dkdv_f32_kernel(
   __shared__ int sCount;
 
   const int lane = threadIdx.x & 63, g = lane >> 4, c16 = lane & 15, w = wave_id();
-  const int BH = gridDim.x / ((S + F_BK - 1) / F_BK);
-  const int kblk = blockIdx.x / BH, bh = blockIdx.x % BH;
+  const int nparts = PART ? n_rep * nseg : 1;
+  const int BH = gridDim.x / ((S + F_BK - 1) / F_BK) / nparts;
+  int item = blockIdx.x;
+  // longest first, and on grids that a CU holds whole, its second workgroup
+  // short where its first is long
+  if ((int)gridDim.x <= 32 * mfma::XCD_CUS) {
+    const int x = item % 8;
+    item = 8 * mfma::zigzag_round(item / 8, gridDim.x / 8 + (x < (int)gridDim.x % 8 ? 1 : 0)) + x;
+  }
+  const int kblk = item / (BH * nparts), bh = item % BH, prt = item / BH % nparts;
   const int b = bh / Hkv, hk = bh % Hkv;
   const int k0 = kblk * F_BK;
   const int key = k0 + 16 * w + c16;
@@ -859,10 +879,15 @@ __global__ __launch_bounds__(256, 2) void bwd_dkdv_f32_kernel(
     return MODE == MASK_DOC ? __builtin_amdgcn_readfirstlane((int)sList[u])
                             : MODE == MASK_KPM && u < ng ? u : t0 + u - ng;
   };
-  const int total = per * n_rep;
+  // PART: the tiles [u0, u0 + total) of head h0 only; otherwise all heads' tiles
+  const int h0 = hk * n_rep + (PART ? prt / nseg : 0);
+  const int u0 = PART ? per * (prt % nseg) / nseg : 0;
+  const int total = PART ? per * (prt % nseg + 1) / nseg - u0 : per * n_rep;
+  auto head_of = [&](int it) { return PART ? h0 : h0 + it / per; };
+  auto walk_of = [&](int it) { return PART ? u0 + it : it % per; };
   const int oss = Hq * D;
   auto stage = [&](int it, int buf) {
-    const int hq = hk * n_rep + it / per, q0 = tile_of(it % per) * F_BN;
+    const int hq = head_of(it), q0 = tile_of(walk_of(it)) * F_BN;
     const int64_t hrow = (int64_t)b * Hq + hq;
     tile_dma<D>(qr_rows + (hrow * Sp + q0) * D, (uint32_t)D, sQ[buf], w, lane, F_BN);
     tile_dma<D>(dout + (((int64_t)b * S + q0) * Hq + hq) * D, (uint32_t)oss, sO[buf], w, lane,
@@ -903,9 +928,13 @@ __global__ __launch_bounds__(256, 2) void bwd_dkdv_f32_kernel(
       asm volatile("" : "+v"(same));
     }
     f32x4 s0 = zero4(), s1 = zero4(), d0 = zero4(), d1 = zero4();
-    scores2<D>(tQ, kr, c16, g, s0, s1);
-    scores2<D>(tO, vr, c16, g, d0, d1);
-    const int q0 = tile_of(it % per) * F_BN;
+    // (PART: the fragment addresses formed per tile; hoisted out of its simpler
+    // loop they spill 37 registers at D 128)
+    int cl = c16;
+    if (PART) asm volatile("" : "+v"(cl));
+    scores2<D>(tQ, kr, cl, g, s0, s1);
+    scores2<D>(tO, vr, cl, g, d0, d1);
+    const int q0 = tile_of(walk_of(it)) * F_BN;
     const bool edge = MODE != MASK_NONE || (causal && q0 < k0 + F_BK - 1);
     const int lim = key - q0;  // position offsets below lim are masked (causal)
     const int klim = kkey - q0;  // MASK_KPM: offsets from klim on see this (valid) key
@@ -944,8 +973,8 @@ __global__ __launch_bounds__(256, 2) void bwd_dkdv_f32_kernel(
         d1[r] = s1[r] * (d1[r] - dl1[r]);
       }
     }
-    accum_t2<D>(tO, s0, s1, adv, tQ, d0, d1, adk, c16, g);
-    if (it % per == per - 1 && it + 1 < total) {
+    accum_t2<D>(tO, s0, s1, adv, tQ, d0, d1, adk, cl, g);
+    if (!PART && it % per == per - 1 && it + 1 < total) {
       // a query head done: its sums (unscaled, before the RoPE backward) join
       // the group's in float64, in this lane's own elements of sum64 (per key
       // row, D dK then D dV values), so the group sum adds no float32
@@ -976,15 +1005,29 @@ __global__ __launch_bounds__(256, 2) void bwd_dkdv_f32_kernel(
       // [32 positions][64 keys] for the dQ pass, after the end-of-tile wait
       // (vmcnt counts stores with the staging loads: a store issued inside
       // the tile would hold that wait until it is written)
-      const int t = q0 / F_BN, hq = hk * n_rep + it / per;
+      const int t = q0 / F_BN, hq = head_of(it);
       float* blk = rec + (((int64_t)b * Hq + hq) * rec_nt + rec_off(t, kblk, causal, nkb_of(S))) *
-                             (F_BN * F_BK) + 16 * w + c16;
+                             (F_BN * F_BK);
+      const int off = 4 * g * F_BK + 16 * w + c16;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        __builtin_nontemporal_store(kvalid ? d0[r] : 0.f, blk + (4 * g + r) * F_BK);
-        __builtin_nontemporal_store(kvalid ? d1[r] : 0.f, blk + (16 + 4 * g + r) * F_BK);
+        __builtin_nontemporal_store(kvalid ? d0[r] : 0.f, blk + off + r * F_BK);
+        __builtin_nontemporal_store(kvalid ? d1[r] : 0.f, blk + off + (16 + r) * F_BK);
       }
     }
+  }
+  if (PART) {
+    if (kvalid) {
+      int kl = key;
+      asm volatile("" : "+v"(kl));
+      float* row = part + (((int64_t)prt * BH + bh) * S + kl) * (2 * D) + 4 * g;
+#pragma unroll
+      for (int db = 0; db < NB; ++db) {
+        *(f32x4*)(row + 16 * db) = adk[db];
+        *(f32x4*)(row + D + 16 * db) = adv[db];
+      }
+    }
+    return;
   }
   if (kvalid) {
     int kl = key;
@@ -1003,6 +1046,45 @@ __global__ __launch_bounds__(256, 2) void bwd_dkdv_f32_kernel(
 #pragma unroll
     for (int db = 0; db < NB; ++db) *(f32x4*)(vrow + 16 * db + 4 * g) = adv[db];
   }
+}
+
+// dK and dV of PART items: a key's parts added in float64 in part order (heads
+// ascending, as the unsplit kernel adds them), then the scale, the RoPE
+// backward and the store.  D / 8 threads per key row take four dK dims and
+// their RoPE partners, and the same dims of dV.
+template <int D>
+__global__ __launch_bounds__(256) void dkdv_parts_f32_kernel(
+    const float* __restrict__ part, int nparts, const float* __restrict__ cos,
+    const float* __restrict__ sin, float* __restrict__ dk, float* __restrict__ dv, int S,
+    int Hkv, int64_t rows, float scale) {
+  const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t row = t / (D / 8);  // bh S + key
+  if (row >= rows) return;
+  const int d = 4 * (int)(t % (D / 8));
+  const int key = (int)(row % S);
+  const int64_t bh = row / S;
+  const float* p = part + row * (2 * D) + d;
+  f64x4 s[4] = {};
+#pragma unroll 4
+  for (int i = 0; i < nparts; ++i, p += rows * (2 * D))
+#pragma unroll
+    for (int c = 0; c < 4; ++c) s[c] += to_f64(*(const f32x4*)(p + c * (D / 2)));
+  const int64_t o = ((bh / Hkv * S + key) * Hkv + bh % Hkv) * D + d;
+  const f32x4 cs = *(const f32x4*)(cos + (int64_t)key * (D / 2) + d);
+  const f32x4 sn = *(const f32x4*)(sin + (int64_t)key * (D / 2) + d);
+  const f32x4 k1 = to_f32x4(s[0]), k2 = to_f32x4(s[1]);
+  f32x4 lo, hi;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    float d1, d2;
+    rope_pair_bwd<float>(k1[e] * scale, k2[e] * scale, cs[e], sn[e], d1, d2);
+    lo[e] = d1;
+    hi[e] = d2;
+  }
+  *(f32x4*)(dk + o) = lo;
+  *(f32x4*)(dk + o + D / 2) = hi;
+  *(f32x4*)(dv + o) = to_f32x4(s[2]);
+  *(f32x4*)(dv + o + D / 2) = to_f32x4(s[3]);
 }
 
 // QK-norm of one element: x / rms(row) * w, the row's sum of squares ss
@@ -1230,13 +1312,16 @@ void launch_merge_f32(const DecodeArgs& a, const float* opart, const float* mlpa
 }
 
 template <int D>
-int launch_rows(const float* src, int64_t sb, int64_t ss, int64_t sh, const float* cos,
-                const float* sin, float* dst, int B, int S, int Sp, int H, int rot,
+int launch_rows(RowsJobs& jobs, int n, const float* cos, const float* sin, int B, int S, int Sp,
                 hipStream_t stream) {
-  const int64_t pairs = (int64_t)B * H * Sp * (D / 8);
-  KF_CHECK_ARG((pairs + 255) / 256 < (1LL << 31), "grid too large");
-  KF_LAUNCH("rows_f32", (rows_f32_kernel<D>), dim3((unsigned)((pairs + 255) / 256)), dim3(256),
-            0, stream, src, sb, ss, sh, cos, sin, dst, S, Sp, H, rot, pairs);
+  int64_t most = 0;
+  for (int i = 0; i < n; ++i) {
+    jobs.j[i].pairs = (int64_t)B * jobs.j[i].H * Sp * (D / 8);
+    most = std::max(most, jobs.j[i].pairs);
+  }
+  KF_CHECK_ARG((most + 255) / 256 < (1LL << 31), "grid too large");
+  KF_LAUNCH("rows_f32", (rows_f32_kernel<D>), dim3((unsigned)((most + 255) / 256), n), dim3(256),
+            0, stream, jobs, cos, sin, S, Sp);
   KF_CHECK_LAUNCH();
   return KF_OK;
 }
@@ -1296,8 +1381,8 @@ int fwd_f32_t(const FwdArgs& a, void* workspace) {
   if (!a.k_rotated) {
     const int Skp = (a.Sk + F_BK - 1) / F_BK * F_BK;
     float* krot = (float*)workspace;
-    const int rc = launch_rows<D>((const float*)a.k, a.ksb, a.kss, a.ksh, a.cos, a.sin, krot, a.B,
-                                  a.Sk, Skp, a.Hkv, 1, a.stream);
+    RowsJobs jobs{{{(const float*)a.k, a.ksb, a.kss, a.ksh, krot, a.Hkv, 0}, {}}};
+    const int rc = launch_rows<D>(jobs, 1, a.cos, a.sin, a.B, a.Sk, Skp, a.stream);
     if (rc) return rc;
     kt = krot;
     kb_h = (int64_t)Skp * D;
@@ -1322,43 +1407,79 @@ int fwd_f32_t(const FwdArgs& a, void* workspace) {
   return KF_OK;
 }
 
-// backward workspace: rotated Q, rotated K, row statistics, then (n_rep > 1)
-// the float64 group sums, then the mask records
+// Runs of query tiles per head when the dK/dV items are split (PART), 0 when
+// they are not: with less than four workgroups per CU a KV group's query heads
+// are items of their own, with less than two also runs of a head's tiles, up to
+// two workgroups per CU.  dK/dV kernel, unsplit / split (the parts' sum, 8 to
+// 30 us, not included): D 128, 32/8 heads B = 1 S = 1024 734 / 209 us, S = 2048
+// 1475 / 719, S = 4096 (512 items) 2966 / 2578; D 64, 4/2 heads, B = 2 S = 256 62 /
+// 13; 16 heads of 96 without groups, B = 2 S = 1024 (512 items) 160 / 152 with two
+// runs, and 15 for their sum: not split.
+int dkdv_parts(int B, int S, int Hq, int Hkv) {
+  const int64_t items = (int64_t)((S + F_BK - 1) / F_BK) * B * Hkv;
+  const int64_t cus = device_cu_count();
+  const int n_rep = Hq / Hkv, nt = (S + F_BN - 1) / F_BN;
+  if (items >= 4 * cus) return 0;
+  if (items >= 2 * cus) return n_rep > 1 ? 1 : 0;
+  const int64_t heads = items * n_rep;
+  const int nseg = (int)std::min<int64_t>({(2 * cus + heads - 1) / heads, 8, nt});
+  return n_rep * nseg == 1 ? 0 : nseg;
+}
+
+// backward workspace: rotated Q, rotated K, row statistics, then the split
+// items' parts or (n_rep > 1) the float64 group sums, then the mask records
 size_t bwd_base_bytes(int B, int S, int Hq, int Hkv, int D, size_t* sum_off) {
   const size_t Sp = (size_t)(S + F_BK - 1) / F_BK * F_BK;
   const size_t f = ((size_t)B * Hq * Sp * D + (size_t)B * Hkv * Sp * D + (size_t)B * Hq * Sp * 2) *
                    sizeof(float);
   *sum_off = al256(f);
-  return *sum_off + (Hq > Hkv ? (size_t)B * S * Hkv * D * 2 * sizeof(double) : 0);
+  const size_t kv = (size_t)B * S * Hkv * D * 2;
+  const int nseg = dkdv_parts(B, S, Hq, Hkv);
+  return *sum_off + (nseg > 0     ? kv * (Hq / Hkv) * nseg * sizeof(float)
+                     : Hq > Hkv ? kv * sizeof(double)
+                                : 0);
+}
+
+template <int D, int MODE, bool REC>
+void launch_dkdv(const BwdArgs& a, const F32BwdWs& w, int n_rep, unsigned nkblk,
+                 const MaskRec& mr, float* rec, int64_t rnt) {
+  const int nseg = dkdv_parts(a.B, a.S, a.Hq, a.Hkv), nparts = nseg > 0 ? n_rep * nseg : 1;
+  float* part = (float*)w.sum64;
+  KF_LAUNCH("bwd_dkdv_f32",
+            (nseg > 0 ? bwd_dkdv_f32_kernel<D, MODE, REC, true>
+                      : bwd_dkdv_f32_kernel<D, MODE, REC, false>),
+            dim3(nkblk * nparts), dim3(256), 0, a.stream, w.qrot, w.krot, (const float*)a.v,
+            a.cos, a.sin, (const float*)a.dout, w.stats, w.sum64, (float*)a.dk, (float*)a.dv,
+            a.S, w.Sp, a.Hq, a.Hkv, n_rep, a.causal, a.scale, a.scale * kLog2e,
+            a.doc ? a.doc : a.kvalid, mr.ranges, mr.first_valid, mr.nt32, rec, rnt, nseg, part);
+  if (nseg > 0) {
+    const int64_t rows = (int64_t)a.B * a.Hkv * a.S;
+    KF_LAUNCH("dkdv_parts_f32", (dkdv_parts_f32_kernel<D>),
+              dim3((unsigned)((rows * (D / 8) + 255) / 256)), dim3(256), 0, a.stream, part, nparts,
+              a.cos, a.sin, (float*)a.dk, (float*)a.dv, a.S, a.Hkv, rows, a.scale);
+  }
 }
 
 template <int D, int MODE>
-void launch_bwd_kernels(const BwdArgs& a, float* qrot, float* krot, float* stats, double* sum64,
-                        int Sp, int n_rep, int bm_pos, int nqb, unsigned nqblk, unsigned nkblk,
-                        const MaskRec& mr, float* rec) {
+void launch_bwd_kernels(const BwdArgs& a, const F32BwdWs& w, int n_rep, int bm_pos, int nqb,
+                        unsigned nqblk, unsigned nkblk, const MaskRec& mr, float* rec) {
   const int32_t* mask = a.doc ? a.doc : a.kvalid;
   if constexpr (MODE == MASK_NONE) {
-   if (rec != nullptr) {
-    // dK/dV first, keeping dS; then dQ from the records
-    const int64_t rnt = rec_blocks(a.S, a.causal);
-    KF_LAUNCH("bwd_dkdv_f32", (bwd_dkdv_f32_kernel<D, MODE, true>), dim3(nkblk), dim3(256), 0,
-              a.stream, qrot, krot, (const float*)a.v, a.cos, a.sin, (const float*)a.dout,
-              stats, sum64, (float*)a.dk, (float*)a.dv, a.S, Sp, a.Hq, a.Hkv, n_rep, a.causal,
-              a.scale, a.scale * kLog2e, mask, mr.ranges, mr.first_valid, mr.nt32, rec, rnt);
-    KF_LAUNCH("bwd_dq_rec_f32", (bwd_dq_rec_f32_kernel<D>), dim3(nqblk), dim3(256), 0, a.stream,
-              krot, rec, a.cos, a.sin, (float*)a.dq, a.S, Sp, a.Hq, a.Hkv, n_rep, bm_pos, nqb,
-              a.causal, a.scale, rnt);
-    return;
-   }
+    if (rec != nullptr) {
+      // dK/dV first, keeping dS; then dQ from the records
+      const int64_t rnt = rec_blocks(a.S, a.causal);
+      launch_dkdv<D, MODE, true>(a, w, n_rep, nkblk, mr, rec, rnt);
+      KF_LAUNCH("bwd_dq_rec_f32", (bwd_dq_rec_f32_kernel<D>), dim3(nqblk), dim3(256), 0, a.stream,
+                w.krot, rec, a.cos, a.sin, (float*)a.dq, a.S, w.Sp, a.Hq, a.Hkv, n_rep, bm_pos,
+                nqb, a.causal, a.scale, rnt);
+      return;
+    }
   }
   KF_LAUNCH("bwd_dq_f32", (bwd_dq_f32_kernel<D, MODE>), dim3(nqblk), dim3(256), 0, a.stream,
-            qrot, krot, (const float*)a.v, a.cos, a.sin, (const float*)a.dout, stats,
-            (float*)a.dq, a.S, Sp, a.Hq, a.Hkv, n_rep, bm_pos, nqb, a.causal, a.scale,
+            w.qrot, w.krot, (const float*)a.v, a.cos, a.sin, (const float*)a.dout, w.stats,
+            (float*)a.dq, a.S, w.Sp, a.Hq, a.Hkv, n_rep, bm_pos, nqb, a.causal, a.scale,
             a.scale * kLog2e, mask, mr.ranges, mr.first_valid, mr.nt32);
-  KF_LAUNCH("bwd_dkdv_f32", (bwd_dkdv_f32_kernel<D, MODE>), dim3(nkblk), dim3(256), 0, a.stream,
-            qrot, krot, (const float*)a.v, a.cos, a.sin, (const float*)a.dout, stats, sum64,
-            (float*)a.dk, (float*)a.dv, a.S, Sp, a.Hq, a.Hkv, n_rep, a.causal, a.scale,
-            a.scale * kLog2e, mask, mr.ranges, mr.first_valid, mr.nt32, nullptr, 0);
+  launch_dkdv<D, MODE, false>(a, w, n_rep, nkblk, mr, nullptr, 0);
 }
 
 // bytes of the dS records, or 0 past the cap (dQ then recomputes S and dP)
@@ -1383,14 +1504,11 @@ int bwd_f32_t(const BwdArgs& a, const F32BwdWs& w, float* rec) {
     if (rc) return rc;
   }
   if (mode == MASK_DOC)
-    launch_bwd_kernels<D, MASK_DOC>(a, w.qrot, w.krot, w.stats, w.sum64, w.Sp, n_rep, bm_pos, nqb,
-                                    (unsigned)nqblk, (unsigned)nkblk, mr, rec);
+    launch_bwd_kernels<D, MASK_DOC>(a, w, n_rep, bm_pos, nqb, (unsigned)nqblk, (unsigned)nkblk, mr, rec);
   else if (mode == MASK_KPM)
-    launch_bwd_kernels<D, MASK_KPM>(a, w.qrot, w.krot, w.stats, w.sum64, w.Sp, n_rep, bm_pos, nqb,
-                                    (unsigned)nqblk, (unsigned)nkblk, mr, rec);
+    launch_bwd_kernels<D, MASK_KPM>(a, w, n_rep, bm_pos, nqb, (unsigned)nqblk, (unsigned)nkblk, mr, rec);
   else
-    launch_bwd_kernels<D, MASK_NONE>(a, w.qrot, w.krot, w.stats, w.sum64, w.Sp, n_rep, bm_pos,
-                                     nqb, (unsigned)nqblk, (unsigned)nkblk, mr, rec);
+    launch_bwd_kernels<D, MASK_NONE>(a, w, n_rep, bm_pos, nqb, (unsigned)nqblk, (unsigned)nkblk, mr, rec);
   KF_CHECK_LAUNCH();
   return KF_OK;
 }
@@ -1398,11 +1516,9 @@ int bwd_f32_t(const BwdArgs& a, const F32BwdWs& w, float* rec) {
 template <int D>
 int bwd_rows_t(const BwdArgs& a, const F32BwdWs& w) {
   const int64_t qss = (int64_t)a.Hq * D, kss = (int64_t)a.Hkv * D;
-  const int rc = launch_rows<D>((const float*)a.q, a.S * qss, qss, D, a.cos, a.sin, w.qrot, a.B,
-                                a.S, w.Sp, a.Hq, 1, a.stream);
-  if (rc) return rc;
-  return launch_rows<D>((const float*)a.k, a.S * kss, kss, D, a.cos, a.sin, w.krot, a.B, a.S,
-                        w.Sp, a.Hkv, 1, a.stream);
+  RowsJobs jobs{{{(const float*)a.q, a.S * qss, qss, D, w.qrot, a.Hq, 0},
+                 {(const float*)a.k, a.S * kss, kss, D, w.krot, a.Hkv, 0}}};
+  return launch_rows<D>(jobs, 2, a.cos, a.sin, a.B, a.S, w.Sp, a.stream);
 }
 
 bool al16(const void* p) { return ((uintptr_t)p & 15) == 0; }

@@ -81,7 +81,7 @@ int bwd_f32(const BwdArgs& a, void* workspace, size_t workspace_bytes);
 struct F32BwdWs {
   float *qrot, *krot;  // [B*Hq][Sp][D], [B*Hkv][Sp][D] after RoPE, rows past S zero
   float* stats;
-  double* sum64;
+  double* sum64;       // the group sums, or the split items' float32 parts
   void* masks;
   int Sp;              // S rounded up to 64
 };

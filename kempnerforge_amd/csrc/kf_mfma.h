@@ -83,6 +83,24 @@ __host__ __device__ __forceinline__ int dealt_order(int c, int n, int L) {
   return (i % ng) * L + i / ng;
 }
 
+// Block id to item for one-item-per-workgroup grids of n causal blocks (n / L
+// groups of L, item group * L + rank, rank 0 the longest).  When a CU holds all
+// its workgroups at once (up to four per CU), the launch lasts as long as the
+// busiest CU: XCD x then takes the items of dealt_order's share x, longest
+// first, and every second round of one workgroup per CU runs through its items
+// backwards, so that a CU's second workgroup is short where its first is long.
+// Larger grids keep xcd_logical_id's order (the dispatcher balances them).
+constexpr int XCD_CUS = 32;
+__device__ __forceinline__ int zigzag_round(int j, int cnt) {
+  const int r = j / XCD_CUS, m = min(XCD_CUS, cnt - r * XCD_CUS);
+  return (r & 1) ? r * XCD_CUS + m - 1 - j % XCD_CUS : j;
+}
+__device__ __forceinline__ int paired_id(int id, int n, int L) {
+  if (n > 32 * XCD_CUS) return xcd_logical_id(id, n, L);
+  const int per = n / 8, rem = n % 8, x = id % 8;
+  return dealt_order(x * per + min(x, rem) + zigzag_round(id / 8, per + (x < rem ? 1 : 0)), n, L);
+}
+
 struct RowInfo {
   int b, g, hq, pos, p0;
   bool q_valid;
