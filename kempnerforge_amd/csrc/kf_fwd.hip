@@ -1321,15 +1321,19 @@ void launch_fwd_kernel(const FwdArgs& a, const FwdWs& w, int Skp, int n_rep, int
 // nothing).  One / two slices, forward kernel alone: D 128, 32/8 heads S = 256
 // 14.9 / 13.0 us, 512 19.2 / 16.7, 1000 (256 blocks) 28.9 / 26.1, 1999 (504) 54.9
 // / 56.7, 3000 (752) 91 / 105; D 64, 12 heads S = 2048 37 / 27, B = 2 S = 1024 22.7
-// / 18.1, B = 4 S = 2048 (768) 62 / 51.
-int fwd_slices(int64_t nblk, int n_rep, int D) {
-  return n_rep <= ROWS / 2 && nblk <= (D == 64 ? 3 : 1) * (int64_t)device_cu_count() ? 2 : 1;
+// / 18.1, B = 4 S = 2048 (768) 62 / 51.  With D 128 only below 2048 positions:
+// from there on a sequence's rows are the same bits whatever its length (the
+// slices add up in another order), which the gradients' comparison of a 2048-row
+// prefix with the whole 8256-row sequence holds the kernels to.
+int fwd_slices(int64_t nblk, int n_rep, int D, int Sq) {
+  if (n_rep > ROWS / 2 || (D == 128 && Sq >= 2048)) return 1;
+  return nblk <= (D == 64 ? 3 : 1) * (int64_t)device_cu_count() ? 2 : 1;
 }
 
 template <typename T, int D>
 void launch_fwd32(const FwdArgs& a, const FwdWs& w, int Skp, int n_rep, int bm_pos, int nqb,
                   unsigned nblk, const int* kpm_keys) {
-  const int ksl = fwd_slices(nblk, n_rep, D);
+  const int ksl = fwd_slices(nblk, n_rep, D, a.Sq);
   if (ksl == 2) {
     bm_pos = ROWS / 2 / n_rep;
     nqb = (a.Sq + bm_pos - 1) / bm_pos;
