@@ -938,35 +938,53 @@ __device__ __forceinline__ void dma16_nt(uint32_t lds, uint32_t voff, const void
 // tiles listed for the query tile, two record columns per 64-key tile; with key
 // padding (KPM) the causal tiles holding a valid key, in batch rows whose key 0
 // is valid (the others are left to the recompute kernel).
-template <typename T, int D, int HB, int MODE, int NBUF>
-__global__ __launch_bounds__(64 * HB) void bwd_dq_ds_kernel(
+// QT > 1 (unmasked): QT adjacent query tiles of each head, so that KV groups of
+// one or two query heads (or an odd number) share each staged K step among more
+// wavefronts.  A wavefront whose tile has fewer columns, or does not exist,
+// loads a record again (the load counts stay equal across wavefronts) and
+// skips the products.
+// KSP > 1 (unmasked): a step takes KSP record columns, one per slice of HB * QT
+// wavefronts, and the slices' float32 sums meet in LDS at the end.  A grid that
+// leaves the chip idle lasts as long as its longest tile's chain of steps (0.5
+// to 0.9 us each), which this divides by KSP.  dq_split() chooses both.
+template <typename T, int D, int HB, int QT, int KSP, int MODE, int NBUF>
+__global__ __launch_bounds__(64 * HB * QT * KSP) void bwd_dq_ds_kernel(
     const u32x4* __restrict__ dsb, const T* __restrict__ krot, const float* __restrict__ cos,
     const float* __restrict__ sin, T* __restrict__ dq, int S, int P, int Hq, int Hkv,
     int n_rep, int nqt, int causal, float scale, const int32_t* __restrict__ doc,
     const int2* __restrict__ ranges) {
   constexpr bool DOC = MODE == MASK_DOC, KPM = MODE == MASK_KPM, LIST = DOC || KPM;
-  constexpr int NW = HB, KR = D / 8, DT = D / 32, HALF = D / 2;
+  constexpr int NW = HB * QT, KR = D / 8, DT = D / 32, HALF = D / 2;
   static_assert(NBUF == 3 || NBUF == 4, "ring depth");
+  static_assert((QT == 1 && KSP == 1) || !LIST, "tile lists are per query tile");
   constexpr int KI = DSK * KR / 64;  // 1 KB load instructions per K step
   static_assert(KI % NW == 0, "K rows must split evenly over the wavefronts");
   // load instructions per wavefront and step: its share of K, its record's 4 KB
   constexpr int NLOAD = KI / NW + 4;
   struct Stage {
-    T k[DSK * D];
-    u32x4 ds[HB * 256];
+    T k[KSP][DSK * D];
+    u32x4 ds[KSP][NW * 256];
   };
   __shared__ __attribute__((aligned(16))) Stage st[NBUF];
-  const int w = wave_id(), lane = threadIdx.x & 63, hh = lane >> 5, c32 = lane & 31;
+  const int wv = wave_id(), lane = threadIdx.x & 63, hh = lane >> 5, c32 = lane & 31;
+  // place in its slice, slice (scalars: the record's base address needs SGPRs)
+  const int w = KSP == 1 ? wv : __builtin_amdgcn_readfirstlane(wv % NW);
+  const int ks = KSP == 1 ? 0 : __builtin_amdgcn_readfirstlane(wv / NW);
   // item (KV head, head group, query tile), a KV head's tiles numbered
   // longest-causal-row first, dealt to the XCDs by xcd_logical_id
   const int ngrp = n_rep / HB;
-  const int logical = xcd_logical_id(blockIdx.x, gridDim.x, nqt);
-  const int qt = nqt - 1 - logical % nqt;
-  const int hg = (logical / nqt) % ngrp, hidx = logical / nqt / ngrp;
-  const int bh = KPM ? kpm_head(hidx, gridDim.x / (nqt * ngrp) / Hkv, Hkv) : hidx;
+  const int nqg = (nqt + QT - 1) / QT;  // tile groups
+  const int logical = xcd_logical_id(blockIdx.x, gridDim.x, nqg);
+  const int qt0 = QT * (nqg - 1 - logical % nqg), qt_last = min(qt0 + QT, nqt) - 1;
+  // this wavefront's tile
+  const int qt = QT == 1 ? qt0 : __builtin_amdgcn_readfirstlane(min(qt0 + w / HB, nqt - 1));
+  const bool live = QT == 1 || qt0 + w / HB < nqt;
+  const int wh = QT == 1 ? w : __builtin_amdgcn_readfirstlane(w % HB);  // its head of the group
+  const int hg = (logical / nqg) % ngrp, hidx = logical / nqg / ngrp;
+  const int bh = KPM ? kpm_head(hidx, gridDim.x / (nqg * ngrp) / Hkv, Hkv) : hidx;
   const int b = bh / Hkv, g = bh % Hkv;
   const int nqtp = P / DSQ;
-  int nk = causal ? min(2 * qt + 2, (S + DSK - 1) / DSK) : (S + DSK - 1) / DSK;
+  int nk = causal ? min(2 * qt_last + 2, (S + DSK - 1) / DSK) : (S + DSK - 1) / DSK;
   // DOC: the 64-key tiles whose document range meets this tile's rows (the
   // dK/dV pass listed this query tile for their key blocks, so their records
   // exist); each listed tile is two steps.  Causal: tiles 0 .. qt.
@@ -977,7 +995,7 @@ __global__ __launch_bounds__(64 * HB) void bwd_dq_ds_kernel(
   if constexpr (KPM) {
     const int2* rec = ranges + (int64_t)b * (P / BN);
     if (__builtin_amdgcn_readfirstlane(rec[0].y) != 0) return;  // guarded rows: dq's
-    if (w == 0) {
+    if (wv == 0) {
       const int n = kpm_tile_list(rec, 0, qt + 1, [](int, int2 r) { return r.x > 0 ? 1 : 0; },
                                   sList, lane);
       if (lane == 0) sCount = n;
@@ -986,7 +1004,7 @@ __global__ __launch_bounds__(64 * HB) void bwd_dq_ds_kernel(
     nk = 2 * __builtin_amdgcn_readfirstlane(sCount);
   }
   if constexpr (DOC) {
-    if (w == 0) {
+    if (wv == 0) {
       const int n = doc_tile_list(doc + (int64_t)b * S, qt * DSQ, min(qt * DSQ + DSQ, S),
                                   ranges + (int64_t)b * (P / BN), 0, qt + 1, sList, lane);
       if (lane == 0) sCount = n;
@@ -999,17 +1017,21 @@ __global__ __launch_bounds__(64 * HB) void bwd_dq_ds_kernel(
     return LIST ? 2 * (__builtin_amdgcn_readfirstlane((int)sList[t >> 1]) & ~DOC_MASK_FLAG) + (t & 1)
                 : t;
   };
-  const u32x4* rec0 = dsb + (ds_pair(bh, qt, 0, nqtp, causal) * n_rep + hg * HB) * 256;
+  // columns of this wavefront's tile
+  const int nk_w = QT == 1 ? nk : !live ? 0 : causal ? min(2 * qt + 2, nk) : nk;
+  const u32x4* rec0 = dsb + (ds_pair(bh, qt, 0, nqtp, causal) * n_rep + hg * HB + wh) * 256;
   const T* kbase = krot + (int64_t)bh * P * D;
+  const int nst = (nk + KSP - 1) / KSP;  // steps
   auto stage = [&](int t_, int buf) {
-    const int t = col(t_);
+    // (a slice past the last column loads it again, and skips the products)
+    const int t = col(KSP == 1 ? t_ : min(KSP * t_ + ks, nk - 1));
 #pragma unroll
     for (int jj = 0; jj < KI / NW; ++jj) {
       const int j = w * (KI / NW) + jj;
       const int L = j * 64 + lane, row = L / KR, pc = L % KR;
       const uint32_t off =
           ((uint32_t)(t * DSK + row) * D + (uint32_t)(pc ^ swz<KR>(row)) * 8u) * 2u;
-      dma16(lds_addr(st[buf].k + j * 512), off, kbase);
+      dma16(lds_addr(st[buf].k[ks] + j * 512), off, kbase);
     }
     // this wavefront's record (read once: streaming loads), 4 x 1 KB of 64
     // 16-byte B-operand pieces; lane i of LDS copy j takes piece
@@ -1017,10 +1039,12 @@ __global__ __launch_bounds__(64 * HB) void bwd_dq_ds_kernel(
     // groups of a transposed read's pass that share a copy in different halves
     // of a 256-byte bank window, the 8 (j & 1) term (128 bytes) does the same
     // for the two groups that read copies j and j + 1
-    const u32x4* src = rec0 + ((int64_t)t * n_rep + w) * 256;
+    const int tr =
+        QT == 1 ? t : __builtin_amdgcn_readfirstlane(min(t, max(nk_w, 1) - 1));
+    const u32x4* src = rec0 + (int64_t)tr * n_rep * 256;
 #pragma unroll
     for (int j = 0; j < 4; ++j)
-      dma16_nt(lds_addr(st[buf].ds + w * 256 + j * 64),
+      dma16_nt(lds_addr(st[buf].ds[ks] + w * 256 + j * 64),
                (uint32_t)((j * 64 + ((lane ^ (8 * (j & 1))) ^ ((lane >> 5) << 2))) * 16), src);
   };
 
@@ -1045,10 +1069,10 @@ __global__ __launch_bounds__(64 * HB) void bwd_dq_ds_kernel(
 
 #pragma unroll
   for (int t = 0; t < NBUF - 1; ++t)
-    if (t < nk) stage(t, t);
-  for (int t = 0; t < nk; ++t) {
+    if (t < nst) stage(t, t);
+  for (int t = 0; t < nst; ++t) {
     // step t's loads are in; those of up to NBUF - 2 later steps may still fly
-    const int ahead = min(NBUF - 2, nk - 1 - t);
+    const int ahead = min(NBUF - 2, nst - 1 - t);
     if (ahead >= 2)
       vm_wait<2 * NLOAD>();
     else if (ahead == 1)
@@ -1056,10 +1080,11 @@ __global__ __launch_bounds__(64 * HB) void bwd_dq_ds_kernel(
     else
       vm_wait<0>();
     __syncthreads();  // every wavefront's share landed; step t - 1's buffer is free
-    if (t + NBUF - 1 < nk) stage(t + NBUF - 1, (t + NBUF - 1) % NBUF);
+    if (t + NBUF - 1 < nst) stage(t + NBUF - 1, (t + NBUF - 1) % NBUF);
+    if ((QT > 1 || KSP > 1) && KSP * t + ks >= nk_w) continue;
     const Stage& S_ = st[t % NBUF];
-    const char* dsl = (const char*)S_.ds + ds_off;
-    const char* dsh = (const char*)S_.ds + (ds_off ^ 128u);
+    const char* dsl = (const char*)S_.ds[ks] + ds_off;
+    const char* dsh = (const char*)S_.ds[ks] + (ds_off ^ 128u);
 #pragma unroll
     for (int c = 0; c < DSK / 16; ++c) {
       bf16x8 bds[2];
@@ -1073,7 +1098,7 @@ __global__ __launch_bounds__(64 * HB) void bwd_dq_ds_kernel(
       }
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) {
-        const bf16x8 ak = lds_frag_t<D>(S_.k, tro, c, dt);
+        const bf16x8 ak = lds_frag_t<D>(S_.k[ks], tro, c, dt);
 #pragma unroll
         for (int mh = 0; mh < 2; ++mh)
           acc[mh][dt] =
@@ -1082,16 +1107,46 @@ __global__ __launch_bounds__(64 * HB) void bwd_dq_ds_kernel(
     }
   }
 
-  const int hq = g * n_rep + hg * HB + w;
+  if constexpr (KSP > 1) {
+    // the slices' sums meet in LDS (the ring is free after the barrier): the
+    // upper half of the slices hands its sums to the lower half, until slice 0
+    // holds the tile's
+    constexpr int SLAB = 2 * DT * 4 * 64;  // f32x4 per wavefront
+    static_assert(KSP / 2 * NW * SLAB * 16 <= NBUF * (int)sizeof(Stage), "slabs exceed the ring");
+#pragma unroll
+    for (int half = KSP / 2; half >= 1; half /= 2) {
+      f32x4* slab = (f32x4*)st + ((ks & (half - 1)) * NW + w) * SLAB + lane;
+      __syncthreads();
+      if (ks >= half && ks < 2 * half) {
+#pragma unroll
+        for (int i = 0; i < 2 * DT * 4; ++i) {
+          const f32x16& x = acc[i / (4 * DT)][i / 4 % DT];
+          slab[i * 64] = f32x4{x[4 * (i % 4)], x[4 * (i % 4) + 1], x[4 * (i % 4) + 2],
+                               x[4 * (i % 4) + 3]};
+        }
+      }
+      __syncthreads();
+      if (ks < half) {
+#pragma unroll
+        for (int i = 0; i < 2 * DT * 4; ++i) {
+          const f32x4 y = slab[i * 64];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[i / (4 * DT)][i / 4 % DT][4 * (i % 4) + e] += y[e];
+        }
+      }
+    }
+  }
+  const int hq = g * n_rep + hg * HB + wh;
   // dQ leaves through LDS (the ring is free once every wavefront is past its
   // last products): each wavefront writes its 64 rows into its own 64 x D
   // slice, 16-byte chunks XOR-swizzled by row, then stores whole chunks, KR
   // consecutive lanes per row, instead of 8 bytes of each of 32 rows.
-  static_assert(HB * 64 * D * 2 <= NBUF * (int)sizeof(Stage), "dQ slices exceed the ring");
+  static_assert(NW * 64 * D * 2 <= NBUF * (int)sizeof(Stage), "dQ slices exceed the ring");
   __syncthreads();
   T* slice = (T*)st + w * 64 * D;
 #pragma unroll
   for (int mh = 0; mh < 2; ++mh) {
+    if (KSP > 1 && ks != 0) break;
     const int r = 32 * mh + c32;
     const int pos = min(qt * DSQ + r, S - 1);  // rows past S are formed, not stored
     const float* cr = cos + (int64_t)pos * HALF;
@@ -1115,9 +1170,10 @@ __global__ __launch_bounds__(64 * HB) void bwd_dq_ds_kernel(
       }
   }
   __syncthreads();
+  if (!live) return;
 #pragma unroll
-  for (int i2 = 0; i2 < KR; ++i2) {
-    const int L = 64 * i2 + lane, r = L / KR, ch = L % KR;
+  for (int i2 = 0; i2 < KR / KSP; ++i2) {  // (the slices store a share of the rows each)
+    const int L = 64 * (ks * (KR / KSP) + i2) + lane, r = L / KR, ch = L % KR;
     const int pos = qt * DSQ + r;
     const u32x4 v = *(const u32x4*)(slice + (r * KR + (ch ^ (r & (KR - 1)))) * 8);
     if (pos < S) *(u32x4*)(dq + (((int64_t)b * S + pos) * Hq + hq) * D + 8 * ch) = v;
@@ -1456,6 +1512,38 @@ Ws carve(void* base, int B, int S, int Hq, int Hkv, int D, const void* rot) {
   return w;
 }
 
+// Query tiles and key slices of an unmasked bwd_dq_ds workgroup, by measurement
+// (us with one tile and slice -> with this rule, bf16; Hq/Hkv, batch, S):
+//  - one head per workgroup (n_rep odd): both two, while all workgroups are
+//    resident at once (10/2 B1 S1024 25.3 -> 19.1; 16/16 D64 B1 S2048 30.5 ->
+//    23.8) and for long sequences at two or more per CU (10/2 B2 S4096 118 ->
+//    106, 12/12 D64 B8 S2048 115 -> 103).  Between, half of the CUs would run
+//    one workgroup more than the others (12/12 D64 B2 S2048 34.8 against 38.5),
+//    and batches of short sequences have tiles enough (10/2 B12 S700 35.2
+//    against 38.2).  Up to three tiles the merge costs what the slices save
+//    (12/12 D64 B1 S65 6.6 against 7.5).
+//  - two heads: two slices up to one workgroup per CU (4/2 D64 B3 S1600 23.8 ->
+//    18.6), two tiles as well on larger grids of long sequences (12/2 B2 S4096
+//    134 -> 110, 16/8 B4 S3000 151 -> 141; 12/2 B4 S3000, whose third round is
+//    a quarter full, 113 -> 118).  Sequences below 1024 or, on larger grids,
+//    2048 keep one tile (16/8 B8 S500 21.1 against 25.9 and 23.6, 12/2 B6 S1100
+//    38.9 against 43.4).
+//  - four heads: one tile; either split came out equal or slower (32/8 B4 S1024
+//    50.7 against 53.6 with two slices).
+struct DqSplit { int qt, ksp; };
+DqSplit dq_split(int hb, int64_t ntile, int nqt) {
+  const int64_t cus = device_cu_count();
+  if (hb == 1 && nqt >= 4) {
+    const int64_t nwg = ntile / nqt * ((nqt + 1) / 2);
+    if (nwg <= cus || (nwg >= 2 * cus && nqt >= 24)) return {2, 2};
+  }
+  if (hb == 2 && nqt >= 16) {
+    if (ntile <= cus) return {1, 2};
+    if (nqt >= 32) return {2, 2};
+  }
+  return {1, 1};
+}
+
 template <typename T, int D, int HB>
 int launch_dq_ds(const BwdArgs& a, const Ws& w) {
   const int P = pad_len(a.S), n_rep = a.Hq / a.Hkv, nqt = (a.S + DSQ - 1) / DSQ;
@@ -1474,14 +1562,23 @@ int launch_dq_ds(const BwdArgs& a, const Ws& w) {
     KF_CHECK_LAUNCH();
     return KF_OK;
   }
-  KF_LAUNCH("bwd_dq_ds",
-            (a.doc      ? (deep ? bwd_dq_ds_kernel<T, D, HB, MASK_DOC, 4>
-                                : bwd_dq_ds_kernel<T, D, HB, MASK_DOC, 3>)
-             : a.kvalid ? (deep ? bwd_dq_ds_kernel<T, D, HB, MASK_KPM, 4>
-                                : bwd_dq_ds_kernel<T, D, HB, MASK_KPM, 3>)
-                        : (deep ? bwd_dq_ds_kernel<T, D, HB, MASK_NONE, 4>
-                                : bwd_dq_ds_kernel<T, D, HB, MASK_NONE, 3>)),
-            dim3(a.B * a.Hkv * (n_rep / HB) * nqt), dim3(64 * HB), 0, a.stream, w.dsb,
+  const bool mask = a.doc || a.kvalid;
+  const int ntile = a.B * a.Hkv * (n_rep / HB) * nqt;
+  const DqSplit sp = mask ? DqSplit{1, 1} : dq_split(HB, ntile, nqt);
+  const int nwg = ntile / nqt * ((nqt + sp.qt - 1) / sp.qt);
+  auto kernel = a.doc      ? (deep ? bwd_dq_ds_kernel<T, D, HB, 1, 1, MASK_DOC, 4>
+                                   : bwd_dq_ds_kernel<T, D, HB, 1, 1, MASK_DOC, 3>)
+                : a.kvalid ? (deep ? bwd_dq_ds_kernel<T, D, HB, 1, 1, MASK_KPM, 4>
+                                   : bwd_dq_ds_kernel<T, D, HB, 1, 1, MASK_KPM, 3>)
+                           : (deep ? bwd_dq_ds_kernel<T, D, HB, 1, 1, MASK_NONE, 4>
+                                   : bwd_dq_ds_kernel<T, D, HB, 1, 1, MASK_NONE, 3>);
+  if constexpr (HB <= 2) {
+    if (sp.qt == 2) kernel = bwd_dq_ds_kernel<T, D, HB, 2, 2, MASK_NONE, 3>;
+  }
+  if constexpr (HB == 2) {
+    if (sp.qt == 1 && sp.ksp == 2) kernel = bwd_dq_ds_kernel<T, D, HB, 1, 2, MASK_NONE, 3>;
+  }
+  KF_LAUNCH("bwd_dq_ds", kernel, dim3(nwg), dim3(64 * HB * sp.qt * sp.ksp), 0, a.stream, w.dsb,
             (const T*)w.krot, a.cos, a.sin, (T*)a.dq, a.S, P, a.Hq, a.Hkv, n_rep, nqt, a.causal,
             a.scale, a.doc, w.ranges);
   KF_CHECK_LAUNCH();
