@@ -613,6 +613,8 @@ class _Attention(torch.autograd.Function):
     def backward(ctx, dout):
         if dout is None:
             return (None,) * 8
+        if not _plain_eager(dout):  # batched gradients, modes around the backward alone
+            return _backward(ctx, dout, None, None)[:8]
         if ctx.use_rot:
             rot, v, cos, sin, out, lse, doc_ids, key_padding_mask = ctx.saved_tensors
             grads = bwd_rot_raw(rot, v, cos, sin, out, lse, dout, causal=ctx.causal,
@@ -638,7 +640,9 @@ def _plain_eager(*ts) -> bool:
             or torch._C._functorch.peek_interpreter_stack() is not None
             or torch.autograd.forward_ad._current_level >= 0):
         return False
-    return all(t is None or (type(t) in _PLAIN and t.is_cuda) for t in ts)
+    # (autograd.grad's is_grads_batched wraps tensors without an interpreter level)
+    return all(t is None or (type(t) in _PLAIN and t.is_cuda
+                             and not torch._C._functorch.is_legacy_batchedtensor(t)) for t in ts)
 
 
 def attention(q, k, v, rope_cos, rope_sin, *, causal: bool = True, doc_ids=None,

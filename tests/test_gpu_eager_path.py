@@ -89,3 +89,26 @@ def test_modes_and_transforms_get_the_operator():
         assert torch.equal(ops.attention(x, *kv, cos, sin), y)
     with pytest.raises(RuntimeError):  # CPU tensors stay refused
         ops.attention(*(t.detach().cpu() for t in qkv), cos, sin)
+
+
+@pytest.mark.parametrize("dtype,D", [(torch.bfloat16, 64), (torch.float32, 64)])
+def test_modes_around_the_backward_get_the_operator(dtype, D):
+    announce(f"eager path backward modes {dtype}")
+    qkv, do, cos, sin = _case(dtype, D=D)
+    dos = torch.stack([do, 2 * do])
+    out = ops.attention(*qkv, cos, sin)
+    for i in range(2):
+        want = torch.autograd.grad(out, qkv, dos[i], retain_graph=True)
+        got = torch.autograd.grad(out, qkv, dos, is_grads_batched=True, retain_graph=True)
+        for x, y in zip(want, got):
+            assert torch.equal(x, y[i])
+    names = []
+
+    class Seen(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            names.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    with Seen():
+        torch.autograd.grad(out, qkv, do)
+    assert any("kf.attn_bwd" in n for n in names)
