@@ -170,8 +170,6 @@ int narrow(NarrowJobs& jobs, int n, int dtype, int D, hipStream_t stream) {
   });
 }
 
-bool al16(const void* p) { return ((uintptr_t)p & 15) == 0; }
-
 // Sequences up to this length stay on the generic kernels: with one launch
 // against three the forward takes 32 us per call there against 39 (S = 16, B =
 // 1, 4 heads of 96, calls queued back to back), from 32 on 51 against 36.
