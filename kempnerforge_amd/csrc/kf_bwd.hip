@@ -982,7 +982,9 @@ __global__ __launch_bounds__(64 * HB * QT * KSP) void bwd_dq_ds_kernel(
   const int wh = QT == 1 ? w : __builtin_amdgcn_readfirstlane(w % HB);  // its head of the group
   const int hg = (logical / nqg) % ngrp, hidx = logical / nqg / ngrp;
   // masked: the batch rows fastest (kpm_head), since their tiles to visit differ
-  // (packed documents, 4 x 4096, 32/8 heads, whole layer 1345 -> 1320 us)
+  // (packed documents, 4 x 4096, 32/8 heads: two sets of documents took the whole
+  // layer from 1345 to 1320 and from 1241 to 1209 us; in a third this kernel
+  // alone went from 326 to 237)
   const int bh = LIST ? kpm_head(hidx, gridDim.x / (nqg * ngrp) / Hkv, Hkv) : hidx;
   const int b = bh / Hkv, g = bh % Hkv;
   const int nqtp = P / DSQ;
