@@ -943,10 +943,13 @@ __device__ __forceinline__ void dma16_nt(uint32_t lds, uint32_t voff, const void
 // wavefronts.  A wavefront whose tile has fewer columns, or does not exist,
 // loads a record again (the load counts stay equal across wavefronts) and
 // skips the products.
-// KSP > 1 (unmasked): a step takes KSP record columns, one per slice of HB * QT
-// wavefronts, and the slices' float32 sums meet in LDS at the end.  A grid that
-// leaves the chip idle lasts as long as its longest tile's chain of steps (0.5
-// to 0.9 us each), which this divides by KSP.  dq_split() chooses both.
+// KSP > 1 (unmasked and KPM): a step takes KSP record columns, one per slice of
+// HB * QT wavefronts, and the slices' float32 sums meet in LDS at the end.  A
+// grid that leaves the chip idle lasts as long as its longest tile's chain of
+// steps (0.5 to 0.9 us each), which this divides by KSP.  dq_split() chooses
+// both; KPM takes the KSP an unmasked launch of its sizes takes (a column's
+// slice is its parity, in a list of whole 64-key tiles too), so that the sums
+// of a batch row without padding are added in the unmasked launch's order.
 template <typename T, int D, int HB, int QT, int KSP, int MODE, int NBUF>
 __global__ __launch_bounds__(64 * HB * QT * KSP) void bwd_dq_ds_kernel(
     const u32x4* __restrict__ dsb, const T* __restrict__ krot, const float* __restrict__ cos,
@@ -956,7 +959,8 @@ __global__ __launch_bounds__(64 * HB * QT * KSP) void bwd_dq_ds_kernel(
   constexpr bool DOC = MODE == MASK_DOC, KPM = MODE == MASK_KPM, LIST = DOC || KPM;
   constexpr int NW = HB * QT, KR = D / 8, DT = D / 32, HALF = D / 2;
   static_assert(NBUF == 3 || NBUF == 4, "ring depth");
-  static_assert((QT == 1 && KSP == 1) || !LIST, "tile lists are per query tile");
+  static_assert(QT == 1 || !LIST, "tile lists are per query tile");
+  static_assert(KSP <= 2 || !LIST, "a listed tile is two columns");
   constexpr int KI = DSK * KR / 64;  // 1 KB load instructions per K step
   static_assert(KI % NW == 0, "K rows must split evenly over the wavefronts");
   // load instructions per wavefront and step: its share of K, its record's 4 KB
@@ -1566,9 +1570,9 @@ int launch_dq_ds(const BwdArgs& a, const Ws& w) {
     KF_CHECK_LAUNCH();
     return KF_OK;
   }
-  const bool mask = a.doc || a.kvalid;
   const int ntile = a.B * a.Hkv * (n_rep / HB) * nqt;
-  const DqSplit sp = mask ? DqSplit{1, 1} : dq_split(HB, ntile, nqt);
+  DqSplit sp = a.doc ? DqSplit{1, 1} : dq_split(HB, ntile, nqt);
+  if (a.kvalid) sp.qt = 1;  // (the same sums: a tile's do not depend on its neighbour)
   const int nwg = ntile / nqt * ((nqt + sp.qt - 1) / sp.qt);
   auto kernel = a.doc      ? (deep ? bwd_dq_ds_kernel<T, D, HB, 1, 1, MASK_DOC, 4>
                                    : bwd_dq_ds_kernel<T, D, HB, 1, 1, MASK_DOC, 3>)
@@ -1581,6 +1585,9 @@ int launch_dq_ds(const BwdArgs& a, const Ws& w) {
   }
   if constexpr (HB == 2) {
     if (sp.qt == 1 && sp.ksp == 2) kernel = bwd_dq_ds_kernel<T, D, HB, 1, 2, MASK_NONE, 3>;
+  }
+  if constexpr (HB <= 2) {
+    if (a.kvalid && sp.ksp == 2) kernel = bwd_dq_ds_kernel<T, D, HB, 1, 2, MASK_KPM, 3>;
   }
   KF_LAUNCH("bwd_dq_ds", kernel, dim3(nwg), dim3(64 * HB * sp.qt * sp.ksp), 0, a.stream, w.dsb,
             (const T*)w.krot, a.cos, a.sin, (T*)a.dq, a.S, P, a.Hq, a.Hkv, n_rep, nqt, a.causal,

@@ -275,3 +275,36 @@ def test_mixed_batch_split_paths():
     dq, dk, dv = ref.attention_bwd(q, k, v, cos, sin, do, key_padding_mask=kpm)
     for got, want, name in ((qd.grad, dq, "dq"), (kd.grad, dk, "dk"), (vd.grad, dv, "dv")):
         check_grad(got, want, dtype, name, group=Hq // Hkv if name != "dq" else 1)
+
+
+@pytest.mark.parametrize("cfg", [
+    # B, S, Hq, Hkv, D: how an unmasked launch of these sizes splits dQ's sums
+    (2, 1100, 12, 12, 64),   # one head per workgroup, two key slices
+    (1, 1300, 6, 2, 128),    # n_rep 3
+    (1, 1300, 4, 2, 128),    # two heads, two slices
+    (2, 2083, 24, 12, 64),   # two heads, two tiles and two slices
+    (1, 700, 4, 2, 64),      # two heads, whole sums
+], ids=lambda c: "-".join(map(str, c)))
+def test_all_valid_mask_equals_unmasked_backward_small_groups(cfg):
+    """As above for KV groups of few query heads, whose unmasked dQ splits each
+    sum over two key slices; a batch row padded on the right beside it keeps
+    within tolerance of the oracle."""
+    B, S, Hq, Hkv, D = cfg
+    announce(f"kpm all-valid == unmasked backward {cfg}")
+    host = _inputs(torch.bfloat16, B, S, Hq, Hkv, D, seed=7)
+    q, k, v, do, cos, sin = (t.to(DEV) for t in host)
+    ones = torch.ones(B, S, dtype=torch.bool, device=DEV)
+    out, lse = ops.fwd_raw(q, k, v, cos, sin, causal=True, k_rotated=False)
+    g_mask = ops.bwd_raw(q, k, v, cos, sin, out, lse, do, causal=True, key_padding_mask=ones)
+    g_none = ops.bwd_raw(q, k, v, cos, sin, out, lse, do, causal=True)
+    torch.cuda.synchronize()
+    for a, b_, name in zip(g_mask, g_none, ("dq", "dk", "dv")):
+        assert torch.equal(a, b_), f"{name}: max diff {(a.float() - b_.float()).abs().max().item()}"
+    kpm = ones.cpu()
+    kpm[-1, S - 333:] = False
+    out, lse = ops.fwd_raw(q, k, v, cos, sin, causal=True, k_rotated=False,
+                           key_padding_mask=kpm.to(DEV))
+    got = ops.bwd_raw(q, k, v, cos, sin, out, lse, do, causal=True, key_padding_mask=kpm.to(DEV))
+    want = ref.attention_bwd(*host[:3], *host[4:], host[3], key_padding_mask=kpm)
+    for a, w, name in zip(got, want, ("dq", "dk", "dv")):
+        check_grad(a, w, torch.bfloat16, name, group=1 if name == "dq" else Hq // Hkv)
