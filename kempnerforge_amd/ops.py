@@ -272,11 +272,19 @@ def bwd_raw(q, k, v, cos, sin, out, lse, dout, *, causal: bool, doc_ids=None,
 _KF_ERR_UNSUPPORTED = 2
 
 
-@functools.lru_cache(maxsize=4096)
 def rot_size(B: int, S: int, Hq: int, Hkv: int, D: int, dtype: torch.dtype, has_doc: bool,
              has_key_padding: bool) -> int:
     """Bytes of the rotated-operand buffer of :func:`fwd_rot_raw`, or 0 when that
-    path does not take these sizes, dtype or mask kinds (``kf_attn_rot_size``)."""
+    path does not take these sizes, dtype or mask kinds (``kf_attn_rot_size``).
+    Symbolic sizes (the fake kernel under dynamic shapes) are specialised."""
+    return _rot_size(int(B), int(S), int(Hq), int(Hkv), int(D), dtype, bool(has_doc),
+                     bool(has_key_padding))
+
+
+# (real ints only: a SymInt does not hash)
+@functools.lru_cache(maxsize=4096)
+def _rot_size(B: int, S: int, Hq: int, Hkv: int, D: int, dtype: torch.dtype, has_doc: bool,
+              has_key_padding: bool) -> int:
     lib = _lib.load()
     if dtype not in _DTYPES or not hasattr(lib, "kf_attn_rot_size"):  # (a KF_ATTN_LIB build
         return 0                                                        # predating the pair)
