@@ -670,7 +670,11 @@ def attention(q, k, v, rope_cos, rope_sin, *, causal: bool = True, doc_ids=None,
     # written (q and k rotated, (B*Hkv + B*Hq)*S*D elements) and never read
     keep_rot = torch.is_grad_enabled() and (q.requires_grad or k.requires_grad
                                             or v.requires_grad)
-    if _plain_eager(q, k, v, rope_cos, rope_sin, doc_ids, key_padding_mask):
+    # (tables that alone require a gradient get none, but the result is still
+    # part of the graph: left to the operator's formula)
+    only_tables = (not keep_rot and torch.is_grad_enabled()
+                   and (rope_cos.requires_grad or rope_sin.requires_grad))
+    if not only_tables and _plain_eager(q, k, v, rope_cos, rope_sin, doc_ids, key_padding_mask):
         if keep_rot:
             return _Attention.apply(q, k, v, rope_cos, rope_sin, causal, doc_ids,
                                     key_padding_mask)

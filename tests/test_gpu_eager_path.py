@@ -112,3 +112,18 @@ def test_modes_around_the_backward_get_the_operator(dtype, D):
     with Seen():
         torch.autograd.grad(out, qkv, do)
     assert any("kf.attn_bwd" in n for n in names)
+
+
+def test_tables_that_require_a_gradient():
+    """Trainable RoPE tables keep the result in the graph, as the operator does,
+    with or without trainable q, k and v; they get no gradient."""
+    announce("eager path trainable tables")
+    qkv, do, cos, sin = _case()
+    cos.requires_grad_(True)
+    for ts in (qkv, [t.detach() for t in qkv]):
+        out = ops.attention(*ts, cos, sin)
+        assert out.requires_grad
+        out.backward(do)
+        assert cos.grad is None
+    with torch.no_grad():
+        assert not ops.attention(*qkv, cos, sin).requires_grad
