@@ -1414,16 +1414,23 @@ int fwd_f32_t(const FwdArgs& a, void* workspace) {
 // 30 us, not included): D 128, 32/8 heads B = 1 S = 1024 734 / 209 us, S = 2048
 // 1475 / 719, S = 4096 (512 items) 2966 / 2578; D 64, 4/2 heads, B = 2 S = 256 62 /
 // 13; 16 heads of 96 without groups, B = 2 S = 1024 (512 items) 160 / 152 with two
-// runs, and 15 for their sum: not split.
-int dkdv_parts(int B, int S, int Hq, int Hkv) {
+// runs, and 15 for their sum: not split.  The parts take 8 D bytes per key row,
+// part and KV head, at most PARTS_MAX: 16 query heads per group at 1024 items of
+// D 128 (64/2 heads, S = 16000, 1000 MiB: dK/dV 90.2 ms unsplit, 76.4 with the
+// parts and their sum; 64/4, B = 2, S = 6000, 750 MiB: 23.0 and 22.0).
+constexpr size_t PARTS_MAX = (size_t)1 << 30;
+size_t parts_bytes(int B, int S, int Hq, int Hkv, int D, int nseg) {
+  return (size_t)B * S * Hkv * (Hq / Hkv) * nseg * 2 * D * sizeof(float);
+}
+int dkdv_parts(int B, int S, int Hq, int Hkv, int D) {
   const int64_t items = (int64_t)((S + F_BK - 1) / F_BK) * B * Hkv;
   const int64_t cus = device_cu_count();
   const int n_rep = Hq / Hkv, nt = (S + F_BN - 1) / F_BN;
   if (items >= 4 * cus) return 0;
-  if (items >= 2 * cus) return n_rep > 1 ? 1 : 0;
   const int64_t heads = items * n_rep;
   const int nseg = (int)std::min<int64_t>({(2 * cus + heads - 1) / heads, 8, nt});
-  return n_rep * nseg == 1 ? 0 : nseg;
+  if (n_rep * nseg == 1 || parts_bytes(B, S, Hq, Hkv, D, nseg) > PARTS_MAX) return 0;
+  return nseg;
 }
 
 // backward workspace: rotated Q, rotated K, row statistics, then the split
@@ -1433,17 +1440,16 @@ size_t bwd_base_bytes(int B, int S, int Hq, int Hkv, int D, size_t* sum_off) {
   const size_t f = ((size_t)B * Hq * Sp * D + (size_t)B * Hkv * Sp * D + (size_t)B * Hq * Sp * 2) *
                    sizeof(float);
   *sum_off = al256(f);
-  const size_t kv = (size_t)B * S * Hkv * D * 2;
-  const int nseg = dkdv_parts(B, S, Hq, Hkv);
-  return *sum_off + (nseg > 0     ? kv * (Hq / Hkv) * nseg * sizeof(float)
-                     : Hq > Hkv ? kv * sizeof(double)
+  const int nseg = dkdv_parts(B, S, Hq, Hkv, D);
+  return *sum_off + (nseg > 0   ? parts_bytes(B, S, Hq, Hkv, D, nseg)
+                     : Hq > Hkv ? (size_t)B * S * Hkv * D * 2 * sizeof(double)
                                 : 0);
 }
 
 template <int D, int MODE, bool REC>
 void launch_dkdv(const BwdArgs& a, const F32BwdWs& w, int n_rep, unsigned nkblk,
                  const MaskRec& mr, float* rec, int64_t rnt) {
-  const int nseg = dkdv_parts(a.B, a.S, a.Hq, a.Hkv), nparts = nseg > 0 ? n_rep * nseg : 1;
+  const int nseg = dkdv_parts(a.B, a.S, a.Hq, a.Hkv, D), nparts = nseg > 0 ? n_rep * nseg : 1;
   float* part = (float*)w.sum64;
   KF_LAUNCH("bwd_dkdv_f32",
             (nseg > 0 ? bwd_dkdv_f32_kernel<D, MODE, REC, true>

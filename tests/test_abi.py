@@ -196,3 +196,18 @@ def test_noalloc_rejects_oversized_partials():
                                     None, None, ctypes.c_float(1e-5), _lib.DTYPE_BF16,
                                     ctypes.c_void_p(0))
     assert rc == 4 and b"static scratch" in lib.kf_last_error()
+
+
+def test_float32_partial_sums_are_bounded():
+    """The float32 backward's workspace beyond the operands, statistics and
+    group sums it always holds: at most 1 GiB of partial dK and dV sums."""
+    if not os.path.exists(_lib.LIB_PATH):
+        pytest.skip("library not built")
+    lib, n = _lib.load(), _lib.size_out()
+    for B, S, Hq, Hkv in ((1, 16000, 64, 2), (1, 16000, 128, 2), (4, 16000, 64, 1),
+                          (15, 4096, 64, 1), (2, 1024, 16, 4)):
+        for D in (32, 64, 96, 128):
+            assert lib.kf_attn_bwd_workspace_size(B, S, Hq, Hkv, D, 0, ctypes.byref(n)) == 0
+            Sp = (S + 63) // 64 * 64
+            held = 4 * (B * (Hq + Hkv) * Sp * D + 2 * B * Hq * Sp) + 16 * B * S * Hkv * D
+            assert n.value - held <= (1 << 30) + (1 << 20)  # and the mask records
