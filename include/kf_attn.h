@@ -44,9 +44,18 @@ int kf_version(void);
 /* Message describing the last error returned on this thread ("" if none). */
 const char* kf_last_error(void);
 
-/* Workspace bytes kf_attn_fwd needs for these sizes (0 is possible). */
+/* Workspace bytes with which kf_attn_fwd takes its fastest kernels for these
+ * sizes (0 is possible). */
 int kf_attn_fwd_workspace_size(int B, int Sq, int Sk, int Hq, int Hkv, int D, int dtype,
                                size_t* bytes);
+
+/* The fewest workspace bytes with which kf_attn_fwd and kf_attn_capture run.
+ * Head sizes 64 and 128: kf_attn_fwd_workspace_size.  Other head sizes: 0; with
+ * less than kf_attn_fwd_workspace_size (float32 copies of q, k, v and out, or
+ * the rotated keys) they run on the generic kernels, one wavefront per row, at
+ * a fraction of the speed. */
+int kf_attn_fwd_workspace_size_min(int B, int Sq, int Sk, int Hq, int Hkv, int D, int dtype,
+                                   size_t* bytes);
 
 /* Causal (or full) GQA attention forward with RoPE fused.
  *
@@ -84,8 +93,19 @@ int kf_attn_fwd(const void* q, const void* k, const void* v, const float* rope_c
                 int k_rotated, int causal, const int32_t* doc_ids, const int32_t* key_valid,
                 int dtype, void* stream);
 
-/* Workspace bytes kf_attn_bwd needs. */
+/* Workspace bytes with which kf_attn_bwd takes its fastest kernels short of
+ * keeping dS (below). */
 int kf_attn_bwd_workspace_size(int B, int S, int Hq, int Hkv, int D, int dtype, size_t* bytes);
+
+/* The fewest workspace bytes with which kf_attn_bwd runs.  bf16 and fp16 at head
+ * sizes 64 and 128: kf_attn_bwd_workspace_size.  float32 at those sizes: without
+ * the partial dK and dV sums of small grids (up to 1 GiB); with less than
+ * kf_attn_bwd_workspace_size the dK/dV items are not split.  Other head sizes:
+ * the row statistics only; with less than kf_attn_bwd_workspace_size (float32
+ * copies of every operand and result, and the partial sums) they run on the
+ * generic kernels. */
+int kf_attn_bwd_workspace_size_min(int B, int S, int Hq, int Hkv, int D, int dtype,
+                                   size_t* bytes);
 
 /* Workspace bytes with which kf_attn_bwd keeps the dS tiles (bf16 or fp16, the
  * input's type) of the dK/dV
@@ -96,7 +116,8 @@ int kf_attn_bwd_workspace_size(int B, int S, int Hq, int Hkv, int D, int dtype, 
  * tiles are written only where documents meet; with key_valid only causal
  * launches keep them, and only for the batch rows whose key 0 is valid, which
  * have no rows attending past the diagonal: the others recompute, decided on
- * the device).  float32 (head_dim 64 or 128, no doc_ids or key_valid) keeps
+ * the device).  float32 (head_dim 32, 64, 96 or 128, no doc_ids or key_valid),
+ * and the head sizes that run on the float32 kernels through copies, keep
  * float32 [32][64] dS blocks, (t/2 + 1) per 32-position tile t when causal,
  * S/32 * ceil(S/64) for full attention, per query head, up to 32 GiB.
  * Otherwise this equals kf_attn_bwd_workspace_size.  kf_attn_bwd takes the faster path whenever

@@ -97,6 +97,14 @@ static size_t bwd_ws(const BwdArgs& a) {
   return bwd_generic_workspace(a.B, a.S, a.Hq);
 }
 
+// the least a call of these arguments runs with
+static size_t bwd_ws_min(const BwdArgs& a) {
+  if (bwd_mfma_supported(a)) return bwd_ws(a);
+  if (bwd_f32_supported(a) && own_dim(a.D))
+    return bwd_f32_workspace_min(a.B, a.S, a.Hq, a.Hkv, a.D);
+  return bwd_generic_workspace(a.B, a.S, a.Hq);
+}
+
 }  // namespace kf
 
 using namespace kf;
@@ -120,6 +128,13 @@ int kf_attn_fwd_workspace_size(int B, int Sq, int Sk, int Hq, int Hkv, int D, in
                        nullptr);
   *bytes = fwd_ws(a);
   return KF_OK;
+}
+
+int kf_attn_fwd_workspace_size_min(int B, int Sq, int Sk, int Hq, int Hkv, int D, int dtype,
+                                   size_t* bytes) {
+  const int rc = kf_attn_fwd_workspace_size(B, Sq, Sk, Hq, Hkv, D, dtype, bytes);
+  if (rc == KF_OK && !own_dim(D)) *bytes = 0;
+  return rc;
 }
 
 int kf_attn_fwd(const void* q, const void* k, const void* v, const float* rope_cos,
@@ -181,6 +196,15 @@ int kf_attn_bwd_workspace_size(int B, int S, int Hq, int Hkv, int D, int dtype, 
   return KF_OK;
 }
 
+int kf_attn_bwd_workspace_size_min(int B, int S, int Hq, int Hkv, int D, int dtype,
+                                   size_t* bytes) {
+  int rc = check_common(B, S, S, Hq, Hkv, D, dtype);
+  if (rc) return rc;
+  KF_CHECK_ARG(bytes != nullptr, "bytes is null");
+  *bytes = bwd_ws_min(sizing_args(B, S, Hq, Hkv, D, dtype, 1));
+  return KF_OK;
+}
+
 int kf_attn_bwd_workspace_size_ds(int B, int S, int Hq, int Hkv, int D, int dtype, int causal,
                                   size_t* bytes) {
   int rc = check_common(B, S, S, Hq, Hkv, D, dtype);
@@ -223,10 +247,10 @@ int kf_attn_bwd(const void* q, const void* k, const void* v, const float* rope_c
   }
   if (bwd_wide_supported(a) && workspace && workspace_bytes >= bwd_wide_workspace(a, false))
     return bwd_wide(a, workspace, workspace_bytes);
-  const bool f32 =
-      bwd_f32_supported(a) &&
-      (own_dim(D) || (workspace && workspace_bytes >= bwd_f32_workspace(B, S, Hq, Hkv, D)));
-  const size_t need = f32 ? bwd_f32_workspace(B, S, Hq, Hkv, D) : bwd_generic_workspace(B, S, Hq);
+  const size_t f32_min = bwd_f32_workspace_min(B, S, Hq, Hkv, D);
+  const bool f32 = bwd_f32_supported(a) &&
+                   (own_dim(D) || (workspace && workspace_bytes >= f32_min));
+  const size_t need = f32 ? f32_min : bwd_generic_workspace(B, S, Hq);
   if (workspace_bytes < need || !workspace) {
     set_error("workspace too small: need %zu bytes, got %zu", need, workspace_bytes);
     return KF_ERR_WORKSPACE;

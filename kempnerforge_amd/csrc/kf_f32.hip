@@ -1434,13 +1434,13 @@ int dkdv_parts(int B, int S, int Hq, int Hkv, int D) {
 }
 
 // backward workspace: rotated Q, rotated K, row statistics, then the split
-// items' parts or (n_rep > 1) the float64 group sums, then the mask records
-size_t bwd_base_bytes(int B, int S, int Hq, int Hkv, int D, size_t* sum_off) {
+// items' parts (nseg > 0) or (n_rep > 1) the float64 group sums, then the mask
+// records
+size_t bwd_base_bytes(int B, int S, int Hq, int Hkv, int D, int nseg, size_t* sum_off) {
   const size_t Sp = (size_t)(S + F_BK - 1) / F_BK * F_BK;
   const size_t f = ((size_t)B * Hq * Sp * D + (size_t)B * Hkv * Sp * D + (size_t)B * Hq * Sp * 2) *
                    sizeof(float);
   *sum_off = al256(f);
-  const int nseg = dkdv_parts(B, S, Hq, Hkv, D);
   return *sum_off + (nseg > 0   ? parts_bytes(B, S, Hq, Hkv, D, nseg)
                      : Hq > Hkv ? (size_t)B * S * Hkv * D * 2 * sizeof(double)
                                 : 0);
@@ -1449,7 +1449,7 @@ size_t bwd_base_bytes(int B, int S, int Hq, int Hkv, int D, size_t* sum_off) {
 template <int D, int MODE, bool REC>
 void launch_dkdv(const BwdArgs& a, const F32BwdWs& w, int n_rep, unsigned nkblk,
                  const MaskRec& mr, float* rec, int64_t rnt) {
-  const int nseg = dkdv_parts(a.B, a.S, a.Hq, a.Hkv, D), nparts = nseg > 0 ? n_rep * nseg : 1;
+  const int nseg = w.nseg, nparts = nseg > 0 ? n_rep * nseg : 1;
   float* part = (float*)w.sum64;
   KF_LAUNCH("bwd_dkdv_f32",
             (nseg > 0 ? bwd_dkdv_f32_kernel<D, MODE, REC, true>
@@ -1614,7 +1614,14 @@ bool bwd_f32_supported(const BwdArgs& a) {
 
 size_t bwd_f32_workspace(int B, int S, int Hq, int Hkv, int D) {
   size_t sum_off = 0;
-  return al256(bwd_base_bytes(B, S, Hq, Hkv, D, &sum_off)) + mask_rec_bytes(B, S);
+  const int nseg = dkdv_parts(B, S, Hq, Hkv, D);
+  return al256(bwd_base_bytes(B, S, Hq, Hkv, D, nseg, &sum_off)) + mask_rec_bytes(B, S);
+}
+
+size_t bwd_f32_workspace_min(int B, int S, int Hq, int Hkv, int D) {
+  size_t sum_off = 0;
+  return std::min(al256(bwd_base_bytes(B, S, Hq, Hkv, D, 0, &sum_off)) + mask_rec_bytes(B, S),
+                  bwd_f32_workspace(B, S, Hq, Hkv, D));
 }
 
 size_t bwd_f32_workspace_ds(int B, int S, int Hq, int Hkv, int D, int causal) {
@@ -1622,11 +1629,12 @@ size_t bwd_f32_workspace_ds(int B, int S, int Hq, int Hkv, int D, int causal) {
   return rb ? al256(bwd_f32_workspace(B, S, Hq, Hkv, D)) + rb : bwd_f32_workspace(B, S, Hq, Hkv, D);
 }
 
-F32BwdWs bwd_f32_carve(int B, int S, int Hq, int Hkv, int D, void* workspace) {
+F32BwdWs bwd_f32_carve(int B, int S, int Hq, int Hkv, int D, void* workspace, size_t bytes) {
   F32BwdWs w;
   w.Sp = (S + F_BK - 1) / F_BK * F_BK;
+  w.nseg = bytes >= bwd_f32_workspace(B, S, Hq, Hkv, D) ? dkdv_parts(B, S, Hq, Hkv, D) : 0;
   size_t sum_off = 0;
-  const size_t base = bwd_base_bytes(B, S, Hq, Hkv, D, &sum_off);
+  const size_t base = bwd_base_bytes(B, S, Hq, Hkv, D, w.nseg, &sum_off);
   w.qrot = (float*)workspace;
   w.krot = w.qrot + (size_t)B * Hq * w.Sp * D;
   w.stats = w.krot + (size_t)B * Hkv * w.Sp * D;
@@ -1660,7 +1668,7 @@ int bwd_f32_kernels(const BwdArgs& a, const F32BwdWs& w, void* workspace, size_t
 }
 
 int bwd_f32(const BwdArgs& a, void* workspace, size_t workspace_bytes) {
-  const F32BwdWs w = bwd_f32_carve(a.B, a.S, a.Hq, a.Hkv, a.D, workspace);
+  const F32BwdWs w = bwd_f32_carve(a.B, a.S, a.Hq, a.Hkv, a.D, workspace, workspace_bytes);
   int rc = by_dim(a.D, [&](auto d) { return bwd_rows_t<decltype(d)::value>(a, w); });
   if (rc) return rc;
   rc = bwd_f32_stats(a.out, a.dout, a.lse, F32, a.B, a.S, a.Hq, a.D, w, a.stream);

@@ -71,6 +71,8 @@ int fwd_f32(const FwdArgs& a, void* workspace);
 int capture_f32(const FwdArgs& a, float* probs, void* workspace);
 bool bwd_f32_supported(const BwdArgs& a);
 size_t bwd_f32_workspace(int B, int S, int Hq, int Hkv, int D);
+// without the split dK/dV items' parts: what bwd_f32 runs with at the least
+size_t bwd_f32_workspace_min(int B, int S, int Hq, int Hkv, int D);
 // with the dS records (used without an explicit mask when workspace_bytes
 // reaches it: dQ then multiplies them by K instead of recomputing S and dP)
 size_t bwd_f32_workspace_ds(int B, int S, int Hq, int Hkv, int D, int causal);
@@ -84,8 +86,9 @@ struct F32BwdWs {
   double* sum64;       // the group sums, or the split items' float32 parts
   void* masks;
   int Sp;              // S rounded up to 64
+  int nseg;            // runs of the split dK/dV items' heads, 0: not split
 };
-F32BwdWs bwd_f32_carve(int B, int S, int Hq, int Hkv, int D, void* workspace);
+F32BwdWs bwd_f32_carve(int B, int S, int Hq, int Hkv, int D, void* workspace, size_t bytes);
 int bwd_f32_stats(const void* out, const void* dout, const float* lse, int dtype, int B, int S,
                   int Hq, int D, const F32BwdWs& w, hipStream_t stream);
 int bwd_f32_kernels(const BwdArgs& a, const F32BwdWs& w, void* workspace, size_t workspace_bytes);

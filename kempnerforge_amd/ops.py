@@ -68,7 +68,15 @@ def _aligned(t: torch.Tensor) -> torch.Tensor:
     return t if t.data_ptr() % 16 == 0 else t.clone()
 
 
-def _workspace(nbytes: int, device) -> torch.Tensor:
+def _workspace(nbytes: int, device, *smaller) -> torch.Tensor:
+    """``nbytes`` bytes or, where the allocator cannot give them, what the next
+    of ``smaller`` says: functions for the sizes of slower routes, largest
+    first, so that a call that fits without the faster routes' scratch runs."""
+    for size in smaller:
+        try:
+            return torch.empty(max(int(nbytes), 1), dtype=torch.uint8, device=device)
+        except torch.OutOfMemoryError:
+            nbytes = min(nbytes, size())
     return torch.empty(max(int(nbytes), 1), dtype=torch.uint8, device=device)
 
 
@@ -139,8 +147,9 @@ def fwd_raw(q, k, v, cos, sin, *, causal: bool, k_rotated: bool, k_layout: str =
     dt = _dtype_code(q)
     out = torch.empty_like(q)
     lse = torch.empty(B, Hq, Sq, dtype=torch.float32, device=q.device)
-    ws = _workspace(_size("kf_attn_fwd_workspace_size", q.device.index, B, Sq, Sk, Hq, Hkv, D, dt),
-                    q.device)
+    sizes = (q.device.index, B, Sq, Sk, Hq, Hkv, D, dt)
+    ws = _workspace(_size("kf_attn_fwd_workspace_size", *sizes), q.device,
+                    lambda: _size("kf_attn_fwd_workspace_size_min", *sizes))
     _lib.check(lib.kf_attn_fwd(_ptr(q), _ptr(k), _ptr(v), _ptr(cos), _ptr(sin), _ptr(out),
                                _ptr(lse), _ptr(ws), ws.numel(), B, Sq, Sk, Hq, Hkv, D, *kstr,
                                *vstr, int(k_rotated), int(causal), _ptr(doc), _ptr(kv), dt,
@@ -158,7 +167,13 @@ _DS_BUDGET_FRACTION: float | None = 0.5
 def set_backward_low_memory(enabled: bool) -> None:
     """Default of ``bwd_raw``'s ``low_memory`` (and so of the autograd backward of
     :func:`attention` and the ``Attention`` module): True never keeps the dS
-    tiles (about B*Hq*S*S bytes), trading ~5-11% of backward time for memory."""
+    tiles (about B*Hq*S*S bytes), trading ~5-11% of backward time for memory.
+    It does not cover the scratch that grows with S only: head sizes that run
+    through float32 copies (multiples of 16 up to 128 except 64 and 128; float32
+    except 32 and 96 too) take about seven float32 arrays of q's shape in the
+    backward and five in the forward, and backwards on the float32 kernels with
+    small grids up to 1 GiB of partial dK and dV sums.  Both are left out, for
+    slower kernels, when the allocator cannot give them."""
     global _BWD_LOW_MEMORY
     _BWD_LOW_MEMORY = bool(enabled)
     _DS_DECISIONS.clear()
@@ -233,9 +248,10 @@ def bwd_raw(q, k, v, cos, sin, out, lse, dout, *, causal: bool, doc_ids=None,
     for causal attention, 2.2 GB at B=4, S=4096, Hq=32) when those fit in the
     budget of :func:`set_backward_ds_budget` (half the memory the allocator can
     still hand out); otherwise, or with ``low_memory=True``, it passes the
-    minimal workspace and dQ recomputes S and dP (None: the default set by
+    workspace without them and dQ recomputes S and dP (None: the default set by
     :func:`set_backward_low_memory`, initially False).  dK and dV are the same
-    bits either way.
+    bits either way.  Where the allocator has not even those bytes left, a
+    smaller workspace and slower kernels serve the call, if there are any.
     """
     _require_gpu(q, k, v, out, lse, dout)
     lib = _lib.load()
@@ -249,18 +265,19 @@ def bwd_raw(q, k, v, cos, sin, out, lse, dout, *, causal: bool, doc_ids=None,
     kv = _key_valid(key_padding_mask, B, S, q.device)
     dt = _dtype_code(q)
     dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
-    nbytes = _size("kf_attn_bwd_workspace_size", q.device.index, B, S, Hq, Hkv, D, dt)
+    sizes = (q.device.index, B, S, Hq, Hkv, D, dt)
+    nbytes = base = _size("kf_attn_bwd_workspace_size", *sizes)
     low_memory = _BWD_LOW_MEMORY if low_memory is None else low_memory
     # key padding keeps dS only causally, and only for the batch rows whose key
     # 0 is valid (decided on the device; the others recompute)
     if not low_memory and (kv is None or causal):
-        with_ds = _size("kf_attn_bwd_workspace_size_ds", q.device.index, B, S, Hq, Hkv, D, dt,
-                        int(causal))
+        with_ds = _size("kf_attn_bwd_workspace_size_ds", *sizes, int(causal))
         key = ("bwd", q.device, B, S, Hq, Hkv, D, q.dtype, bool(causal), doc is not None,
                kv is not None)
         if _keep_ds_for(key, with_ds - nbytes, q.device):
             nbytes = with_ds
-    ws = _workspace(nbytes, q.device)
+    ws = _workspace(nbytes, q.device, lambda: base,
+                    lambda: _size("kf_attn_bwd_workspace_size_min", *sizes))
     _lib.check(lib.kf_attn_bwd(_ptr(q), _ptr(k), _ptr(v), _ptr(cos), _ptr(sin), _ptr(out),
                                _ptr(lse), _ptr(dout), _ptr(dq), _ptr(dk), _ptr(dv), _ptr(ws),
                                ws.numel(), B, S, Hq, Hkv, D, int(causal), _ptr(doc), _ptr(kv),
@@ -372,7 +389,7 @@ def bwd_rot_raw(rot, v, cos, sin, out, lse, dout, *, causal: bool, doc_ids=None,
     dq, dk, dv = torch.empty_like(out), torch.empty_like(v), torch.empty_like(v)
     sizes = ("kf_attn_bwd_rot_workspace_size", out.device.index, B, S, Hq, Hkv, D, dt,
              int(causal))
-    nbytes = _size(*sizes, 0)
+    nbytes = base = _size(*sizes, 0)
     low_memory = _BWD_LOW_MEMORY if low_memory is None else low_memory
     if not low_memory and (kv is None or causal):  # as in bwd_raw
         with_ds = _size(*sizes, 1)
@@ -380,7 +397,7 @@ def bwd_rot_raw(rot, v, cos, sin, out, lse, dout, *, causal: bool, doc_ids=None,
                kv is not None)
         if _keep_ds_for(key, with_ds - nbytes, out.device):
             nbytes = with_ds
-    ws = _workspace(nbytes, out.device)
+    ws = _workspace(nbytes, out.device, lambda: base)
     _lib.check(lib.kf_attn_bwd_rot(_ptr(rot), _ptr(v), _ptr(cos), _ptr(sin), _ptr(out),
                                    _ptr(lse), _ptr(dout), _ptr(dq), _ptr(dk), _ptr(dv),
                                    _ptr(ws), ws.numel(), B, S, Hq, Hkv, D, int(causal),
@@ -493,8 +510,9 @@ def capture_raw(q, k, v, cos, sin, *, causal: bool, k_rotated: bool, k_layout: s
     out = torch.empty_like(q)
     lse = torch.empty(B, Hq, Sq, dtype=torch.float32, device=q.device)
     probs = torch.empty(B, Hq, Sq, Sk, dtype=torch.float32, device=q.device)
-    ws = _workspace(_size("kf_attn_capture_workspace_size", q.device.index, B, Sq, Sk, Hq, Hkv, D,
-                          dt), q.device)
+    sizes = (q.device.index, B, Sq, Sk, Hq, Hkv, D, dt)
+    ws = _workspace(_size("kf_attn_capture_workspace_size", *sizes), q.device,
+                    lambda: _size("kf_attn_fwd_workspace_size_min", *sizes))
     _lib.check(lib.kf_attn_capture(_ptr(q), _ptr(k), _ptr(v), _ptr(cos), _ptr(sin), _ptr(probs),
                                    _ptr(out), _ptr(lse), _ptr(ws), ws.numel(), B, Sq, Sk, Hq, Hkv,
                                    D, *kstr, *vstr, int(k_rotated), int(causal), _ptr(doc),

@@ -211,3 +211,38 @@ def test_float32_partial_sums_are_bounded():
             Sp = (S + 63) // 64 * 64
             held = 4 * (B * (Hq + Hkv) * Sp * D + 2 * B * Hq * Sp) + 16 * B * S * Hkv * D
             assert n.value - held <= (1 << 30) + (1 << 20)  # and the mask records
+
+
+def test_least_workspaces():
+    """The least workspace of a call, what its fastest kernels take and what
+    kept dS tiles take, in this order."""
+    if not os.path.exists(_lib.LIB_PATH):
+        pytest.skip("library not built")
+    lib = _lib.load()
+
+    def size(entry, *sizes):
+        n = _lib.size_out()
+        assert getattr(lib, entry)(*sizes, ctypes.byref(n)) == 0
+        return n.value
+
+    for B, S, Hq, Hkv in ((1, 1, 1, 1), (2, 1024, 16, 4), (1, 16000, 64, 2), (1, 16000, 128, 2),
+                          (4, 4096, 32, 8), (1, 300, 64, 1)):
+        for D in (16, 32, 40, 64, 96, 128, 160):
+            for dt in (_lib.DTYPE_F32, _lib.DTYPE_BF16, _lib.DTYPE_F16):
+                a = (B, S, Hq, Hkv, D, dt)
+                least, base, ds = (size("kf_attn_bwd_workspace_size_min", *a),
+                                   size("kf_attn_bwd_workspace_size", *a),
+                                   size("kf_attn_bwd_workspace_size_ds", *a, 1))
+                assert 0 < least <= base <= ds
+                f = (B, S, S) + a[2:]
+                fleast = size("kf_attn_fwd_workspace_size_min", *f)
+                assert fleast <= size("kf_attn_fwd_workspace_size", *f)
+                if D not in (64, 128):
+                    assert fleast == 0 and least == 4 * B * S * (Hq + 1)  # row statistics
+                elif dt == _lib.DTYPE_F32:
+                    Sp = (S + 63) // 64 * 64
+                    held = 4 * (B * (Hq + Hkv) * Sp * D + 2 * B * Hq * Sp)
+                    sums = 16 * B * S * Hkv * D if Hq > Hkv else 0
+                    assert 0 <= least - held - sums < (1 << 16) + 8 * B * S  # mask records
+                else:
+                    assert least == base
