@@ -162,11 +162,16 @@ def attention_kernel_flops(pairs: int, head_dim: int, backward: bool = True) -> 
 
 
 # ---------------------------------------------------------------- profiler
-_ATTN_KEYS = ("fwd_mfma", "bwd_dkdv", "bwd_dq", "q_prep_bwd", "kv_prep", "decode_stream",
-              "decode_merge", "decode_generic", "capture_probs", "capture_tiles", "fwd_generic",
-              "bwd_dq_generic", "bwd_dkdv_generic", "cache_append", "append_kernel",
-              "doc_block_tiles", "order_by_count", "widen_kernel", "narrow_kernel", "_f32_kernel",
-              "kf::attn", "flash", "fmha", "attention")
+# every kernel of kempnerforge_amd/csrc (a key covers the names it is part of),
+# then the operator and what other attention libraries call theirs
+_ATTN_KEYS = ("fwd_mfma", "fwd32_kernel", "bwd_dkdv", "dkdv_reduce_kernel", "bwd_dq",
+              "bwd_delta_kernel", "q_prep_bwd", "kv_prep", "kpm_row_keys_kernel",
+              "doc_block_tiles", "order_by_count", "decode_stream", "decode_merge",
+              "decode_generic", "decode_f32_kernel", "capture_probs", "capture_tiles",
+              "capture_f32_kernel", "fwd_generic", "fwd_f32_kernel", "rows_f32_kernel",
+              "stats_f32_kernel", "mask_prep_f32_kernel", "dkdv_parts_f32_kernel",
+              "widen_kernel", "narrow_kernel", "cache_append", "append_kernel",
+              "append_rows_kernel", "kf::attn", "flash", "fmha", "attention")
 _MATMUL_KEYS = ("gemm", "mm", "matmul", "dot", "bmm", "cublas", "nvjet", "cutlass",
                 "cijk_", "hipblaslt", "rocblas", "ck_tile", "wvsplitk")
 _COMM_KEYS = ("nccl", "rccl", "allreduce", "allgather", "reduce_scatter", "alltoall")

@@ -5,6 +5,8 @@ checked the way the reference checks its own (tests/unit/test_performance.py:
 from __future__ import annotations
 
 import math
+import os
+import re
 from dataclasses import dataclass
 from types import SimpleNamespace
 from unittest.mock import MagicMock
@@ -161,6 +163,32 @@ class TestClassifier:
     ])
     def test_buckets(self, name, bucket):
         assert mfu.classify_kernel(name) == bucket
+
+    def test_every_kernel_of_the_library(self):
+        """Each __global__ function, by its plain, demangled and mangled name."""
+        src = os.path.join(os.path.dirname(mfu.__file__), "csrc")
+        names = set()
+        for f in sorted(os.listdir(src)):
+            if f.endswith(".hip"):
+                text = open(os.path.join(src, f)).read()
+                names |= set(re.findall(r"__global__[^;{]*?\bvoid\s+(\w+)\(", text))
+        assert {"fwd32_kernel", "append_rows_kernel", "kpm_row_keys_kernel"} <= names
+        assert len(names) > 30
+        for k in sorted(names):
+            for name in (k, f"void kf::(anonymous namespace)::{k}<__bf16, 128>(int)",
+                         f"_ZN2kf12_GLOBAL__N_1{len(k)}{k}IDF16bLi128EEEvi"):
+                assert mfu.classify_kernel(name) == "attention", name
+
+    def test_bench_short_names(self):
+        import bench
+
+        for k, short in (("append_rows_kernel", "kv_append"), ("append_kernel", "kv_append"),
+                         ("fwd32_kernel", "fwd_mfma"), ("kpm_row_keys_kernel", "kpm_row_keys")):
+            assert bench._short(f"_ZN2kf12_GLOBAL__N_1{len(k)}{k}IDF16bEEvi") == short
+
+    def test_other_float32_kernels(self):
+        assert mfu.classify_kernel("gemm_f32_kernel") == "matmul"
+        assert mfu.classify_kernel("softmax_f32_kernel") == "other"
 
     def test_analyze_profiler(self, monkeypatch):
         monkeypatch.setattr(mfu, "get_gpu_peak_tflops", lambda device=0: 2516.6)
