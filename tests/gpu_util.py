@@ -3,6 +3,7 @@
 from __future__ import annotations
 
 import os
+import re
 import sys
 
 import numpy as np
@@ -111,6 +112,27 @@ def check_out(got, want, tol: float, name: str) -> float:
     print(f"[{name}] max-abs err {e:.3e} (tol {tol:g})", flush=True)
     assert e <= tol, f"{name}: max-abs error {e:.3e} > {tol:g}"
     return e
+
+
+def kernel_variants(fn, kernel: str) -> list[tuple[int, ...]]:
+    """The integer and truth-value template arguments of each launch of
+    ``kernel`` while ``fn`` runs, from the profiler's (mangled or demangled)
+    symbol names."""
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+        fn()
+        torch.cuda.synchronize()
+    out = []
+    for e in prof.events():
+        m = re.search(r"\d" + kernel + r"I(.*?)EEv", e.name)
+        if m:
+            out.append(tuple(int(x) for x in re.findall(r"L[ib](\d+)E", m.group(1) + "E")))
+            continue
+        m = re.search(r"\b" + kernel + r"<(.*?)>\(", e.name)
+        if m:
+            words = [w.strip() for w in m.group(1).split(",")]
+            out.append(tuple({"true": 1, "false": 0}.get(w) if w in ("true", "false") else int(w)
+                             for w in words if w in ("true", "false") or w.isdigit()))
+    return out
 
 
 def load_fixture(name):

@@ -7,7 +7,7 @@ from __future__ import annotations
 import pytest
 import torch
 
-from gpu_util import DEV, announce, check_grad, seeded
+from gpu_util import DEV, announce, check_grad, kernel_variants, seeded
 from kempnerforge_amd import _lib, ops
 from oracle import attention_ref as ref
 
@@ -46,3 +46,33 @@ def test_gradients(cfg):
     assert "bwd_dq_ds" in t.stats, t.stats
     want = ref.attention_bwd(q, k, v, cos, sin, do, causal=causal)[0]
     check_grad(dq, want, dtype, "dq")
+
+
+@pytest.mark.parametrize("cfg,form", [
+    # dtype, B, S, Hq, Hkv, D; heads, query tiles and key slices per workgroup
+    ((BF16, 1, 193, 3, 3, 128), (1, 2, 2)),
+    ((BF16, 1, 192, 3, 3, 64), (1, 1, 1)),       # three tiles
+    ((BF16, 1, 1000, 2, 1, 64), (2, 1, 2)),
+    ((BF16, 1, 960, 2, 1, 64), (2, 1, 1)),       # 15 tiles
+    ((F16, 2, 2000, 18, 1, 64), (2, 2, 2)),      # 32 tiles, 576 in all
+    ((F16, 2, 1980, 18, 1, 64), (2, 1, 1)),      # 31 tiles
+    ((BF16, 8, 1500, 8, 4, 64), (2, 1, 1)),
+    ((BF16, 3, 1500, 15, 15, 64), (1, 2, 2)),    # 540 workgroups of two tiles and slices
+    ((BF16, 2, 1500, 15, 15, 64), (1, 1, 1)),    # 360
+    ((BF16, 5, 2055, 4, 1, 64), (4, 1, 1)),
+], ids=lambda c: "-".join(map(str, (str(c[0])[6:],) + c[1:])) if len(c) > 3 else
+    "x".join(map(str, c)))
+@pytest.mark.parametrize("padded", [False, True])
+def test_which_form_ran(cfg, form, padded):
+    """Key padding takes the unmasked launch's key slices and one tile."""
+    dtype, B, S, Hq, Hkv, D = cfg
+    announce(f"dq form {cfg} {padded}")
+    q, k, v, do = (seeded((B, S, h, D), i, dtype).to(DEV) for i, h in enumerate((Hq, Hkv, Hkv, Hq)))
+    cos, sin = (t.to(DEV) for t in ref.rope_tables(D, S, 5e5))
+    kw = {"key_padding_mask": torch.ones(B, S, dtype=torch.bool, device=DEV)} if padded else {}
+    out, lse = ops.fwd_raw(q, k, v, cos, sin, causal=True, k_rotated=False, **kw)
+    ran = kernel_variants(lambda: ops.bwd_raw(q, k, v, cos, sin, out, lse, do, causal=True, **kw),
+                          "bwd_dq_ds_kernel")
+    hb, qt, ksp = form
+    # template arguments: D, heads, tiles, slices, mode, ring depth
+    assert [r[:4] for r in ran] == [(D, hb, 1 if padded else qt, ksp)], ran

@@ -6,7 +6,7 @@ from __future__ import annotations
 import pytest
 import torch
 
-from gpu_util import DEV, TOL, announce, check_out, seeded
+from gpu_util import DEV, TOL, announce, check_out, kernel_variants, seeded
 from kempnerforge_amd import ops
 from oracle import attention_ref as ref
 
@@ -60,3 +60,25 @@ def test_infinite_keys_in_one_half():
                              k_rotated=True)
         keep = v[:, 32:] if half == 0 else v[:, :32]
         check_out(out, keep.float().mean(1, keepdim=True).expand(B, S, H, D), TOL[BF16], "out")
+
+
+@pytest.mark.parametrize("cfg,slices", [
+    ((BF16, 1, 1, 4, 2, 128), 2),
+    ((BF16, 1, 200, 64, 1, 128), 2),
+    ((BF16, 1, 200, 80, 1, 64), 1),
+    ((BF16, 1, 1024, 32, 8, 128), 2),    # 256 blocks
+    ((BF16, 1, 1028, 32, 8, 128), 1),    # one more
+    ((BF16, 1, 2047, 4, 2, 128), 2),
+    ((BF16, 1, 2048, 4, 2, 128), 1),
+    ((BF16, 1, 2048, 4, 2, 64), 2),
+    ((F16, 6, 1024, 16, 16, 64), 2),     # 768 blocks
+    ((F16, 6, 1025, 16, 16, 64), 1),
+], ids=lambda c: "-".join(map(str, (str(c[0])[6:],) + c[1:])) if isinstance(c, tuple) else str(c))
+def test_which_form_ran(cfg, slices):
+    dtype, B, S, Hq, Hkv, D = cfg
+    announce(f"fwd slices form {cfg}")
+    q, k, v = (seeded((B, S, h, D), i, dtype).to(DEV) for i, h in enumerate((Hq, Hkv, Hkv)))
+    cos, sin = (t.to(DEV) for t in ref.rope_tables(D, S, 5e5))
+    ran = kernel_variants(lambda: ops.fwd_raw(q, k, v, cos, sin, causal=True, k_rotated=False),
+                          "fwd32_kernel")
+    assert ran == [(D, slices)]
