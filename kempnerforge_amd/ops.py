@@ -343,7 +343,7 @@ def fwd_rot_raw(q, k, v, cos, sin, *, causal: bool, doc_ids=None, key_padding_ma
     sin = _aligned(_rope_table(sin, S, D // 2, "rope_sin"))
     doc = _doc_ids(doc_ids, B, S, q.device)
     kv = _key_valid(key_padding_mask, B, S, q.device)
-    nrot = rot_size(B, S, Hq, Hkv, D, q.dtype, doc is not None, kv is not None)
+    nrot = _rot_size(B, S, Hq, Hkv, D, q.dtype, doc is not None, kv is not None)
     if nrot == 0:
         return None
     dt = _dtype_code(q)
@@ -378,7 +378,7 @@ def bwd_rot_raw(rot, v, cos, sin, out, lse, dout, *, causal: bool, doc_ids=None,
     kv = _key_valid(key_padding_mask, B, S, out.device)
     # the C ABI takes rot without a length: check it here, before any launch,
     # so a rot from another shape or mask kind cannot send the kernels out of bounds
-    want = rot_size(B, S, Hq, Hkv, D, out.dtype, doc is not None, kv is not None)
+    want = _rot_size(B, S, Hq, Hkv, D, out.dtype, doc is not None, kv is not None)
     if (rot.dtype != out.dtype or not rot.is_contiguous() or rot.device != out.device
             or rot.data_ptr() % 16 or want == 0 or rot.numel() * rot.element_size() != want):
         raise ValueError(
