@@ -986,9 +986,9 @@ __global__ __launch_bounds__(64 * HB * QT * KSP) void bwd_dq_ds_kernel(
   const int wh = QT == 1 ? w : __builtin_amdgcn_readfirstlane(w % HB);  // its head of the group
   const int hg = (logical / nqg) % ngrp, hidx = logical / nqg / ngrp;
   // masked: the batch rows fastest (kpm_head), since their tiles to visit differ
-  // (packed documents, 4 x 4096, 32/8 heads: two sets of documents took the whole
-  // layer from 1345 to 1320 and from 1241 to 1209 us; in a third this kernel
-  // alone went from 326 to 237)
+  // (packed documents, 4 x 4096, 32/8 heads, eight sets of documents: this kernel
+  // 228 to 379 us with a row's heads adjacent, 178 to 266 so, each set less by 10
+  // to 36%; a fifth of the layer's pass)
   const int bh = LIST ? kpm_head(hidx, gridDim.x / (nqg * ngrp) / Hkv, Hkv) : hidx;
   const int b = bh / Hkv, g = bh % Hkv;
   const int nqtp = P / DSQ;
@@ -1532,10 +1532,13 @@ Ws carve(void* base, int B, int S, int Hq, int Hkv, int D, const void* rot) {
 //    (12/12 D64 B1 S65 6.6 against 7.5).
 //  - two heads: two slices up to one workgroup per CU (4/2 D64 B3 S1600 23.8 ->
 //    18.6), two tiles as well on larger grids of long sequences (12/2 B2 S4096
-//    134 -> 110, 16/8 B4 S3000 151 -> 141; 12/2 B4 S3000, whose third round is
-//    a quarter full, 113 -> 118).  Sequences below 1024 or, on larger grids,
-//    2048 keep one tile (16/8 B8 S500 21.1 against 25.9 and 23.6, 12/2 B6 S1100
-//    38.9 against 43.4).
+//    134 -> 110, 16/8 B4 S3000 151 -> 141, B6 S6000 813 -> 702).  Of 104 such grids
+//    (S 2048 to 6000) 87 gain, up to 23%; the losses reach 6% (12/2 B3 S2048
+//    69 -> 73, B4 S3000 113 -> 117).  How full the last round is does not tell them
+//    apart: with a quarter (2.2 to 2.25 workgroups per CU) 12/2 B3 S4096 gains 6%,
+//    B6 S2048 4%, B4 S3000 loses 4%, 4/2 D64 B6 S6000 3%.  Sequences below 1024 or,
+//    on larger grids, 2048 keep one tile (16/8 B8 S500 21.1 against 25.9 and
+//    23.6, 12/2 B6 S1100 38.9 against 43.4).
 //  - four heads: one tile; either split came out equal or slower (32/8 B4 S1024
 //    50.7 against 53.6 with two slices).
 struct DqSplit { int qt, ksp; };

@@ -1321,10 +1321,13 @@ void launch_fwd_kernel(const FwdArgs& a, const FwdWs& w, int Skp, int n_rep, int
 // nothing).  One / two slices, forward kernel alone: D 128, 32/8 heads S = 256
 // 14.9 / 13.0 us, 512 19.2 / 16.7, 1000 (256 blocks) 28.9 / 26.1, 1999 (504) 54.9
 // / 56.7, 3000 (752) 91 / 105; D 64, 12 heads S = 2048 37 / 27, B = 2 S = 1024 22.7
-// / 18.1, B = 4 S = 2048 (768) 62 / 51.  With D 128 only below 2048 positions:
-// from there on a sequence's rows are the same bits whatever its length (the
-// slices add up in another order), which the gradients' comparison of a 2048-row
-// prefix with the whole 8256-row sequence holds the kernels to.
+// / 18.1, B = 4 S = 2048 (768) 62 / 51.  With D 128 only below 2048 positions,
+// though it pays beyond (8/2 heads S = 2048 47.0 / 32.8 us, S = 4096 84.8 / 63.2;
+// 4/1 S = 8192 152.8 / 110.3): the slices add up in another order, and the
+// backward's test of an 8256-row sequence wants the first 2048 rows' dQ, and so
+// their out and LSE, to be the bits of a run on those rows alone.  That is no
+// property of the library: rows at D 64, and of sequences shorter than 2048 at
+// D 128, can differ in the last bits with the length and the batch.
 int fwd_slices(int64_t nblk, int n_rep, int D, int Sq) {
   if (n_rep > ROWS / 2 || (D == 128 && Sq >= 2048)) return 1;
   return nblk <= (D == 64 ? 3 : 1) * (int64_t)device_cu_count() ? 2 : 1;

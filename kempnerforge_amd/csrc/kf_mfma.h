@@ -410,9 +410,10 @@ __device__ __forceinline__ int kpm_first_valid(const int2* __restrict__ rec, int
 
 // Launches with key padding (and dQ from records with packed documents) number
 // their (batch row, KV head) groups with the batch rows fastest: group idx of
-// B * Hkv.  An XCD takes a contiguous range of groups, and with a batch row's heads adjacent the XCDs of short (or skipped)
-// rows ran dry: six rows of 1531 positions, each XCD holding the heads of one or
-// two rows, took 1.29 ms forward and backward.
+// B * Hkv.  An XCD takes a contiguous range of groups, and with a batch row's
+// heads adjacent the XCDs of short (or skipped) rows ran dry: six rows of 1531
+// positions, each XCD holding the heads of one or two rows, took 1.29 ms forward
+// and backward.
 __device__ __forceinline__ int kpm_head(int idx, int B, int Hkv) {
   return (idx % B) * Hkv + idx / B;
 }
