@@ -749,7 +749,10 @@ typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
 // except in guarded rows before the first valid key, which attend every key
 // below Sk, so a workgroup holding one walks every tile); with an explicit
 // mask every tile takes the element test.
-template <typename T, int D, int MODE>
+//
+// PST: how rows of P are stored, by their length (p_store).
+enum { P_NT, P_VEC, P_ANY };
+template <typename T, int D, int MODE, int PST>
 __global__ __launch_bounds__(256, 2) void capture_probs_mfma_kernel(
     const T* __restrict__ q, const float* __restrict__ cos, const float* __restrict__ sin,
     const T* __restrict__ krot, const T* __restrict__ vn, T* __restrict__ out,
@@ -866,11 +869,6 @@ __global__ __launch_bounds__(256, 2) void capture_probs_mfma_kernel(
     // in 2*ntiles pieces, one at the start of each tile iteration of the two
     // walks (ahead of that iteration's tile loads), so the zeros stream out
     // while the block computes instead of after it.
-    // Rows that start off 64-byte blocks leave by write-back stores, which L2
-    // joins into whole lines: a non-temporal store of part of a block is a
-    // partial write to memory (S = 3000: 433 against 530 us; on whole blocks
-    // non-temporal is ahead, 270 against 361 at S = 2000, 64 heads).
-    const bool nt = (Sk & 15) == 0;
     const int zstart = ntiles * BN;
     const int zper = causal && zstart < Sk ? (nrows + 2 * ntiles - 1) / (2 * ntiles) : 0;
     auto zero_rows = [&](int z) {
@@ -881,8 +879,10 @@ __global__ __launch_bounds__(256, 2) void capture_probs_mfma_kernel(
         float* zrow =
             probs + (((int64_t)ri.b * Hq + (int64_t)ri.g * n_rep + r / bm_pos) * Sq + pos) * Sk;
         for (int key = zstart + tid * 4; key < Sk; key += 256 * 4) {
-          if (nt) {
+          if (PST == P_NT) {
             __builtin_nontemporal_store(f32x4{0.f, 0.f, 0.f, 0.f}, (f32x4*)(zrow + key));
+          } else if (PST == P_VEC) {
+            *(f32x4*)(zrow + key) = f32x4{0.f, 0.f, 0.f, 0.f};
           } else if (key + 3 < Sk) {
             *(f32x4u*)(zrow + key) = f32x4u{0.f, 0.f, 0.f, 0.f};
           } else {
@@ -986,8 +986,10 @@ __global__ __launch_bounds__(256, 2) void capture_probs_mfma_kernel(
           const f32x4 v4 = *(const f32x4*)&stg[rr * 32 + ((cl ^ (rr & 7)) * 4)];
           const int key = t * BN + 32 * mt + 4 * cl;
           if (!((pvalid >> j) & 1)) continue;
-          if (nt) {
+          if (PST == P_NT) {
             if (key < Sk) __builtin_nontemporal_store(v4, (f32x4*)(prs[j] + key));
+          } else if (PST == P_VEC) {
+            if (key < Sk) *(f32x4*)(prs[j] + key) = v4;
           } else if (key + 3 < Sk) {
             *(f32x4u*)(prs[j] + key) = v4;
           } else {
@@ -1369,11 +1371,27 @@ void launch_fwd_mode(const FwdArgs& a, const FwdWs& w, int Skp, int n_rep, int b
   }
 }
 
+// How rows of Sk probabilities are stored.  Rows of whole 64-byte blocks leave by
+// non-temporal stores; rows that start off them by write-back stores, which L2
+// joins into whole lines, where a non-temporal store of part of a block is a
+// partial write to memory (32/8 heads of 128, S = 3000: 404 against 495 us; on
+// whole blocks non-temporal is ahead, 147 against 165 at S = 2000); rows of no
+// whole 16-byte pieces with a tail of single elements.  A kernel for each: with
+// the three told apart at each store, by a branch, every capture was 15 to 20%
+// slower (S = 1024 100 -> 117 us, 64/8 heads S = 2048 219 -> 271), and rows off
+// 64-byte blocks under a mask another 5 to 10% (S = 1500, packed documents 166
+// now, 199 so).
+int p_store(int Sk) { return Sk % 16 == 0 ? P_NT : Sk % 4 == 0 ? P_VEC : P_ANY; }
+
 template <typename T, int D, int MODE>
 void launch_capture_kernel(const FwdArgs& a, const FwdWs& w, float* probs, int Skp, int n_rep,
                            int bm_pos, int nqb, unsigned nblk) {
-  KF_LAUNCH("capture_probs_mfma", (capture_probs_mfma_kernel<T, D, MODE>), dim3(nblk), dim3(256),
-            0, a.stream, (const T*)a.q, a.cos, a.sin, (const T*)w.krot, (const T*)w.vn,
+  const int pst = p_store(a.Sk);
+  KF_LAUNCH("capture_probs_mfma",
+            (pst == P_NT    ? capture_probs_mfma_kernel<T, D, MODE, P_NT>
+             : pst == P_VEC ? capture_probs_mfma_kernel<T, D, MODE, P_VEC>
+                            : capture_probs_mfma_kernel<T, D, MODE, P_ANY>),
+            dim3(nblk), dim3(256), 0, a.stream, (const T*)a.q, a.cos, a.sin, (const T*)w.krot, (const T*)w.vn,
             (T*)a.out, a.lse, probs, a.Sq, a.Sk, Skp, a.Hq, a.Hkv, n_rep, bm_pos, nqb,
             a.scale * kLog2e, a.causal, a.doc ? a.doc : a.kvalid, w.ranges);
 }

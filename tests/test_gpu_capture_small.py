@@ -8,7 +8,7 @@ from __future__ import annotations
 import pytest
 import torch
 
-from gpu_util import DEV, announce, max_abs, seeded
+from gpu_util import DEV, announce, kernel_variants, max_abs, seeded
 from kempnerforge_amd import _lib, ops
 from oracle import attention_ref as ref
 
@@ -65,3 +65,31 @@ def test_cache(Sq, causal):
     if causal:
         s = s.masked_fill(torch.ones(Sq, Sk, dtype=torch.bool).triu(1), float("-inf"))
     assert max_abs(p, torch.softmax(s, -1)) <= 1e-5
+
+
+P_NT, P_VEC, P_ANY = 0, 1, 2  # non-temporal, 16-byte write-back, and stores with a tail
+
+
+@pytest.mark.parametrize("S,pst", [(144, P_NT), (148, P_VEC), (150, P_ANY), (151, P_ANY)])
+@pytest.mark.parametrize("mask", [None, "doc_ids", "key_padding_mask"])
+@pytest.mark.parametrize("D", [64, 128])
+def test_stores_of_the_fused_kernel(S, pst, mask, D):
+    announce(f"fused capture stores S={S} {mask} D={D}")
+    B, Hq, Hkv = (30, 16, 16) if mask is None else (2, 6, 2)
+    q, k, v = (seeded((B, S, h, D), i, BF16) for i, h in enumerate((Hq, Hkv, Hkv)))
+    cos, sin = ref.rope_tables(D, S, 5e5)
+    m = {}
+    if mask == "doc_ids":
+        m[mask] = (torch.arange(S)[None, :] // torch.tensor([[47], [64]])).to(torch.int32)
+    elif mask:
+        m[mask] = torch.arange(S)[None, :] >= torch.tensor([[0], [9]])  # row 1: guarded rows
+        m[mask][0, 70:] = False
+    args = [t.to(DEV) for t in (q, k, v, cos, sin)]
+    got = []
+    ran = kernel_variants(lambda: got.extend(ops.capture_raw(
+        *args, causal=True, k_rotated=False, **{n: t.to(DEV) for n, t in m.items()})),
+        "capture_probs_mfma_kernel")
+    assert [(r[0], r[2]) for r in ran] == [(D, pst)], ran
+    o_ref, p_ref = ref.capture(q, k, v, cos, sin, **m)
+    assert max_abs(got[1], p_ref) <= 1e-5 and max_abs(got[0], o_ref) <= 2e-2
+    assert got[1].cpu()[p_ref == 0].abs().max().item() == 0.0
