@@ -1459,14 +1459,21 @@ void launch_capture_tiles(const FwdArgs& a, const FwdWs& w, float* probs, int Sk
 
 // Whether the probabilities are formed after the forward (capture_tiles_kernel)
 // instead of in the fused kernel: when the latter would have less than one
-// workgroup per CU.  Whole capture, fused / after the forward (D 128, one
-// sequence): 8 workgroups (S = 128, 32/8 heads) 53 / 26 us, 104 (S = 777) 145 /
-// 58, 128 (S = 1024) 119 / 76, 192 (S = 1536) 147 / 121, 256 (S = 2000) 168 /
-// 199, 512 (S = 2048, 64/8 heads) 257 / 335.  Explicit masks stay fused.
+// workgroup per CU.  Whole capture, fused / after the forward (graph-timed, 32/8
+// heads of 128, one sequence): S = 65 (16 workgroups) 59 / 23 us, 777 (104) 117 /
+// 60, 1000 (128) 100 / 70; only with one query block per head the second launch
+// just adds (S = 17 14.6 / 18.5; 12/12 of 64, S = 128 14.7 / 18.3), which the
+// tests of these sizes still ask for.  The pieces write P at 1.7 TB/s where its rows are off 64-byte
+// blocks, the fused kernel at up to 2.9, so not past 192 MiB of P (S = 1200, 176
+// MiB, 109 / 97; 1500, 275 MiB, 137 / 168); with rows of whole blocks 3 TB/s, not
+// past 320 (16/2 heads S = 2000, 244 MiB, 142 / 118; S = 2400, 352 MiB, 160 / 162).
+// Explicit masks stay fused.
 bool capture_after_fwd(const FwdArgs& a) {
   if (a.doc || a.kvalid) return false;
   const int bm_pos = pick_bm_pos(a.Hq / a.Hkv), nqb = (a.Sq + bm_pos - 1) / bm_pos;
-  return (int64_t)((nqb + 1) / 2) * a.B * a.Hkv < device_cu_count();
+  const int64_t mib = (int64_t)a.B * a.Hq * a.Sq * a.Sk >> 18;
+  return (int64_t)((nqb + 1) / 2) * a.B * a.Hkv < device_cu_count() &&
+         mib <= (p_store(a.Sk) == P_NT ? 320 : 192);
 }
 
 int capture_probs_mfma(const FwdArgs& a, float* probs, void* workspace) {

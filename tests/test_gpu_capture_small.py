@@ -93,3 +93,23 @@ def test_stores_of_the_fused_kernel(S, pst, mask, D):
     o_ref, p_ref = ref.capture(q, k, v, cos, sin, **m)
     assert max_abs(got[1], p_ref) <= 1e-5 and max_abs(got[0], o_ref) <= 2e-2
     assert got[1].cpu()[p_ref == 0].abs().max().item() == 0.0
+
+
+@pytest.mark.parametrize("cfg,after", [
+    ((1, 1200, 32, 8, 64), True),    # 176 MiB of P
+    ((1, 1300, 32, 8, 64), False),   # 206, rows off 64-byte blocks
+    ((1, 1600, 32, 8, 64), True),    # 312, whole blocks
+    ((1, 1632, 32, 8, 64), False),   # 325
+    ((2, 1000, 32, 8, 64), False),   # 256 workgroups of the fused kernel
+], ids=lambda c: "-".join(map(str, c)) if isinstance(c, tuple) else str(c))
+def test_which_form_ran(cfg, after):
+    B, S, Hq, Hkv, D = cfg
+    announce(f"capture form {cfg}")
+    q, k, v = (seeded((B, S, h, D), i, BF16).to(DEV) for i, h in enumerate((Hq, Hkv, Hkv)))
+    cos, sin = (t.to(DEV) for t in ref.rope_tables(D, S, 5e5))
+    got = []
+    ran = kernel_variants(lambda: got.extend(ops.capture_raw(q, k, v, cos, sin, causal=True,
+                                                             k_rotated=False)),
+                          "capture_tiles_kernel")
+    assert len(ran) == after
+    assert max_abs(got[1].sum(-1), torch.ones(B, Hq, S)) <= 1e-5 and (got[1].triu(1) == 0).all()
