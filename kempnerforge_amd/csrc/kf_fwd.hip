@@ -532,12 +532,11 @@ __global__ __launch_bounds__(256, KSL == 1 ? 3 : 2) void fwd32_kernel(
   bf16x8 qf[KS];
   load_q_frag<T, D>(q, cos, sin, ri, Sq, Hq, hh, qf);
 
-  float m = -INFINITY, lsum = 0.f;
-  // KSL 2: a half may hold no visible key for a while, or at all, its max still
-  // -inf: no inf - inf then (a factor of 1, an exponent base of 0)
-  auto factor = [](float from, float to) {
-    return KSL == 2 && from == to ? 1.f : fast_exp2(from - to);
-  };
+  float m = -INFINITY, base = 0.f, lsum = 0.f;  // base: m, or 0 while m is -inf
+  // a half (KSL 2) may hold no visible key for a while, or at all, and a tile's
+  // scores may all be -inf, the max still -inf: no inf - inf then (a factor of 1,
+  // an exponent base of 0)
+  auto factor = [](float from, float to) { return from == to ? 1.f : fast_exp2(from - to); };
   f32x16 acc[DT];
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt)
@@ -593,8 +592,8 @@ __global__ __launch_bounds__(256, KSL == 1 ? 3 : 2) void fwd32_kernel(
 #pragma unroll
         for (int i = 0; i < 16; ++i) acc[dt][i] *= alpha;
       m = mnew;
+      base = m == -INFINITY ? 0.f : m;
     }
-    const float base = KSL == 2 && m == -INFINITY ? 0.f : m;
     float psum = 0.f;
     u32x4 pk[2];
 #pragma unroll
@@ -1316,33 +1315,56 @@ void launch_fwd_kernel(const FwdArgs& a, const FwdWs& w, int Skp, int n_rep, int
             a.doc ? a.doc : a.kvalid, w.ranges, (T*)w.qrot, order, kpm_keys);
 }
 
-// Key slices per workgroup of an unmasked forward of nblk 128-row blocks: two
-// up to one block per CU (D 64, whose two slices still leave four workgroups
-// per CU: three).  A wavefront's chain of tiles is then what the launch lasts
-// (0.8 us per tile, whatever the ring depth: three or four staged tiles gained
-// nothing).  One / two slices, forward kernel alone: D 128, 32/8 heads S = 256
-// 14.9 / 13.0 us, 512 19.2 / 16.7, 1000 (256 blocks) 28.9 / 26.1, 1999 (504) 54.9
-// / 56.7, 3000 (752) 91 / 105; D 64, 12 heads S = 2048 37 / 27, B = 2 S = 1024 22.7
-// / 18.1, B = 4 S = 2048 (768) 62 / 51.  With D 128 only below 2048 positions,
-// though it pays beyond (8/2 heads S = 2048 47.0 / 32.8 us, S = 4096 84.8 / 63.2;
-// 4/1 S = 8192 152.8 / 110.3): the slices add up in another order, and the
-// backward's test of an 8256-row sequence wants the first 2048 rows' dQ, and so
-// their out and LSE, to be the bits of a run on those rows alone.  That is no
-// property of the library: rows at D 64, and of sequences shorter than 2048 at
-// D 128, can differ in the last bits with the length and the batch.
-int fwd_slices(int64_t nblk, int n_rep, int D, int Sq) {
+// Key slices per workgroup of an unmasked forward whose two-slice form has n2
+// workgroups in `groups` (batch row, KV head) groups.  A wavefront's chain of
+// tiles is what a small grid lasts (0.8 us per tile, whatever the ring depth:
+// three or four staged tiles gained nothing); two slices halve it, for more
+// workgroups with a prologue each and a merge, so the longest row's keys have to
+// outweigh those.  Graph-timed (kv_prep included), one / two slices, 1666 causal
+// grids of 14 head layouts, by two-slice workgroups per CU r: up to one, from 100
+// keys on (at 65 and below, the merge loses 1 to 2 us) all but tiny grids gain,
+// D 128 5% at 100 keys, 9 at 256, 19 from 500 on, D 64 6, 12 and 27.  D 128, r 1 to 2: from 800 keys on
+// all 35 gain, 3 to 20%; 128 to 300 keys lose 10, 500 to 800 neither (12/2 B5
+// S299 20.9 / 22.5 us, 32/8 S1000 28.9 / 26.1).  D 64, r 1 to 3: from 300 (r - 1)
+// on they gain up to 40% and none loses 2; 128 to 300 lose 4 to 6%.  r 4: with groups of query heads
+// 8% from 1000 on, without them 3000 keys 7%, 2048 keys 5% lost; r 5: 14% from
+// 1000 on; r 6: from 2000 on 10% where eight or more groups share the XCDs
+// evenly (16/2 B2 S3000, four groups, 61 / 77).  Past that one slice.  Without the
+// causal mask, whose blocks are equally long, up to r 3 as with it (480 grids, 11%
+// less on average); 4/2 B8 S2047 (r 4) 53 / 59.
+//
+// With D 128 only below 2048 positions, though it pays beyond (8/2 heads S = 2048
+// 47.0 / 32.8 us, S = 4096 84.8 / 63.2; 4/1 S = 8192 152.8 / 110.3): the slices add
+// up in another order, and the backward's test of an 8256-row sequence wants the
+// first 2048 rows' dQ, and so their out and LSE, to be the bits of a run on those
+// rows alone.  That is no property of the library: rows at D 64, and of sequences
+// shorter than 2048 at D 128, can differ in the last bits with the length and
+// the batch.
+int fwd_slices(int64_t n2, int64_t groups, int n_rep, int D, int Sq, int keys, int causal) {
   if (n_rep > ROWS / 2 || (D == 128 && Sq >= 2048)) return 1;
-  return nblk <= (D == 64 ? 3 : 1) * (int64_t)device_cu_count() ? 2 : 1;
+  const int64_t cus = device_cu_count(), r = (n2 + cus - 1) / cus;
+  int from = INT_MAX;  // keys from which two slices gain
+  if (r <= 1) from = 96;
+  else if (D == 128) from = r == 2 ? 800 : INT_MAX;
+  else if (r <= 3) from = 300 * (int)(r - 1);
+  else if (!causal) from = INT_MAX;
+  else if (r == 4) from = n_rep > 1 ? 1000 : 2500;
+  else if (r == 5) from = 1000;
+  else if (r == 6 && groups >= 8) from = 2000;
+  return keys >= from ? 2 : 1;
 }
 
 template <typename T, int D>
 void launch_fwd32(const FwdArgs& a, const FwdWs& w, int Skp, int n_rep, int bm_pos, int nqb,
                   unsigned nblk, const int* kpm_keys) {
-  const int ksl = fwd_slices(nblk, n_rep, D, a.Sq);
+  const int64_t groups = (int64_t)a.B * a.Hkv;
+  const int bm2 = std::max(1, ROWS / 2 / n_rep), nqb2 = (a.Sq + bm2 - 1) / bm2;
+  const int ksl = fwd_slices(nqb2 * groups, groups, n_rep, D, a.Sq,
+                             a.causal ? std::min(a.Sq, a.Sk) : a.Sk, a.causal);
   if (ksl == 2) {
-    bm_pos = ROWS / 2 / n_rep;
-    nqb = (a.Sq + bm_pos - 1) / bm_pos;
-    nblk = (unsigned)nqb * a.B * a.Hkv;
+    bm_pos = bm2;
+    nqb = nqb2;
+    nblk = (unsigned)(nqb2 * groups);
   }
   KF_LAUNCH("fwd_mfma", (ksl == 2 ? fwd32_kernel<T, D, 2> : fwd32_kernel<T, D, 1>), dim3(nblk),
             dim3(256), 0, a.stream, (const T*)a.q, a.cos, a.sin, (const T*)w.krot, (const T*)w.vn,
