@@ -1447,17 +1447,20 @@ int dkdv_splits(int B, int S, int Hq, int Hkv) {
   return n;
 }
 
-// Whether an unmasked, unsplit dK/dV launch deals its items longest first over
-// all KV heads.  Group by group (fewer heads' query tiles in flight on an XCD)
-// the zigzag rounds of G workgroups pair long items with short ones only when
-// a round holds whole sweeps of key blocks or a sweep whole rounds.  Measured
+// Whether an unmasked, unsplit causal dK/dV launch deals its items longest first
+// over all KV heads.  Group by group (fewer heads' query tiles in flight on an
+// XCD) the zigzag rounds of G workgroups pair long items with short ones only
+// when a round holds whole sweeps of key blocks or a sweep whole rounds.  Measured
 // (32 query heads of 128, dK/dV alone, group by group / dealt): S = 1531, B = 6
 // 430 / 293 us, S = 3000, B = 4 820 / 663, S = 5000, B = 2 (64 heads) 2159 /
 // 1816; balanced either way, S = 4096, B = 4 1160 / 1170 and S = 16384 (64 heads)
-// 9219 / 9330.
-bool dkdv_deal(int nkb) {
+// 9219 / 9330.  Whole backwards with 3 to 40 key blocks, 39 sizes: 7 to 29% less.
+// Without the causal mask the items are equally long and dealing only costs
+// locality (whole backward, 32 heads, S = 575, B = 11 344 / 355 us, 32/8, S = 1531,
+// B = 6 786 / 799).
+bool dkdv_deal(int nkb, int causal) {
   const int G = device_cu_count() / 8;
-  return G % nkb != 0 && nkb % G != 0;
+  return causal && G % nkb != 0 && nkb % G != 0;
 }
 
 size_t align256(size_t n) { return (n + 255) / 256 * 256; }
@@ -1686,7 +1689,7 @@ int launch_bwd(const BwdArgs& a, void* workspace, bool keep_ds) {
                                            : bwd_dkdv_kernel<T, D, MASK_KPM, false>)
              : part             ? (keep_ds ? bwd_dkdv_kernel<T, D, MASK_NONE, true, false, true>
                                            : bwd_dkdv_kernel<T, D, MASK_NONE, false, false, true>)
-             : dkdv_deal(nkb)   ? (keep_ds ? bwd_dkdv_kernel<T, D, MASK_NONE, true, false, false, true>
+             : dkdv_deal(nkb, a.causal) ? (keep_ds ? bwd_dkdv_kernel<T, D, MASK_NONE, true, false, false, true>
                                            : bwd_dkdv_kernel<T, D, MASK_NONE, false, false, false, true>)
              : keep_ds          ? bwd_dkdv_kernel<T, D, MASK_NONE, true>
                                 : bwd_dkdv_kernel<T, D, MASK_NONE, false>),

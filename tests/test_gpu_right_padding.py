@@ -96,3 +96,13 @@ def test_limits_split(cfg, limits):
 def test_dealt_without_a_mask(cfg, deal):
     announce(f"dealt dK/dV {cfg}")
     _check(cfg, None, (0, 0, deal))
+
+
+def test_full_attention_is_not_dealt():
+    """Items of equal length: group by group whatever the block count."""
+    announce("dealt dK/dV, full attention")
+    q, k, v, do, cos, sin = (t.to(DEV) for t in _inputs(BF16, 22, 300, 16, 8, 64))
+    out, lse = ops.fwd_raw(q, k, v, cos, sin, causal=False, k_rotated=False)
+    ran = kernel_variants(lambda: ops.bwd_raw(q, k, v, cos, sin, out, lse, do, causal=False),
+                          "bwd_dkdv_kernel")
+    assert [r[1:] for r in ran] == [(MASK_NONE, 1, 0, 0, 0)], ran
