@@ -444,7 +444,7 @@ __global__ __launch_bounds__(256, 2) void fwd_f32_kernel(
   __shared__ int sCount;
 
   const int lane = threadIdx.x & 63, g = lane >> 4, c16 = lane & 15, w = wave_id();
-  const int logical = mfma::paired_id(blockIdx.x, gridDim.x, nqb);
+  const int logical = mfma::block_id(blockIdx.x, gridDim.x, nqb, causal);
   const RowInfo ri = row_info(logical, nqb, Hkv, n_rep, bm_pos, Sq, w * 16 + c16);
   const KeyWalk<MODE> kw =
       key_walk<MODE>(ri, causal ? min(Sk, min(ri.p0 + bm_pos, Sq)) : Sk, Sk, bm_pos, mask,
@@ -552,7 +552,7 @@ __global__ __launch_bounds__(256, 2) void capture_f32_kernel(
   __shared__ int sCount;
 
   const int lane = threadIdx.x & 63, g = lane >> 4, c16 = lane & 15, w = wave_id();
-  const int logical = mfma::paired_id(blockIdx.x, gridDim.x, nqb);
+  const int logical = mfma::block_id(blockIdx.x, gridDim.x, nqb, causal);
   const RowInfo ri = row_info(logical, nqb, Hkv, n_rep, bm_pos, Sq, w * 16 + c16);
   const KeyWalk<MODE> kw =
       key_walk<MODE>(ri, causal ? min(Sk, min(ri.p0 + bm_pos, Sq)) : Sk, Sk, bm_pos, mask,
@@ -692,7 +692,7 @@ __global__ __launch_bounds__(256, 2) void bwd_dq_f32_kernel(
   __shared__ int sCount;
 
   const int lane = threadIdx.x & 63, g = lane >> 4, c16 = lane & 15, w = wave_id();
-  const int logical = mfma::paired_id(blockIdx.x, gridDim.x, nqb);
+  const int logical = mfma::block_id(blockIdx.x, gridDim.x, nqb, causal);
   const RowInfo ri = row_info(logical, nqb, Hkv, n_rep, bm_pos, S, w * 16 + c16);
   const KeyWalk<MODE> kw = key_walk<MODE>(ri, causal ? min(S, ri.p0 + bm_pos) : S, S, bm_pos,
                                           mask, ranges, first_valid, nt32, sList, &sCount, w,
@@ -771,7 +771,7 @@ __global__ __launch_bounds__(256, 2) void bwd_dq_rec_f32_kernel(
   __shared__ __attribute__((aligned(16))) float sK[2][F_BN * D];
 
   const int lane = threadIdx.x & 63, g = lane >> 4, c16 = lane & 15, w = wave_id();
-  const int logical = mfma::paired_id(blockIdx.x, gridDim.x, nqb);
+  const int logical = mfma::block_id(blockIdx.x, gridDim.x, nqb, causal);
   const RowInfo ri = row_info(logical, nqb, Hkv, n_rep, bm_pos, S, w * 16 + c16);
   const int kend = causal ? min(S, ri.p0 + bm_pos) : S;
   const int ntiles = (kend + F_BN - 1) / F_BN;
