@@ -1414,7 +1414,15 @@ int fwd_f32_t(const FwdArgs& a, void* workspace) {
 // 30 us, not included): D 128, 32/8 heads B = 1 S = 1024 734 / 209 us, S = 2048
 // 1475 / 719, S = 4096 (512 items) 2966 / 2578; D 64, 4/2 heads, B = 2 S = 256 62 /
 // 13; 16 heads of 96 without groups, B = 2 S = 1024 (512 items) 160 / 152 with two
-// runs, and 15 for their sum: not split.  The parts take 8 D bytes per key row,
+// runs, and 15 for their sum: not split.  Without groups (n_rep 1) the second
+// launch and the pass over the parts cost what short chains save, so a line in
+// the positions too.  Whole backward, split against unsplit, by items per CU: up
+// to 1/4, 33 to 127 positions 3 to 17% less; to 1/2, 33 and 58 2 to 5% more, 262
+// on 17 to 43% less; to 1, 33 to 127 7 to 17% more (up to 22), 262 on 14 to 28%
+// less; to 2, 100 to 262 4 to 10% more, 800 on 3 to 8% less.  Without the causal mask, whose items are equally
+// long, and with packed documents, whose items list few tiles, they gain later:
+// full attention 8% from 800 on up to one item per CU, packed documents 15% from
+// 800 on up to 1/2, and past that both lose up to 13%.  The parts take 8 D bytes per key row,
 // part and KV head, at most PARTS_MAX: 16 query heads per group at 1024 items of
 // D 128 (64/2 heads, S = 16000, 1000 MiB: dK/dV 90.2 ms unsplit, 76.4 with the
 // parts and their sum; 64/4, B = 2, S = 6000, 750 MiB: 23.0 and 22.0).
@@ -1422,7 +1430,7 @@ constexpr size_t PARTS_MAX = (size_t)1 << 30;
 size_t parts_bytes(int B, int S, int Hq, int Hkv, int D, int nseg) {
   return (size_t)B * S * Hkv * (Hq / Hkv) * nseg * 2 * D * sizeof(float);
 }
-int dkdv_parts(int B, int S, int Hq, int Hkv, int D) {
+int dkdv_parts(int B, int S, int Hq, int Hkv, int D, int causal, bool doc) {
   const int64_t items = (int64_t)((S + F_BK - 1) / F_BK) * B * Hkv;
   const int64_t cus = device_cu_count();
   const int n_rep = Hq / Hkv, nt = (S + F_BN - 1) / F_BN;
@@ -1430,6 +1438,12 @@ int dkdv_parts(int B, int S, int Hq, int Hkv, int D) {
   const int64_t heads = items * n_rep;
   const int nseg = (int)std::min<int64_t>({(2 * cus + heads - 1) / heads, 8, nt});
   if (n_rep * nseg == 1 || parts_bytes(B, S, Hq, Hkv, D, nseg) > PARTS_MAX) return 0;
+  if (n_rep == 1 && 4 * items > cus) {
+    const bool half = 2 * items <= cus, one = items <= cus;
+    const int from = doc ? (half ? 640 : INT_MAX) : !causal ? (half ? 256 : one ? 640 : INT_MAX)
+                                                            : (half ? 96 : one ? 256 : 640);
+    if (S < from) return 0;
+  }
   return nseg;
 }
 
@@ -1614,7 +1628,7 @@ bool bwd_f32_supported(const BwdArgs& a) {
 
 size_t bwd_f32_workspace(int B, int S, int Hq, int Hkv, int D) {
   size_t sum_off = 0;
-  const int nseg = dkdv_parts(B, S, Hq, Hkv, D);
+  const int nseg = dkdv_parts(B, S, Hq, Hkv, D, 1, false);  // (no other mask splits more)
   return al256(bwd_base_bytes(B, S, Hq, Hkv, D, nseg, &sum_off)) + mask_rec_bytes(B, S);
 }
 
@@ -1629,10 +1643,13 @@ size_t bwd_f32_workspace_ds(int B, int S, int Hq, int Hkv, int D, int causal) {
   return rb ? al256(bwd_f32_workspace(B, S, Hq, Hkv, D)) + rb : bwd_f32_workspace(B, S, Hq, Hkv, D);
 }
 
-F32BwdWs bwd_f32_carve(int B, int S, int Hq, int Hkv, int D, void* workspace, size_t bytes) {
+F32BwdWs bwd_f32_carve(int B, int S, int Hq, int Hkv, int D, int causal, bool doc,
+                       void* workspace, size_t bytes) {
   F32BwdWs w;
   w.Sp = (S + F_BK - 1) / F_BK * F_BK;
-  w.nseg = bytes >= bwd_f32_workspace(B, S, Hq, Hkv, D) ? dkdv_parts(B, S, Hq, Hkv, D) : 0;
+  w.nseg = bytes >= bwd_f32_workspace(B, S, Hq, Hkv, D)
+               ? dkdv_parts(B, S, Hq, Hkv, D, causal, doc)
+               : 0;
   size_t sum_off = 0;
   const size_t base = bwd_base_bytes(B, S, Hq, Hkv, D, w.nseg, &sum_off);
   w.qrot = (float*)workspace;
@@ -1668,7 +1685,8 @@ int bwd_f32_kernels(const BwdArgs& a, const F32BwdWs& w, void* workspace, size_t
 }
 
 int bwd_f32(const BwdArgs& a, void* workspace, size_t workspace_bytes) {
-  const F32BwdWs w = bwd_f32_carve(a.B, a.S, a.Hq, a.Hkv, a.D, workspace, workspace_bytes);
+  const F32BwdWs w = bwd_f32_carve(a.B, a.S, a.Hq, a.Hkv, a.D, a.causal, a.doc != nullptr,
+                                   workspace, workspace_bytes);
   int rc = by_dim(a.D, [&](auto d) { return bwd_rows_t<decltype(d)::value>(a, w); });
   if (rc) return rc;
   rc = bwd_f32_stats(a.out, a.dout, a.lse, F32, a.B, a.S, a.Hq, a.D, w, a.stream);

@@ -88,7 +88,8 @@ struct F32BwdWs {
   int Sp;              // S rounded up to 64
   int nseg;            // runs of the split dK/dV items' heads, 0: not split
 };
-F32BwdWs bwd_f32_carve(int B, int S, int Hq, int Hkv, int D, void* workspace, size_t bytes);
+F32BwdWs bwd_f32_carve(int B, int S, int Hq, int Hkv, int D, int causal, bool doc,
+                       void* workspace, size_t bytes);
 int bwd_f32_stats(const void* out, const void* dout, const float* lse, int dtype, int B, int S,
                   int Hq, int D, const F32BwdWs& w, hipStream_t stream);
 int bwd_f32_kernels(const BwdArgs& a, const F32BwdWs& w, void* workspace, size_t workspace_bytes);

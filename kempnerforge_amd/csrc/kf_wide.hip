@@ -311,8 +311,8 @@ size_t bwd_wide_workspace(const BwdArgs& a, bool with_ds) {
 int bwd_wide(const BwdArgs& a, void* workspace, size_t workspace_bytes) {
   const int W = wide_dim(a.D);
   const BwdWide w = carve_bwd(a, workspace);
-  const F32BwdWs fw =
-      bwd_f32_carve(a.B, a.S, a.Hq, a.Hkv, W, w.ws, workspace_bytes - w.head);
+  const F32BwdWs fw = bwd_f32_carve(a.B, a.S, a.Hq, a.Hkv, W, a.causal, a.doc != nullptr, w.ws,
+                                    workspace_bytes - w.head);
   const int64_t qs = (int64_t)a.Hq * a.D, ks = (int64_t)a.Hkv * a.D;
   WideJobs jobs{};
   // q and k straight into the float32 backward's rotated rows [b h][Sp][W]

@@ -26,6 +26,21 @@ F32 = torch.float32
     (16, 130, 16, 16, 64, True, None, False),  # 768 items, no groups
     (16, 130, 32, 16, 64, True, None, True),   # the same items in groups of two: heads only
     (22, 130, 16, 16, 64, True, "doc", False),  # 1056 items
+    # without groups: a line in the positions by items per CU
+    (1, 65, 32, 32, 64, True, None, True),      # 64 items
+    (1, 90, 40, 40, 64, True, None, False),     # 80: 96 positions
+    (1, 96, 40, 40, 64, True, None, True),
+    (1, 250, 40, 40, 32, True, None, False),    # 160: 256
+    (1, 256, 40, 40, 32, True, None, True),
+    (1, 256, 40, 40, 32, False, None, False),   # full attention: 640
+    (1, 640, 16, 16, 32, False, None, True),
+    (2, 600, 16, 16, 32, True, None, False),    # 320: 640
+    (2, 640, 16, 16, 32, True, None, True),
+    (2, 640, 16, 16, 32, False, None, False),
+    (1, 600, 12, 12, 32, True, "doc", False),   # 120: 640
+    (1, 640, 12, 12, 32, True, "doc", True),
+    (1, 640, 16, 16, 32, True, "doc", False),   # 160
+    (2, 640, 16, 16, 32, True, "kpm", True),    # key padding as without a mask
 ], ids=lambda c: "-".join(map(str, c)))
 def test_gradients(cfg):
     B, S, Hq, Hkv, D, causal, mask, split = cfg
