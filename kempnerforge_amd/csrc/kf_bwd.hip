@@ -1528,11 +1528,13 @@ Ws carve(void* base, int B, int S, int Hq, int Hkv, int D, const void* rot) {
 //  - one head per workgroup (n_rep odd): both two, while all workgroups are
 //    resident at once (10/2 B1 S1024 25.3 -> 19.1; 16/16 D64 B1 S2048 30.5 ->
 //    23.8) and for long sequences at two or more per CU (10/2 B2 S4096 118 ->
-//    106, 12/12 D64 B8 S2048 115 -> 103).  Between, half of the CUs would run
-//    one workgroup more than the others (12/12 D64 B2 S2048 34.8 against 38.5),
-//    and batches of short sequences have tiles enough (10/2 B12 S700 35.2
-//    against 38.2).  Up to three tiles the merge costs what the slices save
-//    (12/12 D64 B1 S65 6.6 against 7.5).
+//    106, 12/12 D64 B8 S2048 115 -> 103), where the KV heads fill the XCDs in
+//    whole groups or halves (whole backwards, 341 sizes: 2% less, 12 lose more
+//    than 1.5%; 93 others gain nothing on average and 23 lose, up to 6%: 10/2 B7
+//    S1974 343 -> 365).  Between, half of the CUs would run one workgroup more
+//    than the others (12/12 D64 B2 S2048 34.8 against 38.5), and batches of short
+//    sequences have tiles enough (10/2 B12 S700 35.2 against 38.2).  Up to three
+//    tiles the merge costs what the slices save (12/12 D64 B1 S65 6.6 against 7.5).
 //  - two heads: two slices up to one workgroup per CU (4/2 D64 B3 S1600 23.8 ->
 //    18.6), two tiles as well on larger grids of long sequences (12/2 B2 S4096
 //    134 -> 110, 16/8 B4 S3000 151 -> 141, B6 S6000 813 -> 702).  Of 104 such grids
@@ -1545,11 +1547,11 @@ Ws carve(void* base, int B, int S, int Hq, int Hkv, int D, const void* rot) {
 //  - four heads: one tile; either split came out equal or slower (32/8 B4 S1024
 //    50.7 against 53.6 with two slices).
 struct DqSplit { int qt, ksp; };
-DqSplit dq_split(int hb, int64_t ntile, int nqt) {
+DqSplit dq_split(int hb, int64_t ntile, int nqt, int64_t kv_heads) {
   const int64_t cus = device_cu_count();
   if (hb == 1 && nqt >= 4) {
     const int64_t nwg = ntile / nqt * ((nqt + 1) / 2);
-    if (nwg <= cus || (nwg >= 2 * cus && nqt >= 24)) return {2, 2};
+    if (nwg <= cus || (nwg >= 2 * cus && nqt >= 24 && kv_heads % 4 == 0)) return {2, 2};
   }
   if (hb == 2 && nqt >= 16) {
     if (ntile <= cus) return {1, 2};
@@ -1577,7 +1579,7 @@ int launch_dq_ds(const BwdArgs& a, const Ws& w) {
     return KF_OK;
   }
   const int ntile = a.B * a.Hkv * (n_rep / HB) * nqt;
-  DqSplit sp = a.doc ? DqSplit{1, 1} : dq_split(HB, ntile, nqt);
+  DqSplit sp = a.doc ? DqSplit{1, 1} : dq_split(HB, ntile, nqt, (int64_t)a.B * a.Hkv);
   if (a.kvalid) sp.qt = 1;  // (the same sums: a tile's do not depend on its neighbour)
   const int nwg = ntile / nqt * ((nqt + sp.qt - 1) / sp.qt);
   auto kernel = a.doc      ? (deep ? bwd_dq_ds_kernel<T, D, HB, 1, 1, MASK_DOC, 4>

@@ -57,7 +57,9 @@ def test_gradients(cfg):
     ((F16, 2, 2000, 18, 1, 64), (2, 2, 2)),      # 32 tiles, 576 in all
     ((F16, 2, 1980, 18, 1, 64), (2, 1, 1)),      # 31 tiles
     ((BF16, 8, 1500, 8, 4, 64), (2, 1, 1)),
-    ((BF16, 3, 1500, 15, 15, 64), (1, 2, 2)),    # 540 workgroups of two tiles and slices
+    ((BF16, 4, 1500, 15, 15, 64), (1, 2, 2)),    # 720 workgroups of two tiles and slices
+    ((BF16, 3, 1500, 15, 15, 64), (1, 1, 1)),    # 540, but 45 KV heads
+    ((BF16, 3, 1500, 12, 12, 64), (1, 1, 1)),    # 432
     ((BF16, 2, 1500, 15, 15, 64), (1, 1, 1)),    # 360
     ((BF16, 5, 2055, 4, 1, 64), (4, 1, 1)),
 ], ids=lambda c: "-".join(map(str, (str(c[0])[6:],) + c[1:])) if len(c) > 3 else
