@@ -1661,7 +1661,7 @@ int launch_bwd(const BwdArgs& a, void* workspace, bool keep_ds) {
               (int)nrows);
   };
   if (kpm_keys) {
-    const int rc = launch_kpm_row_keys(a.kvalid, a.S, a.B, w.counts, a.stream);
+    const int rc = launch_kpm_row_keys(a.kvalid, w.ranges, P / BN, a.S, a.B, w.counts, a.stream);
     if (rc) return rc;
     const int ns = dkdv_splits(a.B, a.S, a.Hq, a.Hkv);
     float* dkp = small ? w.dkvp : nullptr;

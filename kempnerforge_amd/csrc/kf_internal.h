@@ -126,8 +126,9 @@ int launch_kv_prep(const FwdArgs& a, void* krot, int krows, void* vn, int Skp, i
 int launch_doc_order(const int32_t* doc, const int2* ranges, int S, int rstride, int rows, int B,
                      int nblk, int key_side, int* counts, int* order, hipStream_t stream);
 // Key padding: keys[b] = n when batch row b's valid keys are exactly the first
-// n > 0 of its S, else 0.
-int launch_kpm_row_keys(const int32_t* kvalid, int S, int B, int* keys, hipStream_t stream);
+// n > 0 of its S, else 0 (ranges: launch_kv_prep's records, rstride per row).
+int launch_kpm_row_keys(const int32_t* kvalid, const int2* ranges, int rstride, int S, int B,
+                        int* keys, hipStream_t stream);
 // bytes of FwdArgs::rot
 size_t rot_bytes(int B, int S, int Hq, int Hkv, int D);
 size_t fwd_mfma_workspace(int B, int Sk, int Hkv, int D);
