@@ -1419,13 +1419,14 @@ int fwd_f32_t(const FwdArgs& a, void* workspace) {
 // the positions too.  Whole backward, split against unsplit, by items per CU: up
 // to 1/4, 33 to 127 positions 3 to 17% less; to 1/2, 33 and 58 2 to 5% more, 262
 // on 17 to 43% less; to 1, 33 to 127 7 to 17% more (up to 22), 262 on 14 to 28%
-// less; to 2, 100 to 262 4 to 10% more, 800 on 3 to 8% less.  Without the causal mask, whose items are equally
-// long, and with packed documents, whose items list few tiles, they gain later:
-// full attention 8% from 800 on up to one item per CU, packed documents 15% from
-// 800 on up to 1/2, and past that both lose up to 13%.  The parts take 8 D bytes per key row,
-// part and KV head, at most PARTS_MAX: 16 query heads per group at 1024 items of
-// D 128 (64/2 heads, S = 16000, 1000 MiB: dK/dV 90.2 ms unsplit, 76.4 with the
-// parts and their sum; 64/4, B = 2, S = 6000, 750 MiB: 23.0 and 22.0).
+// less; to 2, 100 to 262 4 to 10% more, 800 on 3 to 8% less.  Without the causal
+// mask, whose items are equally long, and with packed documents, whose items list
+// few tiles, they gain later: full attention 8% from 800 on up to one item per CU,
+// packed documents 15% from 800 on up to 1/2, and past that both lose up to 13%.
+// The parts take 8 D bytes per key row, part and KV head, at most PARTS_MAX: 16
+// query heads per group at 1024 items of D 128 (64/2 heads, S = 16000, 1000 MiB:
+// dK/dV 90.2 ms unsplit, 76.4 with the parts and their sum; 64/4, B = 2, S = 6000,
+// 750 MiB: 23.0 and 22.0).
 constexpr size_t PARTS_MAX = (size_t)1 << 30;
 size_t parts_bytes(int B, int S, int Hq, int Hkv, int D, int nseg) {
   return (size_t)B * S * Hkv * (Hq / Hkv) * nseg * 2 * D * sizeof(float);

@@ -1323,10 +1323,11 @@ void launch_fwd_kernel(const FwdArgs& a, const FwdWs& w, int Skp, int n_rep, int
 // outweigh those.  Graph-timed (kv_prep included), one / two slices, 1666 causal
 // grids of 14 head layouts, by two-slice workgroups per CU r: up to one, from 100
 // keys on (at 65 and below, the merge loses 1 to 2 us) all but tiny grids gain,
-// D 128 5% at 100 keys, 9 at 256, 19 from 500 on, D 64 6, 12 and 27.  D 128, r 1 to 2: from 800 keys on
-// all 35 gain, 3 to 20%; 128 to 300 keys lose 10, 500 to 800 neither (12/2 B5
-// S299 20.9 / 22.5 us, 32/8 S1000 28.9 / 26.1).  D 64, r 1 to 3: from 300 (r - 1)
-// on they gain up to 40% and none loses 2; 128 to 300 lose 4 to 6%.  r 4: with groups of query heads
+// D 128 5% at 100 keys, 9 at 256, 19 from 500 on, D 64 6, 12 and 27.  D 128, r 1
+// to 2: from 800 keys on all gain, 1 to 20%; 640 to 800 4% on average, at most 3.7%
+// more (777 keys, 32/8 28.0 / 25.5 us); 500 to 640 neither, 128 to 300 lose 10%
+// (12/2 B5 S299 20.9 / 22.5).  D 64, r 1 to 3: from 300 (r - 1) on they gain up to
+// 40% and none loses 2; 128 to 300 lose 4 to 6%.  r 4: with groups of query heads
 // 8% from 1000 on, without them 3000 keys 7%, 2048 keys 5% lost; r 5: 14% from
 // 1000 on; r 6: from 2000 on 10% where eight or more groups share the XCDs
 // evenly (16/2 B2 S3000, four groups, 61 / 77).  Past that one slice.  Without the
@@ -1345,7 +1346,7 @@ int fwd_slices(int64_t n2, int64_t groups, int n_rep, int D, int Sq, int keys, i
   const int64_t cus = device_cu_count(), r = (n2 + cus - 1) / cus;
   int from = INT_MAX;  // keys from which two slices gain
   if (r <= 1) from = 96;
-  else if (D == 128) from = r == 2 ? 800 : INT_MAX;
+  else if (D == 128) from = r == 2 ? 640 : INT_MAX;
   else if (r <= 3) from = 300 * (int)(r - 1);
   else if (!causal) from = INT_MAX;
   else if (r == 4) from = n_rep > 1 ? 1000 : 2500;
@@ -1485,11 +1486,11 @@ void launch_capture_tiles(const FwdArgs& a, const FwdWs& w, float* probs, int Sk
 // heads of 128, one sequence): S = 65 (16 workgroups) 59 / 23 us, 777 (104) 117 /
 // 60, 1000 (128) 100 / 70; only with one query block per head the second launch
 // just adds (S = 17 14.6 / 18.5; 12/12 of 64, S = 128 14.7 / 18.3), which the
-// tests of these sizes still ask for.  The pieces write P at 1.7 TB/s where its rows are off 64-byte
-// blocks, the fused kernel at up to 2.9, so not past 192 MiB of P (S = 1200, 176
-// MiB, 109 / 97; 1500, 275 MiB, 137 / 168); with rows of whole blocks 3 TB/s, not
-// past 320 (16/2 heads S = 2000, 244 MiB, 142 / 118; S = 2400, 352 MiB, 160 / 162).
-// Explicit masks stay fused.
+// tests of these sizes still ask for.  The pieces write P at 1.7 TB/s where its
+// rows are off 64-byte blocks, the fused kernel at up to 2.9, so not past 192 MiB
+// of P (S = 1200, 176 MiB, 109 / 97; 1500, 275 MiB, 137 / 168); with rows of whole
+// blocks 3 TB/s, not past 320 (16/2 heads S = 2000, 244 MiB, 142 / 118; S = 2400,
+// 352 MiB, 160 / 162).  Explicit masks stay fused.
 bool capture_after_fwd(const FwdArgs& a) {
   if (a.doc || a.kvalid) return false;
   const int bm_pos = pick_bm_pos(a.Hq / a.Hkv), nqb = (a.Sq + bm_pos - 1) / bm_pos;

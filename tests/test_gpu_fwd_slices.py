@@ -69,8 +69,8 @@ def test_infinite_keys_in_one_half():
     ((BF16, 1, 200, 64, 1, 128, True), 2),
     ((BF16, 1, 200, 80, 1, 64, True), 1),     # n_rep 80
     ((BF16, 5, 299, 12, 2, 128, True), 1),    # r 2, too short
-    ((BF16, 1, 799, 40, 8, 128, True), 1),
-    ((BF16, 1, 800, 32, 8, 128, True), 2),
+    ((BF16, 1, 639, 40, 8, 128, True), 1),
+    ((BF16, 1, 640, 32, 8, 128, True), 2),
     ((BF16, 1, 1024, 32, 8, 128, False), 2),  # 512 of them
     ((BF16, 1, 1028, 32, 8, 128, True), 1),   # r 3
     ((BF16, 1, 2047, 4, 2, 128, True), 2),
