@@ -1401,11 +1401,11 @@ void launch_fwd_mode(const FwdArgs& a, const FwdWs& w, int Skp, int n_rep, int b
 // joins into whole lines, where a non-temporal store of part of a block is a
 // partial write to memory (32/8 heads of 128, S = 3000: 404 against 495 us; on
 // whole blocks non-temporal is ahead, 147 against 165 at S = 2000); rows of no
-// whole 16-byte pieces with a tail of single elements.  A kernel for each: with
-// the three told apart at each store, by a branch, every capture was 15 to 20%
-// slower (S = 1024 100 -> 117 us, 64/8 heads S = 2048 219 -> 271), and rows off
-// 64-byte blocks under a mask another 5 to 10% (S = 1500, packed documents 166
-// now, 199 so).
+// whole 16-byte pieces with a tail of single elements.  A kernel for each; with
+// the three told apart at each store, by a branch, whole captures took (graph-
+// timed, branch / a kernel each) 64/8 heads S = 1024 113 / 99 us, S = 2048 260 /
+// 253, 32/8 S = 2048 191 / 177, S = 3000 433 / 418, packed documents S = 1500 199 /
+// 167.
 int p_store(int Sk) { return Sk % 16 == 0 ? P_NT : Sk % 4 == 0 ? P_VEC : P_ANY; }
 
 template <typename T, int D, int MODE>
