@@ -1323,18 +1323,18 @@ void launch_fwd_kernel(const FwdArgs& a, const FwdWs& w, int Skp, int n_rep, int
 // outweigh those.  Graph-timed (kv_prep included), one / two slices, 1666 causal
 // grids of 14 head layouts, by two-slice workgroups per CU r: up to one, from 100
 // keys on all but tiny grids gain, D 128 5% at 100 keys, 9 at 256, 19 from 500 on,
-// D 64 6, 12 and 27; at 64, groups of query heads up to 9% (without them 3 to 6%
-// lost); at 33 neither (32/8 B8 15.4 / 14.1 us, 2/1 13.1 / 14.9), at 17 the merge
-// loses up to 3 us.  D 128, r 1 to 2: from 800 keys on all gain, 1 to 20%; 640 to
-// 800 4% on average, at most 3.7% more (777 keys, 32/8 28.0 / 25.5 us); 500 to 640
-// neither, 128 to 300 lose 10% (12/2 B5 S299 20.9 / 22.5).  D 64, r 1 to 3: from
-// 300 (r - 1) on they gain up to 40% and none loses 2; 128 to 300 lose 4 to 6%.
-// r 4: with groups of query heads 8% from 1000 on, without them 3000 keys 7%, 2048
-// keys 5% lost; r 5: 14% from 1000 on; r 6: from 2000 on 10% where eight or more
-// groups share the XCDs evenly (16/2 heads, four groups at B2 S3000 61 / 77, though
-// six at B3 S2048 63 / 51).  Past that one slice.  Without the causal mask, whose
-// blocks are equally long, up to r 3 as with it (480 grids, 11% less on average);
-// 4/2 B8 S2047 (r 4) 53 / 59.
+// D 64 6, 12 and 27; at 65 to 94, D 64 2 to 4%, D 128 even; at 64, groups of query
+// heads up to 9% (without them 3 to 6% lost); at 33 to 56 neither (32/8 B8 S33 15.4
+// / 14.1 us, 2/1 13.1 / 14.9), at 17 the merge loses up to 3 us.  D 128, r 1 to 2:
+// from 800 keys on all gain, 1 to 20%; 640 to 800 4% on average, at most 3.7% more
+// (777 keys, 32/8 28.0 / 25.5 us); 500 to 640 neither, 128 to 300 lose 10% (12/2 B5
+// S299 20.9 / 22.5).  D 64, r 1 to 3: from 300 (r - 1) on they gain up to 40% and
+// none loses 2; 128 to 300 lose 4 to 6%.  r 4: with groups of query heads 8% from
+// 1000 on, without them 3000 keys 7%, 2048 keys 5% lost; r 5: 14% from 1000 on; r 6:
+// from 2000 on 10% where eight or more groups share the XCDs evenly (16/2 heads,
+// four groups at B2 S3000 61 / 77, though six at B3 S2048 63 / 51).  Past that one
+// slice.  Without the causal mask, whose blocks are equally long, up to r 3 as with
+// it (480 grids, 11% less on average); 4/2 B8 S2047 (r 4) 53 / 59.
 //
 // With D 128 only below 2048 positions, though it pays beyond (8/2 heads S = 2048
 // 47.0 / 32.8 us, S = 4096 84.8 / 63.2; 4/1 S = 8192 152.8 / 110.3): the slices add
@@ -1347,7 +1347,7 @@ int fwd_slices(int64_t n2, int64_t groups, int n_rep, int D, int Sq, int keys, i
   if (n_rep > ROWS / 2 || (D == 128 && Sq >= 2048)) return 1;
   const int64_t cus = device_cu_count(), r = (n2 + cus - 1) / cus;
   int from = INT_MAX;  // keys from which two slices gain
-  if (r <= 1) from = n_rep > 1 ? 64 : 96;
+  if (r <= 1) from = n_rep > 1 ? 64 : 65;
   else if (D == 128) from = r == 2 ? 640 : INT_MAX;
   else if (r <= 3) from = 300 * (int)(r - 1);
   else if (!causal) from = INT_MAX;

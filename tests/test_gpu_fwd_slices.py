@@ -66,8 +66,8 @@ def test_infinite_keys_in_one_half():
     # dtype, B, S, Hq, Hkv, D, causal; r: two-slice workgroups per CU, rounded up
     ((BF16, 1, 63, 4, 2, 128, True), 1),
     ((BF16, 1, 64, 4, 2, 128, True), 2),
-    ((BF16, 1, 95, 4, 4, 128, True), 1),      # no groups
-    ((BF16, 1, 96, 4, 4, 128, True), 2),
+    ((BF16, 1, 64, 4, 4, 128, True), 1),      # no groups
+    ((BF16, 1, 65, 4, 4, 128, True), 2),
     ((BF16, 1, 200, 64, 1, 128, True), 2),
     ((BF16, 1, 200, 80, 1, 64, True), 1),     # n_rep 80
     ((BF16, 5, 299, 12, 2, 128, True), 1),    # r 2, too short
