@@ -1419,10 +1419,12 @@ int fwd_f32_t(const FwdArgs& a, void* workspace) {
 // the positions too.  Whole backward, split against unsplit, by items per CU: up
 // to 1/4, 33 to 127 positions 3 to 17% less; to 1/2, 33 and 58 2 to 5% more, 262
 // on 17 to 43% less; to 1, 33 to 127 7 to 17% more (up to 22), 262 on 14 to 28%
-// less; to 2, 100 to 262 4 to 10% more, 800 on 3 to 8% less.  Without the causal
-// mask, whose items are equally long, and with packed documents, whose items list
-// few tiles, they gain later: full attention 8% from 800 on up to one item per CU,
-// packed documents 15% from 800 on up to 1/2, and past that both lose up to 13%.
+// less; to 3/2, 262 to 510 1 to 8% less (masked first keys, 12 heads of 64, B = 4
+// S = 380 129 / 122 us); to 2, 100 to 423 up to 10% more, 800 on 3 to 8% less.
+// Without the causal mask, whose items are equally long, and with packed
+// documents, whose items list few tiles, they gain later: full attention 8% from
+// 800 on up to one item per CU, packed documents 15% from 800 on up to 1/2, and
+// past that both lose up to 13%.
 // The parts take 8 D bytes per key row, part and KV head, at most PARTS_MAX: 16
 // query heads per group at 1024 items of D 128 (64/2 heads, S = 16000, 1000 MiB:
 // dK/dV 90.2 ms unsplit, 76.4 with the parts and their sum; 64/4, B = 2, S = 6000,
@@ -1441,8 +1443,9 @@ int dkdv_parts(int B, int S, int Hq, int Hkv, int D, int causal, bool doc) {
   if (n_rep * nseg == 1 || parts_bytes(B, S, Hq, Hkv, D, nseg) > PARTS_MAX) return 0;
   if (n_rep == 1 && 4 * items > cus) {
     const bool half = 2 * items <= cus, one = items <= cus;
+    const bool more = 2 * items <= 3 * cus;
     const int from = doc ? (half ? 640 : INT_MAX) : !causal ? (half ? 256 : one ? 640 : INT_MAX)
-                                                            : (half ? 96 : one ? 256 : 640);
+                                                            : (half ? 96 : more ? 256 : 640);
     if (S < from) return 0;
   }
   return nseg;

@@ -34,8 +34,10 @@ F32 = torch.float32
     (1, 256, 40, 40, 32, True, None, True),
     (1, 256, 40, 40, 32, False, None, False),   # full attention: 640
     (1, 640, 16, 16, 32, False, None, True),
-    (2, 600, 16, 16, 32, True, None, False),    # 320: 640
-    (2, 640, 16, 16, 32, True, None, True),
+    (2, 250, 40, 40, 32, True, None, False),    # 320: 256
+    (2, 256, 40, 40, 32, True, None, True),
+    (2, 600, 20, 20, 32, True, None, False),    # 400: 640
+    (2, 640, 20, 20, 32, True, None, True),
     (2, 640, 16, 16, 32, False, None, False),
     (1, 600, 12, 12, 32, True, "doc", False),   # 120: 640
     (1, 640, 12, 12, 32, True, "doc", True),
